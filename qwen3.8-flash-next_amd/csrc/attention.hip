@@ -6,7 +6,9 @@
  *   k_rows    one wave per four rows of [q_proj | k_proj | v_proj] (q4) and
  *             index_qk_proj (bf16); x (f32) as bf16 hi + lo pairs, the q4
  *             rows with gemm_q4's per-group identity (gemv_parts.h).  Also
- *             o_proj at the end.
+ *             o_proj at the end.  From QK_AT_MM_N tokens on the q4 rows run
+ *             on MFMA (proj_mm.hip); a 2048-token call of the benchmark's
+ *             shape spent 6500 us in this kernel's q4 rows and o_proj.
  *   k_at_qk   one wave per (token, head): rmsnorm with q_norm / k_norm /
  *             the indexer's q norm, then partial RoPE at position offset+t
  *             (kernel.c:80-93) from the host's cos / sin table; k, v and
@@ -950,11 +952,28 @@ extern "C" int qk_launch_at(const qk_at_shape *s, const qk_at_dev *W, const floa
     r.hyper = nullptr;
     r.inject = nullptr;
     r.hc = 1;
-    at_seg(r, W->q_q, W->q_s, W->q_b, nullptr, 2 * h * hd, sc->qg, 2 * h * hd);
-    at_seg(r, W->k_q, W->k_s, W->k_b, nullptr, kvh * hd, sc->kraw, kvh * hd);
-    at_seg(r, W->v_q, W->v_s, W->v_b, nullptr, kvh * hd, sc->vraw, kvh * hd);
+    int rc;
+    const bool mm = n >= QK_AT_MM_N;
+    if (mm) {
+        if (!sc->pl.hi || !sc->pl.lo || !sc->pl.pg) return (int)hipErrorInvalidValue;
+        rc = qk_launch_pack_rows(x, 0, (size_t)n, s->d, sc->pl.hi, sc->pl.lo, sc->pl.pg, stream);
+        if (rc) return rc;
+        qk_proj p = {};
+        p.seg[0] = {W->q_q, W->q_s, W->q_b, sc->qg, 2 * h * hd, 2 * h * hd};
+        p.seg[1] = {W->k_q, W->k_s, W->k_b, sc->kraw, kvh * hd, kvh * hd};
+        p.seg[2] = {W->v_q, W->v_s, W->v_b, sc->vraw, kvh * hd, kvh * hd};
+        p.nseg = 3;
+        p.hi = sc->pl.hi; p.lo = sc->pl.lo; p.pg = sc->pl.pg;
+        p.K = s->d; p.n = n;
+        rc = qk_launch_proj(&p, stream);
+        if (rc) return rc;
+    } else {
+        at_seg(r, W->q_q, W->q_s, W->q_b, nullptr, 2 * h * hd, sc->qg, 2 * h * hd);
+        at_seg(r, W->k_q, W->k_s, W->k_b, nullptr, kvh * hd, sc->kraw, kvh * hd);
+        at_seg(r, W->v_q, W->v_s, W->v_b, nullptr, kvh * hd, sc->vraw, kvh * hd);
+    }
     at_seg(r, nullptr, nullptr, nullptr, W->idx_w, (ih + 1) * ihd, sc->qk, (ih + 1) * ihd);
-    int rc = at_rows_launch(r, st);
+    rc = at_rows_launch(r, st);
     if (rc) return rc;
 
     AtQkArgs q;
@@ -1024,6 +1043,18 @@ extern "C" int qk_launch_at(const qk_at_shape *s, const qk_at_dev *W, const floa
     else hipLaunchKernelGGL(k_at_comb<AT_MAXCH / 4>, dim3(n * h), dim3(256), 0, st, cb);
     rc = QK_CHECK_LAUNCH();
     if (rc) return rc;
+
+    if (mm) {
+        rc = qk_launch_pack_rows(sc->ao, 0, (size_t)n, h * hd, sc->pl.hi, sc->pl.lo, sc->pl.pg, stream);
+        if (rc) return rc;
+        qk_proj p = {};
+        p.seg[0] = {W->o_q, W->o_s, W->o_b, out, s->d, s->d};
+        p.nseg = 1;
+        p.hi = sc->pl.hi; p.lo = sc->pl.lo; p.pg = sc->pl.pg;
+        p.K = h * hd; p.n = n;
+        if (inj && inj->hyper) { p.hyper = inj->hyper; p.inject = inj->inject; p.hc = inj->hc; }
+        return qk_launch_proj(&p, stream);
+    }
 
     RowsArgs o;
     o.nseg = 0;

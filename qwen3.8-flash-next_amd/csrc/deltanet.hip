@@ -26,6 +26,13 @@
  *             moves the conv state on by n tokens (its old rows are read by
  *             k_dn_rec, so it changes only here).
  *
+ * From QK_DN_MM_N tokens on the projections run on MFMA instead (proj_mm.hip):
+ * x packed once into operand planes, one grouped product for qkv | z and one
+ * for a | b, and k_dn_pack in place of k_dn_out's scaling and conv state.
+ * The GEMVs above walk the tokens one after another and convert x again in
+ * every wave: at 2048 tokens (hidden 2048, heads 16/32 of 128) 10050 us for
+ * k_dn_in and 5830 for k_dn_out, against 300 + 15 and 110 + 12.
+ *
  * Sums run in parallel orders (lane trees), so results match the reference
  * to rounding, not bit for bit.
  */
@@ -427,6 +434,66 @@ __global__ __launch_bounds__(256) void k_dn_out(DnOutArgs a) {
     }
 }
 
+/*
+ * Many tokens: core scaled by its head's 1/sqrt(sum(o^2)/dv + eps) as
+ * operand planes of out_proj (k_pack_rows' arithmetic and order), one
+ * thread per 8 columns; the workgroups past the planes move the conv state
+ * on by n tokens.
+ */
+struct DnPackArgs {
+    const float *core, *ssp, *mixed;
+    float *conv_state;
+    uint16_t *hi, *lo;
+    float *pg;
+    int n, value_dim, dv, kc, conv_dim;
+};
+
+__global__ __launch_bounds__(256) void k_dn_pack(DnPackArgs a) {
+    const size_t nch = (size_t)a.n * (a.value_dim / 8);
+    const unsigned pack_wgs = (unsigned)(nch / 256 + 1);
+    if (blockIdx.x >= pack_wgs) {
+        const int cc = (int)(blockIdx.x - pack_wgs) * 256 + threadIdx.x;
+        if (cc >= a.conv_dim) return;
+        float cv[DN_KCMAX - 1];
+#pragma unroll
+        for (int j = 0; j < DN_KCMAX - 1; j++)
+            if (j < a.kc - 1) {
+                const int m = a.n + j;
+                cv[j] = m < a.kc - 1 ? a.conv_state[(size_t)m * a.conv_dim + cc]
+                                     : qk_ld(a.mixed + (size_t)(m - (a.kc - 1)) * a.conv_dim + cc);
+            }
+#pragma unroll
+        for (int j = 0; j < DN_KCMAX - 1; j++)
+            if (j < a.kc - 1) a.conv_state[(size_t)j * a.conv_dim + cc] = cv[j];
+        return;
+    }
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nch) return; /* nch is a multiple of 8: whole groups leave together */
+    const int cpr = a.value_dim / 8;
+    const size_t t = i / cpr;
+    const int col = (int)(i - t * cpr) * 8, nb = a.dv / DN_RB;
+    const float4 a0 = qk_ld((const float4 *)a.core + 2 * i), a1 = qk_ld((const float4 *)a.core + 2 * i + 1);
+    const float *sp = a.ssp + (t * (a.value_dim / a.dv) + col / a.dv) * nb;
+    float ss = 0.0f;
+    for (int j0 = 0; j0 < nb; j0 += 8) {
+        float pv[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) pv[j] = qk_ld(sp + min(j0 + j, nb - 1));
+#pragma unroll
+        for (int j = 0; j < 8; j++) ss = ss + (j0 + j < nb ? pv[j] : 0.0f);
+    }
+    const float r = 1.0f / sqrtf(ss / (float)a.dv + 1e-6f);
+    const float v[8] = {a0.x * r, a0.y * r, a0.z * r, a0.w * r, a1.x * r, a1.y * r, a1.z * r, a1.w * r};
+    uint32_t ph[4], pl[4];
+    float s = qk_f32x8_pairs(v, ph, pl);
+    ((uint4 *)a.hi)[i] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
+    ((uint4 *)a.lo)[i] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
+    s += qk_dpp<QK_DPP_XOR1>(s);
+    s += qk_dpp<QK_DPP_XOR2>(s);
+    s += __shfl_xor(s, 4, QK_WAVE);
+    if ((i & 7) == 0) a.pg[i >> 3] = -128.0f * s;
+}
+
 /* ------------------------------------------------------------ host side */
 
 extern "C" int qk_dn_shape_ok(const qk_dn_shape *s) {
@@ -448,13 +515,32 @@ extern "C" int qk_dn_shape_ok(const qk_dn_shape *s) {
 
 extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const float *x, int n, float *out,
                             float *conv_state, float *rec_state, float *mixed, float *z, float *av,
-                            float *bv, float *core, float *ssp, const qk_inject *inj_in, void *stream) {
+                            float *bv, float *core, float *ssp, const qk_planes *pl, const qk_inject *inj_in,
+                            void *stream) {
     if (n <= 0) return 0;
     if (!qk_dn_shape_ok(s)) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)stream;
     const int key_dim = s->hk * s->dk, value_dim = s->hv * s->dv;
     const int conv_dim = 2 * key_dim + value_dim;
-
+    const bool inj = inj_in && inj_in->hyper;
+    if (inj && (inj_in->hc < 1 || inj_in->hc > QK_INJECT_MAX_HC || !inj_in->inject)) return (int)hipErrorInvalidValue;
+    int rc;
+    const bool mm = n >= QK_DN_MM_N;
+    if (mm) {
+        if (!pl || !pl->hi || !pl->lo || !pl->pg) return (int)hipErrorInvalidValue;
+        rc = qk_launch_pack_rows(x, 0, (size_t)n, s->d, pl->hi, pl->lo, pl->pg, stream);
+        if (rc) return rc;
+        qk_proj p = {};
+        p.seg[0] = {W->qkv_q, W->qkv_s, W->qkv_b, mixed, conv_dim, conv_dim};
+        p.seg[1] = {W->z_q, W->z_s, W->z_b, z, value_dim, value_dim};
+        p.nseg = 2;
+        p.hi = pl->hi; p.lo = pl->lo; p.pg = pl->pg;
+        p.K = s->d; p.n = n;
+        rc = qk_launch_proj(&p, stream);
+        if (rc) return rc;
+        rc = qk_launch_proj_bf16(W->a_w, W->b_w, s->hv, pl->hi, pl->lo, s->d, n, av, bv, stream);
+        if (rc) return rc;
+    } else {
     DnInArgs ia;
     ia.qkv_q = W->qkv_q; ia.qkv_s = W->qkv_s; ia.qkv_b = W->qkv_b;
     ia.z_q = W->z_q; ia.z_s = W->z_s; ia.z_b = W->z_b;
@@ -471,8 +557,9 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     case 3: hipLaunchKernelGGL(k_dn_in<3>, igrid, dim3(256), 0, st, ia); break;
     default: hipLaunchKernelGGL(k_dn_in<4>, igrid, dim3(256), 0, st, ia); break;
     }
-    int rc = QK_CHECK_LAUNCH();
+    rc = QK_CHECK_LAUNCH();
     if (rc) return rc;
+    }
 
     DnRecArgs ra;
     ra.mixed = mixed; ra.a = av; ra.b = bv;
@@ -492,12 +579,25 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     rc = QK_CHECK_LAUNCH();
     if (rc) return rc;
 
+    if (mm) {
+        const DnPackArgs ka = {core, ssp, mixed, conv_state, pl->hi, pl->lo, pl->pg, n, value_dim, s->dv, s->kc, conv_dim};
+        hipLaunchKernelGGL(k_dn_pack, dim3((unsigned)((size_t)n * (value_dim / 8) / 256 + 1 + (conv_dim + 255) / 256)),
+                           dim3(256), 0, st, ka);
+        rc = QK_CHECK_LAUNCH();
+        if (rc) return rc;
+        qk_proj p = {};
+        p.seg[0] = {W->out_q, W->out_s, W->out_b, out, s->d, s->d};
+        p.nseg = 1;
+        p.hi = pl->hi; p.lo = pl->lo; p.pg = pl->pg;
+        p.K = value_dim; p.n = n;
+        if (inj) { p.hyper = inj_in->hyper; p.inject = inj_in->inject; p.hc = inj_in->hc; }
+        return qk_launch_proj(&p, stream);
+    }
+
     DnOutArgs oa;
     oa.out_q = W->out_q; oa.out_s = W->out_s; oa.out_b = W->out_b;
     oa.core = core; oa.ssp = ssp; oa.mixed = mixed;
     oa.conv_state = conv_state; oa.out = out;
-    const bool inj = inj_in && inj_in->hyper;
-    if (inj && (inj_in->hc < 1 || inj_in->hc > QK_INJECT_MAX_HC || !inj_in->inject)) return (int)hipErrorInvalidValue;
     oa.hyper = inj ? inj_in->hyper : nullptr;
     oa.inject = inj ? inj_in->inject : nullptr;
     oa.hc = inj ? inj_in->hc : 1;

@@ -1,0 +1,493 @@
+/*
+ * proj_mm.hip -- the mixers' q4 projections for many tokens on bf16 MFMA
+ * (v_mfma_f32_32x32x16_bf16): out[t, r] = x[t] . W[r] for the row segments
+ * of one input (DeltaNet in_proj_qkv | in_proj_z, and out_proj; attention
+ * q | k | v, and o_proj), replacing the per-token GEMVs of linear_forward
+ * (reference c/src/model.c:193-202 -> gemm_q4, kernel.c:230-309).
+ *
+ * The arithmetic is the expert GEMM's (ffn_mfma.hip): f32 activations as
+ * bf16 hi + lo planes in (x_i, x_{i+4}) pair order (k_pack_rows), codes as
+ * the exact bf16 numbers 16 + q, every 64-column group's accumulator
+ * started at -16 sum(x) so it ends at sum x q, one fp32 fma per output
+ * and group for the scale, and the bias term sum_g b_g X_g as a K = G
+ * product at the end.  Accumulation is fp32 throughout, as in the GEMV.
+ *
+ * Bound: matrix cores (n = 2048: 103 GFLOP for qkv | z, twice that issued
+ * for hi + lo).  Measured 300 us there, 343 TFLOP/s (687 issued); the matrix
+ * cores are busy 31 % of the time, the rest goes to the decode, the scale
+ * fmas and the waits between them.
+ *
+ * 32x32x16 lane layout: A lane l holds row l%32, B lane l column l%32, both
+ * eight K elements of half h = l/32; D lane l holds column l%32, rows
+ * 8*(i/4) + 4*h + i%4.  K-step j of a group gives half h the chunk 4*h + j
+ * (8 columns, one code word), so a lane's four code words of a group are
+ * one 16-byte load.
+ */
+#include "qk_device.h"
+#include "mfma_parts.h"
+
+typedef float qm_f32x16 __attribute__((ext_vector_type(16)));
+
+/* one code word -> the B operand: bf16 16 + q (0x4180 | q << 3, exact: the
+ * ulp in [16, 32) is 1/8) in (q_i, q_{i+4}) pair order.  The offset is what
+ * the running sums carry until the group ends, so its size sets their
+ * rounding: with 128 + q (one instruction fewer) out_proj's error against
+ * 64 bits at 4096 columns was 9.6e-6, more than the per-token GEMV's 9.3e-6 */
+__device__ __forceinline__ qm_bf16x8 pj_codes(uint32_t w) {
+    const uint32_t lo = ((w << 3) & 0x78787878u) | 0x80808080u, hi = ((w >> 1) & 0x78787878u) | 0x80808080u;
+    const uint32_t k = 0x41414141u;
+    return __builtin_bit_cast(qm_bf16x8,
+                              make_uint4(__builtin_amdgcn_perm(k, lo, 0x04020400u), __builtin_amdgcn_perm(k, hi, 0x04020400u),
+                                         __builtin_amdgcn_perm(k, lo, 0x04030401u), __builtin_amdgcn_perm(k, hi, 0x04030401u)));
+}
+#define PJ_P 0.125f /* -16 X from the planes' P = -128 X */
+
+#define PJ_THREADS 256
+#define QK_PROJ_FEW_N 320
+
+/* the segment and local first row of column block cb (64 columns); false
+ * past the last one */
+__device__ __forceinline__ bool pj_segment(const qk_proj &a, int cb, const uint32_t *&q, const uint16_t *&s,
+                                           const uint16_t *&b, float *&out, int &ostride, int &r0) {
+    int sg = 0, base = 0;
+    if (a.nseg > 1 && cb >= a.end64[0]) { sg = 1; base = a.end64[0]; }
+    if (a.nseg > 2 && cb >= a.end64[1]) { sg = 2; base = a.end64[1]; }
+    q = a.seg[0].q; s = a.seg[0].s; b = a.seg[0].b; out = a.seg[0].out; ostride = a.seg[0].ostride;
+    if (sg == 1) { q = a.seg[1].q; s = a.seg[1].s; b = a.seg[1].b; out = a.seg[1].out; ostride = a.seg[1].ostride; }
+    if (sg == 2) { q = a.seg[2].q; s = a.seg[2].s; b = a.seg[2].b; out = a.seg[2].out; ostride = a.seg[2].ostride; }
+    r0 = (cb - base) * 64;
+    return cb < a.end64[a.nseg - 1];
+}
+
+/* eight group sums P of a row from group k0 on (0 past G) as X = P / -128 in
+ * three bf16 parts, 24 bits: with a zero point inside the code range the
+ * bias term is as large as the code term and cancels most of it, so two
+ * parts (2^-17 of it) would show in the result */
+__device__ __forceinline__ void pj_bias_x(const float *pg, int k0, int G, qm_bf16x8 (&X)[3]) {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float p0 = qk_ld(pg + min(k0 + 2 * j, G - 1)), p1 = qk_ld(pg + min(k0 + 2 * j + 1, G - 1));
+        float x0 = k0 + 2 * j < G ? p0 * (-1.0f / 128.0f) : 0.0f;
+        float x1 = k0 + 2 * j + 1 < G ? p1 * (-1.0f / 128.0f) : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            w[i][j] = qk_cvt_pk_bf16(x0, x1);
+            x0 = x0 - qk_bf16_lo(w[i][j]);
+            x1 = x1 - qk_bf16_hi(w[i][j]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) X[i] = __builtin_bit_cast(qm_bf16x8, make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]));
+}
+
+/* the bias words b[col][k0 .. k0+8) (0 past G), one load each: a row of
+ * biases is only 2-byte aligned when G is odd */
+__device__ __forceinline__ qm_bf16x8 pj_bias_w(const uint16_t *bp, int k0, int G) {
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t b0 = qk_ld(bp + min(k0 + 2 * j, G - 1)), b1 = qk_ld(bp + min(k0 + 2 * j + 1, G - 1));
+        w[j] = (k0 + 2 * j < G ? b0 : 0u) | ((k0 + 2 * j + 1 < G ? b1 : 0u) << 16);
+    }
+    return __builtin_bit_cast(qm_bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+}
+
+#define PJ_MFMA(A, B, C) __builtin_amdgcn_mfma_f32_32x32x16_bf16((A), (B), (C), 0, 0, 0)
+
+/* one output: the store, and with INJ the gated residual's update */
+template <bool INJ>
+__device__ __forceinline__ void pj_store(const qk_proj &a, float *out, int ostride, int t, int r, float v) {
+    if (out) qk_st(out + (size_t)t * ostride + r, v);
+    if (INJ)
+        for (int j = 0; j < a.hc; j++) {
+            float *hp = a.hyper + ((size_t)t * a.hc + j) * ostride + r;
+            qk_st(hp, fmaf(qk_ld(a.inject + (size_t)t * a.hc + j), v, qk_ld(hp)));
+        }
+}
+
+/*
+ * Tiles of BM = 32*RT*WR tokens x BN = 64*(4/WR) columns; wave (wr, wc) owns
+ * RT row tiles and two column tiles.  Per group the rows' planes go through
+ * LDS (two buffers, one barrier, 16-byte chunks xor-swizzled by row so a
+ * wave's reads touch every bank), loaded into registers one group ahead;
+ * code words and scales come straight into registers one group ahead.
+ */
+template <int RT, int WR, bool INJ>
+__global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
+    constexpr int BM = 32 * RT * WR, WC = 4 / WR;
+    constexpr int ACH = BM * 8 / PJ_THREADS; /* chunks per thread and plane */
+    __shared__ __attribute__((aligned(16))) uint4 s_a[2][2][BM * 8];
+    __shared__ __attribute__((aligned(16))) float s_p[2][BM];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = lane & 31, h = lane >> 5;
+    const int wr = wave % WR, wc = wave / WR;
+    /* workgroups go round-robin over the 8 XCDs: the row tiles of one column
+     * tile are consecutive workgroups of one XCD and share its L2 copy of
+     * the weights */
+    const int per = (a.mtiles * a.ntiles + 7) >> 3;
+    const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (id >= a.mtiles * a.ntiles) return;
+    const int nt = id / a.mtiles, mt = id - nt * a.mtiles;
+    const int m0 = mt * BM;
+    const int G = a.K >> 6;
+    const size_t wrow = (size_t)a.K >> 3;
+
+    const uint32_t *q;
+    const uint16_t *s, *b;
+    float *out;
+    int ostride, r0;
+    const int cb = nt * WC + wc;
+    const bool live = pj_segment(a, min(cb, a.end64[a.nseg - 1] - 1), q, s, b, out, ostride, r0) &&
+                      cb < a.end64[a.nseg - 1];
+    const uint32_t *wq[2];
+    const uint16_t *sp[2];
+#pragma unroll
+    for (int ct = 0; ct < 2; ct++) {
+        wq[ct] = q + (size_t)(r0 + 32 * ct + c) * wrow + 4 * h;
+        sp[ct] = s + (size_t)(r0 + 32 * ct + c) * G;
+    }
+
+    const uint16_t *ap[ACH];
+#pragma unroll
+    for (int i = 0; i < ACH; i++) {
+        const int ci = tid + PJ_THREADS * i;
+        ap[i] = a.hi + (size_t)min(m0 + (ci >> 3), a.n - 1) * a.K + (ci & 7) * 8;
+    }
+    const size_t lo_off = a.lo - a.hi;
+    uint4 ar[2][ACH];
+    float pr = 0.0f;
+    auto load_a = [&](int g) {
+#pragma unroll
+        for (int i = 0; i < ACH; i++) {
+            ar[0][i] = qk_ld((const uint4 *)(ap[i] + 64 * g));
+            ar[1][i] = qk_ld((const uint4 *)(ap[i] + lo_off + 64 * g));
+        }
+        pr = qk_ld(a.pg + (size_t)min(m0 + min(tid, BM - 1), a.n - 1) * G + g);
+    };
+    auto store_a = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < ACH; i++) {
+            const int ci = tid + PJ_THREADS * i, row = ci >> 3, kc = ci & 7;
+            s_a[buf][0][row * 8 + (kc ^ (row & 7))] = ar[0][i];
+            s_a[buf][1][row * 8 + (kc ^ (row & 7))] = ar[1][i];
+        }
+        if (tid < BM) s_p[buf][tid] = pr * PJ_P;
+    };
+    uint4 wv[2];
+    uint16_t sv[2];
+    auto load_w = [&](int g) {
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) {
+            wv[ct] = qk_ld((const uint4 *)(wq[ct] + 8 * g));
+            sv[ct] = qk_ld(sp[ct] + g);
+        }
+    };
+    qm_f32x16 acc[RT][2];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[rt][ct][i] = 0.0f;
+
+    load_a(0);
+    load_w(0);
+    for (int g = 0; g < G; g++) {
+        const int buf = g & 1;
+        store_a(buf);
+        qm_bf16x8 bop[2][4];
+        float sc[2];
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) {
+            bop[ct][0] = pj_codes(wv[ct].x);
+            bop[ct][1] = pj_codes(wv[ct].y);
+            bop[ct][2] = pj_codes(wv[ct].z);
+            bop[ct][3] = pj_codes(wv[ct].w);
+            sc[ct] = qk_bf16(sv[ct]);
+        }
+        const int gn = min(g + 1, G - 1); /* past the end: loaded, not used */
+        load_a(gn);
+        load_w(gn);
+        /* buffer buf was last read in group g-2, before the barrier of g-1 */
+        qk_lds_barrier();
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            const int row = 32 * (RT * wr + rt) + c;
+            qm_f32x16 p;
+#pragma unroll
+            for (int i4 = 0; i4 < 4; i4++) {
+                const qm_f32x4 v = *(const qm_f32x4 *)&s_p[buf][32 * (RT * wr + rt) + 8 * i4 + 4 * h];
+#pragma unroll
+                for (int i = 0; i < 4; i++) p[4 * i4 + i] = v[i];
+            }
+            qm_f32x16 t[2];
+#pragma unroll
+            for (int tm = 0; tm < 2; tm++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const qm_bf16x8 A = __builtin_bit_cast(qm_bf16x8, s_a[buf][tm][row * 8 + ((4 * h + j) ^ (row & 7))]);
+#pragma unroll
+                    for (int ct = 0; ct < 2; ct++) t[ct] = PJ_MFMA(A, bop[ct][j], (tm == 0 && j == 0) ? p : t[ct]);
+                }
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[rt][ct][i] = fmaf(sc[ct], t[ct][i], acc[rt][ct][i]);
+        }
+    }
+
+    /* bias term: acc += sum_g b[col][g] X[row][g] */
+    for (int k0 = 0; k0 < G; k0 += 16) {
+        qm_bf16x8 bb[2];
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) bb[ct] = pj_bias_w(b + (size_t)(r0 + 32 * ct + c) * G, k0 + 8 * h, G);
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            qm_bf16x8 X[3];
+            pj_bias_x(a.pg + (size_t)min(m0 + 32 * (RT * wr + rt) + c, a.n - 1) * G, k0 + 8 * h, G, X);
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+                for (int i = 0; i < 3; i++) acc[rt][ct] = PJ_MFMA(X[i], bb[ct], acc[rt][ct]);
+        }
+    }
+    if (!live) return;
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int t = m0 + 32 * (RT * wr + rt) + 8 * (i >> 2) + 4 * h + (i & 3);
+            if (t < a.n)
+#pragma unroll
+                for (int ct = 0; ct < 2; ct++) pj_store<INJ>(a, out, ostride, t, r0 + 32 * ct + c, acc[rt][ct][i]);
+        }
+}
+
+/*
+ * Few tokens: 32 tokens x 32*CT columns per workgroup, the K groups dealt to
+ * its WK waves (wave w: groups w, w + WK, ..) and their sums added through
+ * LDS in wave order.  A tile of 32 rows leaves too few workgroups of the
+ * tiles above to fill the chip, and each would walk the whole K alone; here
+ * a wave walks K / WK with its operands read straight from the planes (the
+ * workgroup's rows are L1/L2 hits), no LDS and no barrier in the loop.
+ */
+template <int CT, int WK, bool INJ>
+__global__ __launch_bounds__(64 * WK) void k_proj_few(qk_proj a) {
+    __shared__ float s_r[WK][32][32 * CT + 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = lane & 31, h = lane >> 5;
+    const int nt = blockIdx.x, m0 = blockIdx.y * 32;
+    const int G = a.K >> 6;
+    const size_t wrow = (size_t)a.K >> 3;
+    const uint32_t *q;
+    const uint16_t *s, *b;
+    float *out;
+    int ostride, r0;
+    pj_segment(a, nt * CT / 2, q, s, b, out, ostride, r0);
+    if (CT == 1) r0 += 32 * (nt & 1);
+    const uint32_t *wq[CT];
+    const uint16_t *sp[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+        wq[ct] = q + (size_t)(r0 + 32 * ct + c) * wrow + 4 * h;
+        sp[ct] = s + (size_t)(r0 + 32 * ct + c) * G;
+    }
+    const size_t lo_off = a.lo - a.hi;
+    const uint16_t *ap = a.hi + (size_t)min(m0 + c, a.n - 1) * a.K + 32 * h;
+    uint4 wv[CT], av[2][4];
+    uint16_t sv[CT];
+    float pv[16];
+    auto load = [&](int g) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+            wv[ct] = qk_ld((const uint4 *)(wq[ct] + 8 * g));
+            sv[ct] = qk_ld(sp[ct] + g);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            av[0][j] = qk_ld((const uint4 *)(ap + 64 * g) + j);
+            av[1][j] = qk_ld((const uint4 *)(ap + lo_off + 64 * g) + j);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            pv[i] = qk_ld(a.pg + (size_t)min(m0 + 8 * (i >> 2) + 4 * h + (i & 3), a.n - 1) * G + g);
+    };
+    qm_f32x16 acc[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[ct][i] = 0.0f;
+    if (wave < G) load(wave);
+    for (int g = wave; g < G; g += WK) {
+        qm_bf16x8 A[2][4], bop[CT][4];
+        float sc[CT];
+        qm_f32x16 t[CT];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            A[0][j] = __builtin_bit_cast(qm_bf16x8, av[0][j]);
+            A[1][j] = __builtin_bit_cast(qm_bf16x8, av[1][j]);
+        }
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+            bop[ct][0] = pj_codes(wv[ct].x);
+            bop[ct][1] = pj_codes(wv[ct].y);
+            bop[ct][2] = pj_codes(wv[ct].z);
+            bop[ct][3] = pj_codes(wv[ct].w);
+            sc[ct] = qk_bf16(sv[ct]);
+#pragma unroll
+            for (int i = 0; i < 16; i++) t[ct][i] = pv[i] * PJ_P;
+        }
+        load(min(g + WK, G - 1));
+#pragma unroll
+        for (int tm = 0; tm < 2; tm++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) t[ct] = PJ_MFMA(A[tm][j], bop[ct][j], t[ct]);
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[ct][i] = fmaf(sc[ct], t[ct][i], acc[ct][i]);
+    }
+    /* bias term, 16 groups per step, the steps dealt to the waves */
+    for (int k0 = 16 * wave; k0 < G; k0 += 16 * WK) {
+        qm_bf16x8 X[3];
+        pj_bias_x(a.pg + (size_t)min(m0 + c, a.n - 1) * G, k0 + 8 * h, G, X);
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+            const qm_bf16x8 bb = pj_bias_w(b + (size_t)(r0 + 32 * ct + c) * G, k0 + 8 * h, G);
+#pragma unroll
+            for (int i = 0; i < 3; i++) acc[ct] = PJ_MFMA(X[i], bb, acc[ct]);
+        }
+    }
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) s_r[wave][8 * (i >> 2) + 4 * h + (i & 3)][32 * ct + c] = acc[ct][i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 32 * 32 * CT; i += 64 * WK) {
+        const int row = i / (32 * CT), col = i - row * (32 * CT);
+        if (m0 + row >= a.n) break; /* rows ascend with i */
+        float v = s_r[0][row][col];
+#pragma unroll
+        for (int w = 1; w < WK; w++) v = v + s_r[w][row][col];
+        pj_store<INJ>(a, out, ostride, m0 + row, r0 + col, v);
+    }
+}
+
+/*
+ * bf16 weight rows (DeltaNet in_proj_a | in_proj_b, 2*hv of them) on the
+ * same planes: workgroup = 32 tokens x 32 rows, K dealt to four waves.
+ */
+struct PjBf16Args {
+    const uint16_t *w[2];  /* [rows, K] each */
+    float *out[2];         /* [n, rows] */
+    const uint16_t *hi, *lo;
+    int rows, K, n;
+};
+
+__global__ __launch_bounds__(256) void k_proj_bf16(PjBf16Args a) {
+    __shared__ float s_r[4][32][33];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = lane & 31, h = lane >> 5;
+    const int m0 = blockIdx.y * 32, col = blockIdx.x * 32 + c;
+    const int cc = min(col, 2 * a.rows - 1);
+    const uint16_t *wp = (cc < a.rows ? a.w[0] + (size_t)cc * a.K : a.w[1] + (size_t)(cc - a.rows) * a.K) + 32 * h;
+    const size_t lo_off = a.lo - a.hi;
+    const uint16_t *ap = a.hi + (size_t)min(m0 + c, a.n - 1) * a.K + 32 * h;
+    const int G = a.K >> 6;
+    qm_f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i] = 0.0f;
+    uint4 av[2][4], wv[4];
+    auto load = [&](int g) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            av[0][j] = qk_ld((const uint4 *)(ap + 64 * g) + j);
+            av[1][j] = qk_ld((const uint4 *)(ap + lo_off + 64 * g) + j);
+            wv[j] = qk_ld((const uint4 *)(wp + 64 * g) + j);
+        }
+    };
+    if (wave < G) load(wave);
+    for (int g = wave; g < G; g += 4) {
+        qm_bf16x8 A[2][4], B[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            uint32_t p[4];
+            qk_bf16x8_to_pairs(wv[j], p);
+            B[j] = __builtin_bit_cast(qm_bf16x8, make_uint4(p[0], p[1], p[2], p[3]));
+            A[0][j] = __builtin_bit_cast(qm_bf16x8, av[0][j]);
+            A[1][j] = __builtin_bit_cast(qm_bf16x8, av[1][j]);
+        }
+        load(min(g + 4, G - 1));
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            acc = PJ_MFMA(A[0][j], B[j], acc);
+            acc = PJ_MFMA(A[1][j], B[j], acc);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) s_r[wave][8 * (i >> 2) + 4 * h + (i & 3)][c] = acc[i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 32 * 32; i += 256) {
+        const int row = i >> 5, r = blockIdx.x * 32 + (i & 31);
+        if (m0 + row >= a.n || r >= 2 * a.rows) continue;
+        const float v = ((s_r[0][row][i & 31] + s_r[1][row][i & 31]) + s_r[2][row][i & 31]) + s_r[3][row][i & 31];
+        const int k = r >= a.rows;
+        qk_st(a.out[k] + (size_t)(m0 + row) * a.rows + (r - k * a.rows), v);
+    }
+}
+
+/* ------------------------------------------------------------ host side */
+
+extern "C" int qk_launch_proj(const qk_proj *in, void *stream) {
+    qk_proj a = *in;
+    if (a.n <= 0) return 0;
+    if (a.K <= 0 || a.K % 64 || a.nseg < 1 || a.nseg > QK_PROJ_SEGS || (a.hyper && (a.nseg != 1 || a.hc < 1)))
+        return (int)hipErrorInvalidValue;
+    int end = 0;
+    for (int i = 0; i < a.nseg; i++) {
+        if (a.seg[i].rows <= 0 || a.seg[i].rows % 64) return (int)hipErrorInvalidValue;
+        end += a.seg[i].rows / 64;
+        a.end64[i] = end;
+    }
+    hipStream_t st = (hipStream_t)stream;
+    const bool inj = a.hyper != nullptr;
+#define PJ_MM(RT, WR)                                                                                        \
+    do {                                                                                                     \
+        a.mtiles = (a.n + 32 * RT * WR - 1) / (32 * RT * WR);                                                \
+        a.ntiles = (end + 4 / WR - 1) / (4 / WR);                                                            \
+        const dim3 grid(((unsigned)(a.mtiles * a.ntiles) + 7) / 8 * 8);                                      \
+        if (inj) hipLaunchKernelGGL((k_proj_mm<RT, WR, true>), grid, dim3(PJ_THREADS), 0, st, a);            \
+        else hipLaunchKernelGGL((k_proj_mm<RT, WR, false>), grid, dim3(PJ_THREADS), 0, st, a);               \
+    } while (0)
+#define PJ_FEW(CT, WK)                                                                                       \
+    do {                                                                                                     \
+        const dim3 grid(end * 2 / CT, (a.n + 31) / 32);                                                      \
+        if (inj) hipLaunchKernelGGL((k_proj_few<CT, WK, true>), grid, dim3(64 * WK), 0, st, a);              \
+        else hipLaunchKernelGGL((k_proj_few<CT, WK, false>), grid, dim3(64 * WK), 0, st, a);                 \
+    } while (0)
+    /* The K-split tiles while the others would leave the chip short of
+     * workgroups (DeltaNet mixer of hidden 2048, both products, us without
+     * the recurrence: 77 tokens 85 against 120, 256 tokens 133 / 145, 512
+     * tokens 245 / 200; up to 32 tokens the narrower one, 9 tokens 47
+     * against 52); 128-row tiles once they give every CU four workgroups
+     * (2048 tokens: 427 together, 64-row tiles 520). */
+    if (a.n <= 32) PJ_FEW(1, 4);
+    else if (a.n <= QK_PROJ_FEW_N) PJ_FEW(2, 4);
+    else if ((long long)((a.n + 127) / 128) * ((end + 1) / 2) < 1024) PJ_MM(1, 2);
+    else PJ_MM(2, 2);
+#undef PJ_MM
+#undef PJ_FEW
+    return QK_CHECK_LAUNCH();
+}
+
+extern "C" int qk_launch_proj_bf16(const uint16_t *w0, const uint16_t *w1, int rows, const uint16_t *hi,
+                                   const uint16_t *lo, int K, int n, float *out0, float *out1, void *stream) {
+    if (n <= 0) return 0;
+    if (K <= 0 || K % 64 || rows <= 0) return (int)hipErrorInvalidValue;
+    const PjBf16Args a = {{w0, w1}, {out0, out1}, hi, lo, rows, K, n};
+    hipLaunchKernelGGL(k_proj_bf16, dim3((2 * rows + 31) / 32, (n + 31) / 32), dim3(256), 0, (hipStream_t)stream, a);
+    return QK_CHECK_LAUNCH();
+}

@@ -33,6 +33,7 @@ struct qmoe_dn_ctx {
     dn_layer *layers;
     void *scratch;
     float *mixed, *z, *a, *b, *core, *ssp;
+    qk_planes pl; /* NULLs when max_tokens stays below QK_DN_MM_N */
 };
 
 static void dn_set_err(qmoe_err *err, const char *fmt, ...) {
@@ -109,10 +110,11 @@ int qmoe_dn_create(qmoe_dn_ctx **out, const qmoe_dn_config *cfg, qmoe_err *err) 
     c->off[DT_COUNT] = total;
     c->layers = (dn_layer *)calloc((size_t)cfg->n_layers, sizeof(dn_layer));
     const size_t n = (size_t)cfg->max_tokens;
-    const size_t ssz[6] = {n * conv_dim * 4, n * value_dim * 4, n * hv * 4, n * hv * 4, n * value_dim * 4,
-                           n * (value_dim / 16) * 4};
-    size_t stot = 0, soff[6];
-    for (int i = 0; i < 6; i++) {
+    const size_t wide = n >= QK_DN_MM_N ? n * (d > value_dim ? d : value_dim) : 0;
+    const size_t ssz[9] = {n * conv_dim * 4, n * value_dim * 4, n * hv * 4, n * hv * 4, n * value_dim * 4,
+                           n * (value_dim / 16) * 4, wide * 2, wide * 2, wide / 64 * 4};
+    size_t stot = 0, soff[9];
+    for (int i = 0; i < 9; i++) {
         soff[i] = stot;
         stot = dn_align(stot + ssz[i]);
     }
@@ -128,6 +130,11 @@ int qmoe_dn_create(qmoe_dn_ctx **out, const qmoe_dn_config *cfg, qmoe_err *err) 
     c->b = (float *)(b + soff[3]);
     c->core = (float *)(b + soff[4]);
     c->ssp = (float *)(b + soff[5]);
+    if (wide) {
+        c->pl.hi = (uint16_t *)(b + soff[6]);
+        c->pl.lo = (uint16_t *)(b + soff[7]);
+        c->pl.pg = (float *)(b + soff[8]);
+    }
     for (int l = 0; l < cfg->n_layers; l++) {
         if (dn_hip_fail(err, (int)hipMalloc(&c->layers[l].mem, total), "layer weights")) {
             qmoe_dn_destroy(c);
@@ -249,7 +256,7 @@ static int dn_forward(qmoe_dn_ctx *c, int layer, const float *x, int n, float *o
     W.dt_bias = (const float *)dn_ptr(c, layer, DT_DT_BIAS);
     const int rc = qk_launch_dn(&c->shape, &W, x, n, out, (float *)dn_ptr(c, layer, DT_CONV_STATE),
                                 (float *)dn_ptr(c, layer, DT_REC_STATE), c->mixed, c->z, c->a, c->b,
-                                c->core, c->ssp, inj, stream);
+                                c->core, c->ssp, &c->pl, inj, stream);
     return dn_hip_fail(err, rc, "DeltaNet launch");
 }
 

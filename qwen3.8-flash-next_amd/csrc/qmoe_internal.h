@@ -202,6 +202,54 @@ int qk_launch_combine(qk_shape s, int n, const float *y, const int32_t *pos, con
                       const float *sg, const void *x_res, int x_bf16, float *out, float *hyper,
                       const float *inject, int hc, void *stream);
 
+/* the gated residual's update after a mixer, fused into the mixer's last
+ * launch: hyper[t, j] = fma(inject[t, j], out[t], hyper[t, j]) for j < hc,
+ * the arithmetic of qk_launch_hc_inject (hyper NULL or no struct: none) */
+#define QK_INJECT_MAX_HC 8
+typedef struct {
+    float *hyper;         /* [n, hc, d] */
+    const float *inject;  /* [n, hc] */
+    int hc;
+} qk_inject;
+
+/* the mixers' q4 projections of many tokens on MFMA (proj_mm.hip): every
+ * segment's out[t * ostride + r] = x[t] . W[r] over operand planes hi, lo
+ * [n, K] and pg [n, K/64] of qk_launch_pack_rows (f32 rows).  rows and K
+ * are multiples of 64.  With hyper set (one segment): also the inject
+ * update of its output, [n, hc, ostride]; out may then be NULL. */
+#define QK_PROJ_SEGS 3
+typedef struct {
+    const uint32_t *q;     /* [rows, K/8] */
+    const uint16_t *s, *b; /* [rows, K/64] */
+    float *out;
+    int rows, ostride;
+} qk_proj_seg;
+typedef struct {
+    qk_proj_seg seg[QK_PROJ_SEGS];
+    int nseg;
+    const uint16_t *hi, *lo;
+    const float *pg;
+    int K, n;
+    float *hyper;
+    const float *inject;
+    int hc;
+    int end64[QK_PROJ_SEGS], mtiles, ntiles; /* filled by the launcher */
+} qk_proj;
+int qk_launch_proj(const qk_proj *a, void *stream);
+/* two bf16 matrices of `rows` rows on the same planes -> out0, out1 [n, rows] */
+int qk_launch_proj_bf16(const uint16_t *w0, const uint16_t *w1, int rows, const uint16_t *hi,
+                        const uint16_t *lo, int K, int n, float *out0, float *out1, void *stream);
+/* the mixers take these from this many tokens on.  The per-token GEMVs cost
+ * 9 us a token in DeltaNet and 3 us in attention at hidden 2048 (6 tokens: 66
+ * and 44 us the mixer, 9 tokens 94 and 53), these 57 and 48 us up to 9. */
+#define QK_DN_MM_N 6
+#define QK_AT_MM_N 9
+/* operand planes of a mixer call, in its scratch: hi, lo [n, K], pg [n, K/64] */
+typedef struct {
+    uint16_t *hi, *lo;
+    float *pg;
+} qk_planes;
+
 /* the gated DeltaNet mixer (deltanet.hip) */
 typedef struct {
     int d, hk, hv, dk, dv, kc; /* hidden, key/value heads, head dims, conv taps */
@@ -215,20 +263,11 @@ typedef struct {
 int qk_dn_shape_ok(const qk_dn_shape *s);
 /* x [n, d] f32 -> out [n, d]; conv_state and rec_state are updated;
  * mixed [n, conv_dim], z [n, value_dim], a, b [n, hv], core [n, value_dim]
- * and ssp [n, hv, dv/16] are scratch */
-/* the gated residual's update after a mixer, fused into the mixer's last
- * launch: hyper[t, j] = fma(inject[t, j], out[t], hyper[t, j]) for j < hc,
- * the arithmetic of qk_launch_hc_inject (hyper NULL or no struct: none) */
-#define QK_INJECT_MAX_HC 8
-typedef struct {
-    float *hyper;         /* [n, hc, d] */
-    const float *inject;  /* [n, hc] */
-    int hc;
-} qk_inject;
-
+ * and ssp [n, hv, dv/16] are scratch; pl, planes of max(d, value_dim)
+ * columns, is used from QK_DN_MM_N tokens on (and may be all NULL below) */
 int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const float *x, int n, float *out,
                  float *conv_state, float *rec_state, float *mixed, float *z, float *a, float *b,
-                 float *core, float *ssp, const qk_inject *inj, void *stream);
+                 float *core, float *ssp, const qk_planes *pl, const qk_inject *inj, void *stream);
 int qk_launch_dn_zero(float *p, size_t count, void *stream);
 
 /* the full-attention mixer with the QSA indexer (attention.hip) */
@@ -254,6 +293,7 @@ typedef struct {
     float *part;  /* [n, h, nchunks, hd+2]: part_units (token, chunk) pairs per head */
     float *ao;    /* [n, h*hd] */
     uint32_t *skey; /* [n, cap/comp] order keys of the block scores */
+    qk_planes pl; /* planes of max(d, h*hd) columns, used from QK_AT_MM_N tokens on */
     long long part_units; /* capacity of part in (token, key chunk) pairs per head */
 } qk_at_scratch;
 int qk_at_shape_ok(const qk_at_shape *s);
