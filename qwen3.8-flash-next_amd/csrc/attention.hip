@@ -31,6 +31,8 @@
  *             exp-weighted v per head.
  *   k_at_comb one wave per (token, head): the chunks merged (max, rescaled
  *             sums), times sigmoid(gate).
+ *             From QK_AT_MM_N tokens on attn_mm.hip replaces these two; the
+ *             256-key kernel then serves calls of few tokens at long caches.
  * The indexer path (index_qk_proj in the router's R64 order, rmsnorm sums
  * in index order, the table's cos / sin, the block scores in the
  * reference's order) has the oracle's bits, so the kept blocks are the
@@ -174,7 +176,6 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
 
 #define AI_TOK 4 /* tokens per wave */
 #define AI_RB 4  /* rows per stage */
-#define AI_MIN_N 16
 static_assert(AI_TOK * AI_RB == 16, "a wave reduces 16 partials per lane");
 
 struct AtIdxArgs {
@@ -280,7 +281,7 @@ __global__ __launch_bounds__(256, 2) void k_at_idx(AtIdxArgs a) {
 }
 
 /* hidden sizes up to 2048 (a token's share of a wave is 32 registers there) */
-static bool at_idx_ok(int d, int n) { return n >= AI_MIN_N && d <= 2048; }
+static bool at_idx_ok(int d, int n) { return n >= QK_AT_MM_N && d <= 2048; }
 
 static int at_idx_launch(const float *x, const uint16_t *w, int d, int n, int rows, float *out, hipStream_t st) {
     AtIdxArgs a = {x, w, out, d, n, rows, 0};
@@ -1149,6 +1150,19 @@ extern "C" int qk_launch_at(const qk_at_shape *s, const qk_at_dev *W, const floa
         if (rc) return rc;
     }
 
+    if (mm) {
+        rc = qk_launch_attn_mm(s, n, offset - pos0, kv_total, sc->qn, sc->qg, k_cache, v_cache,
+                               use_idx ? sc->keep : nullptr, nb, kw, sc, stream);
+        if (rc) return rc;
+        qk_proj p = {};
+        p.seg[0] = {W->o_q, W->o_s, W->o_b, out, s->d, s->d};
+        p.nseg = 1;
+        p.hi = sc->pl.hi; p.lo = sc->pl.lo; p.pg = sc->pl.pg;
+        p.K = h * hd; p.n = n;
+        if (inj && inj->hyper) { p.hyper = inj->hyper; p.inject = inj->inject; p.hc = inj->hc; }
+        return qk_launch_proj(&p, stream);
+    }
+
     AtAttnArgs at;
     at.qn = sc->qn; at.k_cache = k_cache; at.v_cache = v_cache;
     at.keep = use_idx ? sc->keep : nullptr;
@@ -1175,18 +1189,6 @@ extern "C" int qk_launch_at(const qk_at_shape *s, const qk_at_dev *W, const floa
     else hipLaunchKernelGGL(k_at_comb<AT_MAXCH / 4>, dim3(n * h), dim3(256), 0, st, cb);
     rc = QK_CHECK_LAUNCH();
     if (rc) return rc;
-
-    if (mm) {
-        rc = qk_launch_pack_rows(sc->ao, 0, (size_t)n, h * hd, sc->pl.hi, sc->pl.lo, sc->pl.pg, stream);
-        if (rc) return rc;
-        qk_proj p = {};
-        p.seg[0] = {W->o_q, W->o_s, W->o_b, out, s->d, s->d};
-        p.nseg = 1;
-        p.hi = sc->pl.hi; p.lo = sc->pl.lo; p.pg = sc->pl.pg;
-        p.K = h * hd; p.n = n;
-        if (inj && inj->hyper) { p.hyper = inj->hyper; p.inject = inj->inject; p.hc = inj->hc; }
-        return qk_launch_proj(&p, stream);
-    }
 
     RowsArgs o;
     o.nseg = 0;

@@ -239,11 +239,14 @@ int qk_launch_proj(const qk_proj *a, void *stream);
 /* two bf16 matrices of `rows` rows on the same planes -> out0, out1 [n, rows] */
 int qk_launch_proj_bf16(const uint16_t *w0, const uint16_t *w1, int rows, const uint16_t *hi,
                         const uint16_t *lo, int K, int n, float *out0, float *out1, void *stream);
-/* the mixers take these from this many tokens on.  The per-token GEMVs cost
- * 9 us a token in DeltaNet and 3 us in attention at hidden 2048 (6 tokens: 66
- * and 44 us the mixer, 9 tokens 94 and 53), these 57 and 48 us up to 9. */
+/* the mixers take their matrix kernels from this many tokens on.  DeltaNet's
+ * per-token GEMVs cost 9 us a token at hidden 2048: 66 us the mixer at 6
+ * tokens, 94 at 9, against 57 and 63.  Attention's whole path (projections,
+ * indexer rows, attn_mm.hip) has more launches: at 9 tokens 50..71 us on the
+ * per-token kernels and 46..86 on these over four shapes, at 16 tokens 59..122
+ * against 37..97. */
 #define QK_DN_MM_N 6
-#define QK_AT_MM_N 9
+#define QK_AT_MM_N 16
 /* operand planes of a mixer call, in its scratch: hi, lo [n, K], pg [n, K/64] */
 typedef struct {
     uint16_t *hi, *lo;
@@ -294,9 +297,20 @@ typedef struct {
     float *ao;    /* [n, h*hd] */
     uint32_t *skey; /* [n, cap/comp] order keys of the block scores */
     qk_planes pl; /* planes of max(d, h*hd) columns, used from QK_AT_MM_N tokens on */
+    void *img;       /* qk_am_img_bytes: k and v as matrix operands */
+    uint32_t *kmask; /* qk_am_mask_bytes: key bits per token */
     long long part_units; /* capacity of part in (token, key chunk) pairs per head */
 } qk_at_scratch;
 int qk_at_shape_ok(const qk_at_shape *s);
+/* attention of many tokens on MFMA (attn_mm.hip): from the normed queries qn
+ * and the k and v rows [0, T) (the call's own included; token t sees the rows
+ * up to offset + t, and with keep only kept blocks and its own tail) to the
+ * gated output as operand planes in sc->pl */
+size_t qk_am_img_bytes(const qk_at_shape *s);
+size_t qk_am_mask_bytes(const qk_at_shape *s, int n);
+int qk_launch_attn_mm(const qk_at_shape *s, int n, int offset, int T, const float *qn, const float *qg,
+                      const float *k_cache, const float *v_cache, const uint32_t *keep, int nb, int kw,
+                      const qk_at_scratch *sc, void *stream);
 size_t qk_at_sel_lds(const qk_at_shape *s, int nb);
 /* x [n, d] f32 at positions offset.. -> out [n, d]; the caches hold len0
  * rows before the call and len0 + n after it (len0 + n <= cap); pooled

@@ -26,7 +26,49 @@ def test_deltanet_token_counts(torch_dev, shape, calls):
 
 
 @pytest.mark.parametrize("case", [(320, 5, 1, 64, 3, 68, 12, 3, 768, 1.0), (256, 4, 2, 64, 2, 64, 4096, 4, 768, 0.25)])
-@pytest.mark.parametrize("calls", [[8, 9, 31], [32, 33, 1, 64], [65, 1, 129], [320, 1, 321]])
+@pytest.mark.parametrize("calls", [[15, 16, 31], [32, 33, 1, 64], [65, 1, 129], [320, 1, 321]])
 def test_attention_token_counts(torch_dev, case, calls):
     torch, dev = torch_dev
     ta.run_calls(torch, dev, case, calls, seed=9)
+
+
+@pytest.mark.parametrize("hd,cap", [(64, 80), (128, 1100), (192, 80), (256, 80)])
+def test_attention_head_dims_and_ranges(torch_dev, hd, cap):
+    """every head dim of the matrix kernel, 3 query heads per kv head (rows
+    of one workgroup from uneven token groups), the last image of a call
+    partly filled, several key ranges at 1100 rows"""
+    torch, dev = torch_dev
+    n = cap - 12
+    ta.run_calls(torch, dev, (192, 6, 2, hd, 1, 64, 4096, 4, cap, 0.25), [n, 1, 11], seed=10)
+    ta.run_calls(torch, dev, (192, 6, 2, hd, 1, 64, 16, 4, cap, 0.25), [n, 1, 11], seed=11)
+
+
+@pytest.mark.parametrize("bad", ["nan", "inf", "1e30"])
+def test_attention_values_past_the_parts(torch_dev, bad):
+    """a token whose value no bf16 parts carry: the tokens before it are
+    those of the call without it, and the ones that see it are NaN (nan, inf)
+    or the oracle's (1e30: v rows of that size, keys and queries normed)"""
+    import numpy as np
+    torch, dev = torch_dev
+    case = (256, 4, 2, 64, 2, 64, 4096, 4, 64, 0.25)
+    n, j = 40, 17
+    A = ta.orc.Attention(*case[:8], kv_cap=64, rotary_factor=0.25, seed=12)
+    x = ta.orc.gen_attn_x(n, 256, 13)
+    outs = []
+    for v in (None, float(bad)):
+        xi = x.copy()
+        if v is not None:
+            xi[j, 5] = v
+        with ta.load_pkg().AttentionContext(*case[:8], kv_cap=64, rotary_factor=0.25, max_tokens=n) as ctx:
+            ctx.upload_layer(0, A.arrays())
+            outs.append(ctx.forward(0, torch.from_numpy(xi).to(dev), 0).cpu().numpy())
+    clean, got = outs
+    assert np.isfinite(clean).all()
+    # fp32 sums in another order: 2^-24 per term over 64 dims and 40 keys
+    assert ta.rel(got[:j], clean[:j]) < 1e-5
+    if bad == "1e30":
+        ref = A.forward(xi, A.new_state(), 0)
+        for t in range(j, n):
+            assert ta.rel(got[t], ref[t]) < ta.REL_L2, t
+    else:
+        assert np.isnan(got[j:]).all()
