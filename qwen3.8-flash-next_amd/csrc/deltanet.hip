@@ -31,16 +31,18 @@
  * for a | b, and k_dn_pack in place of k_dn_out's scaling and conv state.
  * The GEMVs above walk the tokens one after another and convert x again in
  * every wave: at 2048 tokens (hidden 2048, heads 16/32 of 128) 10050 us for
- * k_dn_in and 5830 for k_dn_out, against 300 + 15 and 110 + 12.
+ * k_dn_in and 5830 for k_dn_out, against 315 + 16 and 141 + 21.
+ * From QK_DN_CHUNK_N tokens on k_dn_rec gives way to dn_chunk.hip (3225 us
+ * there against 103 + 142).
  *
  * Sums run in parallel orders (lane trees), so results match the reference
  * to rounding, not bit for bit.
  */
 #include "qk_device.h"
 #include "gemv_parts.h"
+#include "dn_rec.h"
 
 #define DN_RPW 4   /* rows per wave in the two GEMV kernels */
-#define DN_RB 16   /* state rows per recurrence workgroup */
 
 struct DnInArgs {
     const uint32_t *qkv_q, *z_q;
@@ -146,62 +148,12 @@ __global__ __launch_bounds__(256) void k_dn_in(DnInArgs a) {
 
 /* ------------------------------------------------------------ recurrence */
 
-struct DnRecArgs {
-    const float *mixed, *a, *b;  /* [n, conv_dim], [n, hv], [n, hv] */
-    const float *conv_state;     /* [kc-1, conv_dim], the state before these tokens */
-    const uint16_t *conv_w;      /* [conv_dim, kc] */
-    const float *a_log, *dt_bias;
-    const float *z;              /* [n, value_dim] */
-    const float *norm_w;         /* [dv] */
-    float *rec_state;            /* [hv, dv, dk] */
-    float *core;                 /* [n, value_dim]: o * norm_w * sigmoid(z) */
-    float *ssp;                  /* [n, hv, dv/16]: sums of o^2 over each block's rows */
-    int n, hk, hv, dk, dv, kc, conv_dim;
-};
-
-/* silu(conv) of channels ch[0..NC) at token t: sum over taps i of
- * w[c, i] * seq[t+i, c] with seq = [conv_state rows; mixed rows], the fma
- * chain over i ascending.  The taps come four at a time with every load of
- * a round (all NC channels) in flight: a loop with a runtime trip count
- * would wait on each load.  Past kc the last tap is read again, unused. */
-template <int NC>
-__device__ __forceinline__ void dn_conv_silu(const DnRecArgs &a, int t, const int (&ch)[NC], float (&out)[NC]) {
-    float acc[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = 0.0f;
-    for (int i0 = 0; i0 < a.kc; i0 += 4) {
-        float sv[NC][4];
-        uint16_t wv[NC][4];
-#pragma unroll
-        for (int c = 0; c < NC; c++)
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int i = min(i0 + u, a.kc - 1), j = t + i;
-                const float *src = j < a.kc - 1 ? a.conv_state + (size_t)j * a.conv_dim + ch[c]
-                                                : a.mixed + (size_t)(j - (a.kc - 1)) * a.conv_dim + ch[c];
-                sv[c][u] = qk_ld(src);
-                wv[c][u] = qk_ld(a.conv_w + (size_t)ch[c] * a.kc + i);
-            }
-#pragma unroll
-        for (int c = 0; c < NC; c++)
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (i0 + u < a.kc) acc[c] = fmaf(sv[c][u], qk_bf16(wv[c][u]), acc[c]);
-    }
-#pragma unroll
-    for (int c = 0; c < NC; c++) out[c] = qk_silu(acc[c]);
-}
-
 template <int EPL>
 __global__ __launch_bounds__(256) void k_dn_rec(DnRecArgs a) {
     constexpr int DK = 16 * EPL;
-    __shared__ float s_ch[2 * DK + DN_RB]; /* q, k, v of the block's rows */
-    __shared__ float s_sc[4];              /* q and k norms, decay, beta */
-    __shared__ float s_o[DN_RB];           /* the block's outputs of this token */
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ DnRecSmem<DK> sh;
+    const int tid = threadIdx.x;
     const int h = blockIdx.y, rb = blockIdx.x * DN_RB;
-    const int kh = h / (a.hv / a.hk);
-    const int key_dim = a.hk * DK, value_dim = a.hv * a.dv;
     const int row = rb + (tid >> 4), i0 = (tid & 15) * EPL;
     float *srow = a.rec_state + ((size_t)h * a.dv + row) * DK + i0;
     float s[EPL];
@@ -215,83 +167,7 @@ __global__ __launch_bounds__(256) void k_dn_rec(DnRecArgs a) {
 #pragma unroll
         for (int e = 0; e < EPL; e++) s[e] = qk_ld(srow + e);
     }
-    const float al = expf(qk_ld(a.a_log + h)), dtb = qk_ld(a.dt_bias + h);
-    const float scale_q = 1.0f / sqrtf((float)DK);
-    for (int t = 0; t < a.n; t++) {
-        /* what the token's later steps read, loaded with the channels' taps
-         * (every thread loads them; the addresses are shared) */
-        const size_t zi = (size_t)t * value_dim + (size_t)h * a.dv + row;
-        const float zv = qk_ld(a.z + zi), nwv = qk_ld(a.norm_w + row);
-        const float av = qk_ld(a.a + (size_t)t * a.hv + h), bv = qk_ld(a.b + (size_t)t * a.hv + h);
-        {
-            /* the block's q, k, v channels, NCC per thread (all their loads
-             * in flight); past the last one a thread repeats it */
-            constexpr int NCC = (2 * DK + DN_RB + 255) / 256;
-            int ch[NCC];
-#pragma unroll
-            for (int u = 0; u < NCC; u++) {
-                const int c = min(tid + 256 * u, 2 * DK + DN_RB - 1);
-                ch[u] = c < DK ? kh * DK + c
-                      : c < 2 * DK ? key_dim + kh * DK + (c - DK)
-                                   : 2 * key_dim + h * a.dv + rb + (c - 2 * DK);
-            }
-            float v[NCC];
-            dn_conv_silu<NCC>(a, t, ch, v);
-#pragma unroll
-            for (int u = 0; u < NCC; u++)
-                if (tid + 256 * u < 2 * DK + DN_RB) s_ch[tid + 256 * u] = v[u];
-        }
-        __syncthreads();
-        if (wave < 2) {
-            /* wave 0: |q|^2, wave 1: |k|^2 */
-            float ss = 0.0f;
-            for (int i = lane; i < DK; i += 64) {
-                const float v = s_ch[wave * DK + i];
-                ss = fmaf(v, v, ss);
-            }
-            ss = qk_group_sum<64>(ss);
-            if (lane == 0) s_sc[wave] = 1.0f / sqrtf(ss + 1e-6f);
-        } else if (tid == 128) {
-            s_sc[2] = expf(-al * log1pf(expf(av + dtb)));
-            s_sc[3] = 1.0f / (1.0f + expf(-bv));
-        }
-        __syncthreads();
-        const float rq = s_sc[0], rk = s_sc[1], g = s_sc[2], beta = s_sc[3];
-        float kk[EPL], qq[EPL];
-#pragma unroll
-        for (int e = 0; e < EPL; e++) {
-            kk[e] = s_ch[DK + i0 + e] * rk;
-            qq[e] = (s_ch[i0 + e] * rq) * scale_q;
-        }
-        float kv = 0.0f;
-#pragma unroll
-        for (int e = 0; e < EPL; e++) {
-            s[e] = s[e] * g;
-            kv = fmaf(s[e], kk[e], kv);
-        }
-        kv = qk_group_sum<16>(kv);
-        const float delta = (s_ch[2 * DK + (tid >> 4)] - kv) * beta;
-        float o = 0.0f;
-#pragma unroll
-        for (int e = 0; e < EPL; e++) {
-            s[e] = fmaf(kk[e], delta, s[e]);
-            o = fmaf(s[e], qq[e], o);
-        }
-        o = qk_group_sum<16>(o);
-        if ((tid & 15) == 0) {
-            /* the gated norm's row factors here, its head factor (from the
-             * sums of squares) in k_dn_out */
-            qk_st(a.core + zi, (o * nwv) * (1.0f / (1.0f + expf(-zv))));
-            s_o[tid >> 4] = o;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            float ss = 0.0f;
-            for (int j = 0; j < DN_RB; j++) ss = fmaf(s_o[j], s_o[j], ss);
-            qk_st(a.ssp + ((size_t)t * a.hv + h) * (a.dv / DN_RB) + blockIdx.x, ss);
-        }
-        __syncthreads(); /* s_ch, s_sc, s_o are rewritten for the next token */
-    }
+    dn_rec_tokens<EPL, false>(a, h, rb, 0, a.n, s, sh);
     if (EPL % 4 == 0) {
 #pragma unroll
         for (int e = 0; e < EPL; e += 4)
@@ -442,6 +318,7 @@ __global__ __launch_bounds__(256) void k_dn_out(DnOutArgs a) {
  */
 struct DnPackArgs {
     const float *core, *ssp, *mixed;
+    const float *z, *norm_w; /* z set: core is o itself (the chunked recurrence), gated here */
     float *conv_state;
     uint16_t *hi, *lo;
     float *pg;
@@ -483,7 +360,18 @@ __global__ __launch_bounds__(256) void k_dn_pack(DnPackArgs a) {
         for (int j = 0; j < 8; j++) ss = ss + (j0 + j < nb ? pv[j] : 0.0f);
     }
     const float r = 1.0f / sqrtf(ss / (float)a.dv + 1e-6f);
-    const float v[8] = {a0.x * r, a0.y * r, a0.z * r, a0.w * r, a1.x * r, a1.y * r, a1.z * r, a1.w * r};
+    float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+    if (a.z) {
+        const float4 z0 = qk_ld((const float4 *)a.z + 2 * i), z1 = qk_ld((const float4 *)a.z + 2 * i + 1);
+        const float4 *np = (const float4 *)(a.norm_w + col % a.dv);
+        const float4 n0 = qk_ld(np), n1 = qk_ld(np + 1);
+        const float zv[8] = {z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
+        const float nv[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = (v[j] * nv[j]) * (1.0f / (1.0f + expf(-zv[j])));
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] *= r;
     uint32_t ph[4], pl[4];
     float s = qk_f32x8_pairs(v, ph, pl);
     ((uint4 *)a.hi)[i] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
@@ -515,8 +403,8 @@ extern "C" int qk_dn_shape_ok(const qk_dn_shape *s) {
 
 extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const float *x, int n, float *out,
                             float *conv_state, float *rec_state, float *mixed, float *z, float *av,
-                            float *bv, float *core, float *ssp, const qk_planes *pl, const qk_inject *inj_in,
-                            void *stream) {
+                            float *bv, float *core, float *ssp, const qk_planes *pl, float *chunk,
+                            const qk_inject *inj_in, void *stream) {
     if (n <= 0) return 0;
     if (!qk_dn_shape_ok(s)) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)stream;
@@ -570,7 +458,12 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     ra.n = n; ra.hk = s->hk; ra.hv = s->hv; ra.dk = s->dk; ra.dv = s->dv; ra.kc = s->kc;
     ra.conv_dim = conv_dim;
     const dim3 rgrid(s->dv / DN_RB, s->hv);
-    switch (s->dk) {
+    const bool chunks = n >= QK_DN_CHUNK_N;
+    if (chunks) {
+        if (!chunk) return (int)hipErrorInvalidValue;
+        rc = qk_launch_dn_chunks(&ra, chunk, stream);
+        if (rc) return rc;
+    } else switch (s->dk) {
     case 32: hipLaunchKernelGGL(k_dn_rec<2>, rgrid, dim3(256), 0, st, ra); break;
     case 64: hipLaunchKernelGGL(k_dn_rec<4>, rgrid, dim3(256), 0, st, ra); break;
     case 128: hipLaunchKernelGGL(k_dn_rec<8>, rgrid, dim3(256), 0, st, ra); break;
@@ -580,7 +473,8 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     if (rc) return rc;
 
     if (mm) {
-        const DnPackArgs ka = {core, ssp, mixed, conv_state, pl->hi, pl->lo, pl->pg, n, value_dim, s->dv, s->kc, conv_dim};
+        const DnPackArgs ka = {core, ssp, mixed, chunks ? z : nullptr, W->norm_w, conv_state, pl->hi, pl->lo,
+                               pl->pg, n, value_dim, s->dv, s->kc, conv_dim};
         hipLaunchKernelGGL(k_dn_pack, dim3((unsigned)((size_t)n * (value_dim / 8) / 256 + 1 + (conv_dim + 255) / 256)),
                            dim3(256), 0, st, ka);
         rc = QK_CHECK_LAUNCH();

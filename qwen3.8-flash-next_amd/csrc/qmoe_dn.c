@@ -32,7 +32,7 @@ struct qmoe_dn_ctx {
     size_t off[DT_COUNT + 1], bytes[DT_COUNT];
     dn_layer *layers;
     void *scratch;
-    float *mixed, *z, *a, *b, *core, *ssp;
+    float *mixed, *z, *a, *b, *core, *ssp, *chunk;
     qk_planes pl; /* NULLs when max_tokens stays below QK_DN_MM_N */
 };
 
@@ -111,10 +111,11 @@ int qmoe_dn_create(qmoe_dn_ctx **out, const qmoe_dn_config *cfg, qmoe_err *err) 
     c->layers = (dn_layer *)calloc((size_t)cfg->n_layers, sizeof(dn_layer));
     const size_t n = (size_t)cfg->max_tokens;
     const size_t wide = n >= QK_DN_MM_N ? n * (d > value_dim ? d : value_dim) : 0;
-    const size_t ssz[9] = {n * conv_dim * 4, n * value_dim * 4, n * hv * 4, n * hv * 4, n * value_dim * 4,
-                           n * (value_dim / 16) * 4, wide * 2, wide * 2, wide / 64 * 4};
-    size_t stot = 0, soff[9];
-    for (int i = 0; i < 9; i++) {
+    const size_t ssz[10] = {n * conv_dim * 4, n * value_dim * 4, n * hv * 4, n * hv * 4, n * value_dim * 4,
+                           n * (value_dim / 16) * 4, wide * 2, wide * 2, wide / 64 * 4,
+                           n >= QK_DN_CHUNK_N ? qk_dn_chunk_bytes(&s, cfg->max_tokens) : 0};
+    size_t stot = 0, soff[10];
+    for (int i = 0; i < 10; i++) {
         soff[i] = stot;
         stot = dn_align(stot + ssz[i]);
     }
@@ -135,6 +136,7 @@ int qmoe_dn_create(qmoe_dn_ctx **out, const qmoe_dn_config *cfg, qmoe_err *err) 
         c->pl.lo = (uint16_t *)(b + soff[7]);
         c->pl.pg = (float *)(b + soff[8]);
     }
+    if (n >= QK_DN_CHUNK_N) c->chunk = (float *)(b + soff[9]);
     for (int l = 0; l < cfg->n_layers; l++) {
         if (dn_hip_fail(err, (int)hipMalloc(&c->layers[l].mem, total), "layer weights")) {
             qmoe_dn_destroy(c);
@@ -256,7 +258,7 @@ static int dn_forward(qmoe_dn_ctx *c, int layer, const float *x, int n, float *o
     W.dt_bias = (const float *)dn_ptr(c, layer, DT_DT_BIAS);
     const int rc = qk_launch_dn(&c->shape, &W, x, n, out, (float *)dn_ptr(c, layer, DT_CONV_STATE),
                                 (float *)dn_ptr(c, layer, DT_REC_STATE), c->mixed, c->z, c->a, c->b,
-                                c->core, c->ssp, &c->pl, inj, stream);
+                                c->core, c->ssp, &c->pl, c->chunk, inj, stream);
     return dn_hip_fail(err, rc, "DeltaNet launch");
 }
 

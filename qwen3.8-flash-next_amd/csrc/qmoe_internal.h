@@ -267,10 +267,18 @@ int qk_dn_shape_ok(const qk_dn_shape *s);
 /* x [n, d] f32 -> out [n, d]; conv_state and rec_state are updated;
  * mixed [n, conv_dim], z [n, value_dim], a, b [n, hv], core [n, value_dim]
  * and ssp [n, hv, dv/16] are scratch; pl, planes of max(d, value_dim)
- * columns, is used from QK_DN_MM_N tokens on (and may be all NULL below) */
+ * columns, is used from QK_DN_MM_N tokens on and chunk, of
+ * qk_dn_chunk_bytes, from QK_DN_CHUNK_N on (they may be NULL below) */
 int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const float *x, int n, float *out,
                  float *conv_state, float *rec_state, float *mixed, float *z, float *a, float *b,
-                 float *core, float *ssp, const qk_planes *pl, const qk_inject *inj, void *stream);
+                 float *core, float *ssp, const qk_planes *pl, float *chunk, const qk_inject *inj,
+                 void *stream);
+/* the recurrence in chunks (dn_chunk.hip) from QK_DN_CHUNK_N tokens on (up to
+ * 32 tokens it takes 28 us at 32 heads of 128, token by token 1.6 each);
+ * rec_args is deltanet.hip's DnRecArgs, scratch of qk_dn_chunk_bytes */
+#define QK_DN_CHUNK_N 20
+size_t qk_dn_chunk_bytes(const qk_dn_shape *s, int max_n);
+int qk_launch_dn_chunks(const void *rec_args, float *scratch, void *stream);
 int qk_launch_dn_zero(float *p, size_t count, void *stream);
 
 /* the full-attention mixer with the QSA indexer (attention.hip) */

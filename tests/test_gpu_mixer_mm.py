@@ -72,3 +72,47 @@ def test_attention_values_past_the_parts(torch_dev, bad):
             assert ta.rel(got[t], ref[t]) < ta.REL_L2, t
     else:
         assert np.isnan(got[j:]).all()
+
+
+# the chunked recurrence: its first count, one token past a chunk, every key
+# dim, value dims above its column round, 1 to 16 taps, a call past one
+# segment of 2048 tokens
+@pytest.mark.parametrize("shape", [(64, 1, 2, 32, 32, 1), (128, 1, 2, 64, 512, 3), (64, 2, 2, 256, 64, 4), (64, 3, 9, 128, 64, 4)])
+def test_deltanet_chunks(torch_dev, shape):
+    torch, dev = torch_dev
+    td.run_steps(torch, dev, shape, [19, 20, 33, 1, 64, 95], seed=14, seed_state=True)
+
+
+def test_deltanet_segments(torch_dev):
+    torch, dev = torch_dev
+    td.run_steps(torch, dev, (64, 1, 2, 64, 64, 4), [2048, 2049, 2100], seed=15)
+
+
+@pytest.mark.parametrize("bad", ["nan", "inf", "1e30"])
+def test_deltanet_values_past_the_products(torch_dev, bad):
+    """a token whose values a chunk's products would spread: the tokens before
+    it are those of the call without it, and from it on the outputs are NaN
+    (nan, inf) or the oracle's (1e30)"""
+    import numpy as np
+    torch, dev = torch_dev
+    shape, n, j = (128, 1, 2, 64, 64, 4), 80, 45
+    D = td.orc.DeltaNet(*shape, seed=16)
+    x = td.orc.gen_dn_x(n, shape[0], 17)
+    outs = []
+    for v in (None, float(bad)):
+        xi = x.copy()
+        if v is not None:
+            xi[j, 5] = v
+        with td.load_pkg().DeltaNetContext(*shape, max_tokens=n) as ctx:
+            ctx.upload_layer(0, D.arrays())
+            outs.append(ctx.forward(0, torch.from_numpy(xi).to(dev)).cpu().numpy())
+    clean, got = outs
+    assert np.isfinite(clean).all()
+    # the tokens of j's chunk are stepped one by one: fp32 sums in another order
+    assert td.rel(got[:j], clean[:j]) < 1e-5
+    if bad == "1e30":
+        ref = D.forward(xi, *D.new_state())
+        for t in range(j, n):
+            assert td.rel(got[t], ref[t]) < td.REL_L2, t
+    else:
+        assert np.isnan(got[j:]).all()
