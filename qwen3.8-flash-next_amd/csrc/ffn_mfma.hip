@@ -687,9 +687,16 @@ static int mm_max_tasks16(qk_shape s, int n) {
     return (int)((nk < s.E ? nk : s.E) + nk / MM_BM16 + (n + MM_BM16 - 1) / MM_BM16 + 1);
 }
 
+/* the lists of any call of up to n tokens: a call of at most MM_NARROW_N
+ * tokens has a second list, so the largest call is not always the largest */
 extern "C" size_t qk_mfma_task_bytes(qk_shape s, int n) {
-    const size_t t16 = n <= MM_NARROW_N ? (size_t)MM_TASK_HDR + 4 * (size_t)mm_max_tasks16(s, n) : 0;
-    return ((size_t)MM_TASK_HDR + 4 * (size_t)qk_mfma_max_tasks(s, n) + (size_t)MM_SMALL16(s.E) + t16) * 4;
+    size_t most = 0;
+    for (int m = n;; m = MM_NARROW_N) {
+        const size_t t16 = m <= MM_NARROW_N ? (size_t)MM_TASK_HDR + 4 * (size_t)mm_max_tasks16(s, m) : 0;
+        const size_t b = ((size_t)MM_TASK_HDR + 4 * (size_t)qk_mfma_max_tasks(s, m) + (size_t)MM_SMALL16(s.E) + t16) * 4;
+        most = b > most ? b : most;
+        if (m <= MM_NARROW_N) return most;
+    }
 }
 
 extern "C" int32_t *qk_mfma_small_list(qk_shape s, int n, int32_t *tasks) {
