@@ -21,8 +21,8 @@
  * x column tiles.  The workgroup's 4 waves each own CT = 4 column tiles of
  * 16 (gate/up: 32 columns of Wg and the same 32 of Wu, so h = silu(g)*u is
  * formed in registers; down: 64 columns of Wd) and every 16-row tile of
- * the chunk.  Batches of at most 64 tokens use CT = 2 and 64-row chunks:
- * twice the workgroups, each with less LDS and fewer registers.  Per group the chunk's activation rows are staged in LDS
+ * the chunk.  Batches of at most MM_NARROW_N tokens use CT = 2 and 64-row
+ * chunks: twice the workgroups, each with less LDS and fewer registers.  Per group the chunk's activation rows are staged in LDS
  * (double buffered, XOR-swizzled 16-byte chunks), the code words come from
  * a register ring MM_WD groups ahead, and the scales of the whole tile sit
  * in LDS.  The kernel body is specialised on the number of 16-row tiles.
@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256, 2) void k_mm(MmArgs a) {
     const int mt = (i8 / a.ntile) * 8 + (L & 7), nt = i8 - (i8 / a.ntile) * a.ntile;
     if (mt >= qk_ld(a.tasks)) return;
     const int4 tk = qk_ld((const int4 *)(a.tasks + MM_TASK_HDR) + mt);
-    const int e = tk.x, p0 = tk.y, m = tk.z, mstart = tk.w * MM_BM;
+    const int e = tk.x, p0 = tk.y, m = tk.z, mstart = tk.w * (BMT * 16);
     const int mrows = min(BMT * 16, m - mstart);
     if (mrows <= 0) return;
     const int tid = threadIdx.x;
@@ -637,12 +637,16 @@ __global__ __launch_bounds__(1024) void k_mm_tasks(const int32_t *segtab, int n,
     mm_tasks_block(segtab, n, k, E, min_m, tasks, small);
 }
 
-/* Up to MM_NARROW_N tokens no segment exceeds 64 rows: the kernels then
- * hold 64-row chunks and give each wave 2 column tiles instead of 4, so a
- * batch of mostly small segments spreads over twice the workgroups (with
- * few rows per task the per-group latency, not the MFMA rate, bounds a
- * workgroup); the down projection at K = 512 runs on k_mm_down16 over the
- * 16-row list. */
+/* Up to MM_NARROW_N tokens the kernels hold 64-row chunks and give each wave
+ * 2 column tiles instead of 4, so a batch of mostly small segments spreads
+ * over twice the workgroups (with few rows per task the per-group latency,
+ * not the MFMA rate, bounds a workgroup); the down projection at K = 512 runs
+ * on k_mm_down16 over the 16-row list.  The line lies where the two meet
+ * (hidden 2048, 512 experts top-10, the layer in us, wide against narrow):
+ * f32 333 tokens 437 / 388, 512 tokens 452 / 407, 768 tokens 475 / 453;
+ * bf16 96 tokens 292 / 279, 333 tokens 389 / 356, 768 tokens 414 / 410,
+ * 1024 tokens 438 / 471; with Zipf-skewed routing 128 tokens 138 / 108, 333
+ * tokens 181 / 185, 512 tokens 222 / 223, 768 tokens 254 / 286. */
 
 static int mm_launch(MmArgs &a, bool down, int terms, int max_tasks, hipStream_t st,
                      const int32_t *list16 = nullptr, int max16 = 0) {
@@ -676,7 +680,8 @@ static int mm_launch(MmArgs &a, bool down, int terms, int max_tasks, hipStream_t
 extern "C" int qk_mfma_max_tasks(qk_shape s, int n) {
     /* routed segments: at most min(E, n*k), plus their extra chunks; shared: ceil(n/BM) */
     const long long nk = (long long)n * s.k;
-    const long long t = (nk < s.E ? nk : s.E) + nk / MM_BM + (n + MM_BM - 1) / MM_BM + 1;
+    const int bm = mm_chunk_rows(n);
+    const long long t = (nk < s.E ? nk : s.E) + nk / bm + (n + bm - 1) / bm + 1;
     return (int)t;
 }
 

@@ -13,8 +13,10 @@
 #define MM_BM (16 * MM_MT)   /* rows per chunk */
 #define MM_TASK_HDR 4        /* int32 header before the int4 task entries */
 
-#define MM_NARROW_N 64       /* batches up to this many tokens also get a 16-row list */
+#define MM_NARROW_N 512      /* batches up to this many tokens: 64-row chunks, and a 16-row list too */
 #define MM_BM16 16
+#define MM_NBM 64            /* rows per chunk up to MM_NARROW_N tokens */
+static __host__ __device__ inline int mm_chunk_rows(int n) { return n <= MM_NARROW_N ? MM_NBM : MM_BM; }
 
 /* a segment-table word: from LDS (the table this workgroup just built,
  * mirrored there) or from global memory */
@@ -120,7 +122,7 @@ static __device__ void mm_tasks_list(const int32_t *segtab, int n, int k, int E,
 template <bool LDS = false>
 static __device__ void mm_tasks_block(const int32_t *segtab, int n, int k, int E, int min_m, int32_t *tasks,
                                int32_t *small) {
-    mm_tasks_list<LDS>(segtab, n, k, E, min_m, MM_BM, tasks, small);
+    mm_tasks_list<LDS>(segtab, n, k, E, min_m, mm_chunk_rows(n), tasks, small);
     if (n <= MM_NARROW_N) mm_tasks_list<LDS>(segtab, n, k, E, min_m, MM_BM16, small + MM_SMALL16(E), nullptr);
 }
 
