@@ -1082,7 +1082,7 @@ extern "C" int qk_launch_at(const qk_at_shape *s, const qk_at_dev *W, const floa
     const bool mm = n >= QK_AT_MM_N;
     if (mm) {
         if (!sc->pl.hi || !sc->pl.lo || !sc->pl.pg) return (int)hipErrorInvalidValue;
-        rc = qk_launch_pack_rows(x, 0, (size_t)n, s->d, sc->pl.hi, sc->pl.lo, sc->pl.pg, stream);
+        rc = qk_launch_proj_pack(x, n, s->d, &sc->pl, stream);
         if (rc) return rc;
         qk_proj p = {};
         p.seg[0] = {W->q_q, W->q_s, W->q_b, sc->qg, 2 * h * hd, 2 * h * hd};

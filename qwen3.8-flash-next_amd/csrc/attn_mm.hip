@@ -41,7 +41,7 @@ struct AmArgs {
     float2 *pml;           /* [n, h, nch]: maximum (log2 units), sum */
     const float *qg;       /* [n, h, 2, hd] */
     uint16_t *hi, *lo;     /* [n, h * hd] planes */
-    float *pg;             /* [n, h * hd / 64] */
+    float *pg;             /* [h * hd / 64, qk_planes_ld(n)] */
     int n, h, kvh, hd, T, tiles, offset, comp, nb, kw, nch, ctiles, nqb;
 };
 
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void k_am_attn(AmArgs a) {
 }
 
 /* one thread per 8 columns of a token's attention output: the key ranges up
- * to the token's own merged, the gate, and the planes (k_pack_rows'
+ * to the token's own merged, the gate, and the planes (k_proj_pack's
  * arithmetic).  Bound: HBM / L2, the partial outputs read once. */
 __global__ __launch_bounds__(256) void k_am_comb(AmArgs a) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(256) void k_am_comb(AmArgs a) {
     s += qk_dpp<QK_DPP_XOR1>(s);
     s += qk_dpp<QK_DPP_XOR2>(s);
     s += __shfl_xor(s, 4, QK_WAVE);
-    if ((i & 7) == 0) a.pg[i >> 3] = -128.0f * s;
+    if ((i & 7) == 0) a.pg[(size_t)(col >> 6) * qk_planes_ld(a.n) + t] = -128.0f * s;
 }
 
 /* ------------------------------------------------------------ host side */

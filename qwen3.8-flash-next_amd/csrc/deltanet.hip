@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) void k_dn_out(DnOutArgs a) {
 
 /*
  * Many tokens: core scaled by its head's 1/sqrt(sum(o^2)/dv + eps) as
- * operand planes of out_proj (k_pack_rows' arithmetic and order), one
+ * operand planes of out_proj (k_proj_pack's arithmetic and order), one
  * thread per 8 columns; the workgroups past the planes move the conv state
  * on by n tokens.
  */
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256) void k_dn_pack(DnPackArgs a) {
     s += qk_dpp<QK_DPP_XOR1>(s);
     s += qk_dpp<QK_DPP_XOR2>(s);
     s += __shfl_xor(s, 4, QK_WAVE);
-    if ((i & 7) == 0) a.pg[i >> 3] = -128.0f * s;
+    if ((i & 7) == 0) a.pg[(size_t)(col >> 6) * qk_planes_ld(a.n) + t] = -128.0f * s;
 }
 
 /* ------------------------------------------------------------ host side */
@@ -416,7 +416,7 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     const bool mm = n >= QK_DN_MM_N;
     if (mm) {
         if (!pl || !pl->hi || !pl->lo || !pl->pg) return (int)hipErrorInvalidValue;
-        rc = qk_launch_pack_rows(x, 0, (size_t)n, s->d, pl->hi, pl->lo, pl->pg, stream);
+        rc = qk_launch_proj_pack(x, n, s->d, pl, stream);
         if (rc) return rc;
         qk_proj p = {};
         p.seg[0] = {W->qkv_q, W->qkv_s, W->qkv_b, mixed, conv_dim, conv_dim};

@@ -22,4 +22,18 @@ __device__ __forceinline__ qm_bf16x8 qm_codes(uint32_t w) {
                                          __builtin_amdgcn_perm(k, lo, 0x04030401u), __builtin_amdgcn_perm(k, hi, 0x04030401u)));
 }
 
+/* the same as 16 + q (0x4180 | q << 3, exact: the ulp in [16, 32) is 1/8).
+ * The offset is what the running sums carry until the group ends, so its size
+ * sets their rounding: with 128 + q (one instruction fewer) the DeltaNet
+ * out_proj's error against 64 bits at 4096 columns was 9.6e-6, more than the
+ * per-token GEMV's 9.3e-6; with 16 + q 7.5e-6. */
+__device__ __forceinline__ qm_bf16x8 qm_codes16(uint32_t w) {
+    const uint32_t lo = ((w << 3) & 0x78787878u) | 0x80808080u, hi = ((w >> 1) & 0x78787878u) | 0x80808080u;
+    const uint32_t k = 0x41414141u;
+    return __builtin_bit_cast(qm_bf16x8,
+                              make_uint4(__builtin_amdgcn_perm(k, lo, 0x04020400u), __builtin_amdgcn_perm(k, hi, 0x04020400u),
+                                         __builtin_amdgcn_perm(k, lo, 0x04030401u), __builtin_amdgcn_perm(k, hi, 0x04030401u)));
+}
+#define QM_P16 0.125f /* a group's start -16 X from the planes' P = -128 X */
+
 #endif

@@ -28,20 +28,6 @@
 
 typedef float qm_f32x16 __attribute__((ext_vector_type(16)));
 
-/* one code word -> the B operand: bf16 16 + q (0x4180 | q << 3, exact: the
- * ulp in [16, 32) is 1/8) in (q_i, q_{i+4}) pair order.  The offset is what
- * the running sums carry until the group ends, so its size sets their
- * rounding: with 128 + q (one instruction fewer) out_proj's error against
- * 64 bits at 4096 columns was 9.6e-6, more than the per-token GEMV's 9.3e-6 */
-__device__ __forceinline__ qm_bf16x8 pj_codes(uint32_t w) {
-    const uint32_t lo = ((w << 3) & 0x78787878u) | 0x80808080u, hi = ((w >> 1) & 0x78787878u) | 0x80808080u;
-    const uint32_t k = 0x41414141u;
-    return __builtin_bit_cast(qm_bf16x8,
-                              make_uint4(__builtin_amdgcn_perm(k, lo, 0x04020400u), __builtin_amdgcn_perm(k, hi, 0x04020400u),
-                                         __builtin_amdgcn_perm(k, lo, 0x04030401u), __builtin_amdgcn_perm(k, hi, 0x04030401u)));
-}
-#define PJ_P 0.125f /* -16 X from the planes' P = -128 X */
-
 #define PJ_THREADS 256
 #define QK_PROJ_FEW_N 320
 
@@ -59,15 +45,15 @@ __device__ __forceinline__ bool pj_segment(const qk_proj &a, int cb, const uint3
     return cb < a.end64[a.nseg - 1];
 }
 
-/* eight group sums P of a row from group k0 on (0 past G) as X = P / -128 in
- * three bf16 parts, 24 bits: with a zero point inside the code range the
+/* eight group sums P of a row (pg: of group 0, the next group ld on) from
+ * group k0 on (0 past G) as X = P / -128 in three bf16 parts, 24 bits: with a zero point inside the code range the
  * bias term is as large as the code term and cancels most of it, so two
  * parts (2^-17 of it) would show in the result */
-__device__ __forceinline__ void pj_bias_x(const float *pg, int k0, int G, qm_bf16x8 (&X)[3]) {
+__device__ __forceinline__ void pj_bias_x(const float *pg, size_t ld, int k0, int G, qm_bf16x8 (&X)[3]) {
     uint32_t w[3][4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const float p0 = qk_ld(pg + min(k0 + 2 * j, G - 1)), p1 = qk_ld(pg + min(k0 + 2 * j + 1, G - 1));
+        const float p0 = qk_ld(pg + ld * min(k0 + 2 * j, G - 1)), p1 = qk_ld(pg + ld * min(k0 + 2 * j + 1, G - 1));
         float x0 = k0 + 2 * j < G ? p0 * (-1.0f / 128.0f) : 0.0f;
         float x1 = k0 + 2 * j + 1 < G ? p1 * (-1.0f / 128.0f) : 0.0f;
 #pragma unroll
@@ -113,7 +99,7 @@ __device__ __forceinline__ void pj_store(const qk_proj &a, float *out, int ostri
  * wave's reads touch every bank), loaded into registers one group ahead;
  * code words and scales come straight into registers one group ahead.
  */
-template <int RT, int WR, bool INJ>
+template <int RT, int WR, bool INJ, bool S8>
 __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
     constexpr int BM = 32 * RT * WR, WC = 4 / WR;
     constexpr int ACH = BM * 8 / PJ_THREADS; /* chunks per thread and plane */
@@ -154,7 +140,7 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
         const int ci = tid + PJ_THREADS * i;
         ap[i] = a.hi + (size_t)min(m0 + (ci >> 3), a.n - 1) * a.K + (ci & 7) * 8;
     }
-    const size_t lo_off = a.lo - a.hi;
+    const size_t lo_off = a.lo - a.hi, ldp = qk_planes_ld(a.n);
     uint4 ar[2][ACH];
     float pr = 0.0f;
     auto load_a = [&](int g) {
@@ -163,7 +149,7 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
             ar[0][i] = qk_ld((const uint4 *)(ap[i] + 64 * g));
             ar[1][i] = qk_ld((const uint4 *)(ap[i] + lo_off + 64 * g));
         }
-        pr = qk_ld(a.pg + (size_t)min(m0 + min(tid, BM - 1), a.n - 1) * G + g);
+        pr = qk_ld(a.pg + ldp * g + min(m0 + min(tid, BM - 1), a.n - 1));
     };
     auto store_a = [&](int buf) {
 #pragma unroll
@@ -172,16 +158,23 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
             s_a[buf][0][row * 8 + (kc ^ (row & 7))] = ar[0][i];
             s_a[buf][1][row * 8 + (kc ^ (row & 7))] = ar[1][i];
         }
-        if (tid < BM) s_p[buf][tid] = pr * PJ_P;
+        if (tid < BM) s_p[buf][tid] = pr * QM_P16;
     };
     uint4 wv[2];
-    uint16_t sv[2];
-    auto load_w = [&](int g) {
+    /* scales: eight groups of a column per load where its row of scales is
+     * 16-byte aligned (a load of one touches a line per column all the same),
+     * shifted down a group at a time */
+    uint4 s8[2], s8n[2];
+    auto load_s = [&](uint4 (&d)[2], int g) {
 #pragma unroll
         for (int ct = 0; ct < 2; ct++) {
-            wv[ct] = qk_ld((const uint4 *)(wq[ct] + 8 * g));
-            sv[ct] = qk_ld(sp[ct] + g);
+            if (S8) d[ct] = qk_ld((const uint4 *)(sp[ct] + min(g, G - 8)));
+            else d[ct].x = qk_ld(sp[ct] + min(g, G - 1));
         }
+    };
+    auto load_w = [&](int g) {
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) wv[ct] = qk_ld((const uint4 *)(wq[ct] + 8 * g));
     };
     qm_f32x16 acc[RT][2];
 #pragma unroll
@@ -193,6 +186,7 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
 
     load_a(0);
     load_w(0);
+    load_s(s8, 0);
     for (int g = 0; g < G; g++) {
         const int buf = g & 1;
         store_a(buf);
@@ -200,15 +194,30 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
         float sc[2];
 #pragma unroll
         for (int ct = 0; ct < 2; ct++) {
-            bop[ct][0] = pj_codes(wv[ct].x);
-            bop[ct][1] = pj_codes(wv[ct].y);
-            bop[ct][2] = pj_codes(wv[ct].z);
-            bop[ct][3] = pj_codes(wv[ct].w);
-            sc[ct] = qk_bf16(sv[ct]);
+            bop[ct][0] = qm_codes16(wv[ct].x);
+            bop[ct][1] = qm_codes16(wv[ct].y);
+            bop[ct][2] = qm_codes16(wv[ct].z);
+            bop[ct][3] = qm_codes16(wv[ct].w);
+            sc[ct] = qk_bf16_lo(s8[ct].x);
+            if (S8) {
+                s8[ct].x = (s8[ct].x >> 16) | (s8[ct].y << 16);
+                s8[ct].y = (s8[ct].y >> 16) | (s8[ct].z << 16);
+                s8[ct].z = (s8[ct].z >> 16) | (s8[ct].w << 16);
+                s8[ct].w >>= 16;
+            }
         }
         const int gn = min(g + 1, G - 1); /* past the end: loaded, not used */
         load_a(gn);
         load_w(gn);
+        if (!S8) {
+            load_s(s8, gn);
+        } else {
+            if ((g & 7) == 0) load_s(s8n, g + 8);
+            if ((g & 7) == 7) {
+                s8[0] = s8n[0];
+                s8[1] = s8n[1];
+            }
+        }
         /* buffer buf was last read in group g-2, before the barrier of g-1 */
         qk_lds_barrier();
 #pragma unroll
@@ -245,7 +254,7 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             qm_bf16x8 X[3];
-            pj_bias_x(a.pg + (size_t)min(m0 + 32 * (RT * wr + rt) + c, a.n - 1) * G, k0 + 8 * h, G, X);
+            pj_bias_x(a.pg + min(m0 + 32 * (RT * wr + rt) + c, a.n - 1), ldp, k0 + 8 * h, G, X);
 #pragma unroll
             for (int ct = 0; ct < 2; ct++)
 #pragma unroll
@@ -293,7 +302,7 @@ __global__ __launch_bounds__(64 * WK) void k_proj_few(qk_proj a) {
         wq[ct] = q + (size_t)(r0 + 32 * ct + c) * wrow + 4 * h;
         sp[ct] = s + (size_t)(r0 + 32 * ct + c) * G;
     }
-    const size_t lo_off = a.lo - a.hi;
+    const size_t lo_off = a.lo - a.hi, ldp = qk_planes_ld(a.n);
     const uint16_t *ap = a.hi + (size_t)min(m0 + c, a.n - 1) * a.K + 32 * h;
     uint4 wv[CT], av[2][4];
     uint16_t sv[CT];
@@ -310,8 +319,10 @@ __global__ __launch_bounds__(64 * WK) void k_proj_few(qk_proj a) {
             av[1][j] = qk_ld((const uint4 *)(ap + lo_off + 64 * g) + j);
         }
 #pragma unroll
-        for (int i = 0; i < 16; i++)
-            pv[i] = qk_ld(a.pg + (size_t)min(m0 + 8 * (i >> 2) + 4 * h + (i & 3), a.n - 1) * G + g);
+        for (int i = 0; i < 4; i++) { /* rows past n: within the leading dimension, not used */
+            const float4 v = qk_ld((const float4 *)(a.pg + ldp * g + m0 + 8 * i + 4 * h));
+            pv[4 * i] = v.x; pv[4 * i + 1] = v.y; pv[4 * i + 2] = v.z; pv[4 * i + 3] = v.w;
+        }
     };
     qm_f32x16 acc[CT];
 #pragma unroll
@@ -330,13 +341,13 @@ __global__ __launch_bounds__(64 * WK) void k_proj_few(qk_proj a) {
         }
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) {
-            bop[ct][0] = pj_codes(wv[ct].x);
-            bop[ct][1] = pj_codes(wv[ct].y);
-            bop[ct][2] = pj_codes(wv[ct].z);
-            bop[ct][3] = pj_codes(wv[ct].w);
+            bop[ct][0] = qm_codes16(wv[ct].x);
+            bop[ct][1] = qm_codes16(wv[ct].y);
+            bop[ct][2] = qm_codes16(wv[ct].z);
+            bop[ct][3] = qm_codes16(wv[ct].w);
             sc[ct] = qk_bf16(sv[ct]);
 #pragma unroll
-            for (int i = 0; i < 16; i++) t[ct][i] = pv[i] * PJ_P;
+            for (int i = 0; i < 16; i++) t[ct][i] = pv[i] * QM_P16;
         }
         load(min(g + WK, G - 1));
 #pragma unroll
@@ -353,7 +364,7 @@ __global__ __launch_bounds__(64 * WK) void k_proj_few(qk_proj a) {
     /* bias term, 16 groups per step, the steps dealt to the waves */
     for (int k0 = 16 * wave; k0 < G; k0 += 16 * WK) {
         qm_bf16x8 X[3];
-        pj_bias_x(a.pg + (size_t)min(m0 + c, a.n - 1) * G, k0 + 8 * h, G, X);
+        pj_bias_x(a.pg + min(m0 + c, a.n - 1), ldp, k0 + 8 * h, G, X);
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) {
             const qm_bf16x8 bb = pj_bias_w(b + (size_t)(r0 + 32 * ct + c) * G, k0 + 8 * h, G);
@@ -439,7 +450,37 @@ __global__ __launch_bounds__(256) void k_proj_bf16(PjBf16Args a) {
     }
 }
 
+/* k_pack_rows (ffn_mfma.hip) with the group sums transposed: a tile's rows
+ * then read them as runs, where a row-major sum is a line per row */
+__global__ __launch_bounds__(256) void k_proj_pack(const float *x, size_t nchunks, int G, size_t ldp, uint16_t *hi,
+                                                   uint16_t *lo, float *pg) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nchunks) return; /* nchunks is a multiple of 8: whole groups leave together */
+    const float4 a0 = qk_ld((const float4 *)x + 2 * i), a1 = qk_ld((const float4 *)x + 2 * i + 1);
+    const float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+    uint32_t ph[4], pl[4];
+    float s = qk_f32x8_pairs(v, ph, pl);
+    ((uint4 *)lo)[i] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
+    ((uint4 *)hi)[i] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
+    s += qk_dpp<QK_DPP_XOR1>(s);
+    s += qk_dpp<QK_DPP_XOR2>(s);
+    s += __shfl_xor(s, 4, QK_WAVE);
+    if ((i & 7) == 0) {
+        const size_t row = (i >> 3) / G;
+        pg[((i >> 3) - row * G) * ldp + row] = -128.0f * s;
+    }
+}
+
 /* ------------------------------------------------------------ host side */
+
+extern "C" int qk_launch_proj_pack(const float *x, int n, int K, const qk_planes *pl, void *stream) {
+    if (n <= 0) return 0;
+    if (K <= 0 || K % 64) return (int)hipErrorInvalidValue;
+    const size_t nch = (size_t)n * (K / 8);
+    hipLaunchKernelGGL(k_proj_pack, dim3((unsigned)((nch + 255) / 256)), dim3(256), 0, (hipStream_t)stream, x, nch, K / 64,
+                       qk_planes_ld(n), pl->hi, pl->lo, pl->pg);
+    return QK_CHECK_LAUNCH();
+}
 
 extern "C" int qk_launch_proj(const qk_proj *in, void *stream) {
     qk_proj a = *in;
@@ -454,13 +495,20 @@ extern "C" int qk_launch_proj(const qk_proj *in, void *stream) {
     }
     hipStream_t st = (hipStream_t)stream;
     const bool inj = a.hyper != nullptr;
+    bool s8 = a.K % 512 == 0; /* G a multiple of 8, and the scales' bases aligned */
+    for (int i = 0; i < a.nseg; i++) s8 = s8 && ((uintptr_t)a.seg[i].s & 15) == 0;
 #define PJ_MM(RT, WR)                                                                                        \
     do {                                                                                                     \
         a.mtiles = (a.n + 32 * RT * WR - 1) / (32 * RT * WR);                                                \
         a.ntiles = (end + 4 / WR - 1) / (4 / WR);                                                            \
         const dim3 grid(((unsigned)(a.mtiles * a.ntiles) + 7) / 8 * 8);                                      \
-        if (inj) hipLaunchKernelGGL((k_proj_mm<RT, WR, true>), grid, dim3(PJ_THREADS), 0, st, a);            \
-        else hipLaunchKernelGGL((k_proj_mm<RT, WR, false>), grid, dim3(PJ_THREADS), 0, st, a);               \
+        if (s8) {                                                                                            \
+            if (inj) hipLaunchKernelGGL((k_proj_mm<RT, WR, true, true>), grid, dim3(PJ_THREADS), 0, st, a);  \
+            else hipLaunchKernelGGL((k_proj_mm<RT, WR, false, true>), grid, dim3(PJ_THREADS), 0, st, a);     \
+        } else {                                                                                             \
+            if (inj) hipLaunchKernelGGL((k_proj_mm<RT, WR, true, false>), grid, dim3(PJ_THREADS), 0, st, a); \
+            else hipLaunchKernelGGL((k_proj_mm<RT, WR, false, false>), grid, dim3(PJ_THREADS), 0, st, a);    \
+        }                                                                                                    \
     } while (0)
 #define PJ_FEW(CT, WK)                                                                                       \
     do {                                                                                                     \

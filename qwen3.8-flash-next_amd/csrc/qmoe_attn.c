@@ -159,7 +159,7 @@ int qmoe_attn_create(qmoe_attn_ctx **out, const qmoe_attn_config *cfg, qmoe_err 
     const size_t wide = n >= QK_AT_MM_N ? n * (d > ok ? d : ok) : 0;
     const size_t ssz[15] = {n * qr * 4, n * kr * 4, n * kr * 4, n * (ih + 1) * ihd * 4, n * h * hd * 4,
                             n * ih * ihd * 4, n * kw * 4, units * h * (hd + 2) * 4, n * h * hd * 4,
-                            n * (cap / (size_t)s.comp) * 4, wide * 2, wide * 2, wide / 64 * 4,
+                            n * (cap / (size_t)s.comp) * 4, wide * 2, wide * 2, wide ? qk_planes_ld((int)n) * (wide / n / 64) * 4 : 0,
                             wide ? qk_am_img_bytes(&s) : 0, wide ? qk_am_mask_bytes(&s, cfg->max_tokens) : 0};
     size_t stot = 0, soff[15];
     for (int i = 0; i < 15; i++) {

@@ -112,7 +112,7 @@ int qmoe_dn_create(qmoe_dn_ctx **out, const qmoe_dn_config *cfg, qmoe_err *err) 
     const size_t n = (size_t)cfg->max_tokens;
     const size_t wide = n >= QK_DN_MM_N ? n * (d > value_dim ? d : value_dim) : 0;
     const size_t ssz[10] = {n * conv_dim * 4, n * value_dim * 4, n * hv * 4, n * hv * 4, n * value_dim * 4,
-                           n * (value_dim / 16) * 4, wide * 2, wide * 2, wide / 64 * 4,
+                           n * (value_dim / 16) * 4, wide * 2, wide * 2, wide ? qk_planes_ld((int)n) * (wide / n / 64) * 4 : 0,
                            n >= QK_DN_CHUNK_N ? qk_dn_chunk_bytes(&s, cfg->max_tokens) : 0};
     size_t stot = 0, soff[10];
     for (int i = 0; i < 10; i++) {

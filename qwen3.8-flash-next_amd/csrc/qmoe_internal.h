@@ -212,9 +212,21 @@ typedef struct {
     int hc;
 } qk_inject;
 
+/* operand planes of a mixer call, in its scratch: hi, lo [n, K] as
+ * qk_launch_pack_rows writes them, pg [K/64, qk_planes_ld(n)] */
+typedef struct {
+    uint16_t *hi, *lo;
+    float *pg;
+} qk_planes;
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+static inline size_t qk_planes_ld(int n) { return ((size_t)n + 31) / 32 * 32; }
+int qk_launch_proj_pack(const float *x, int n, int K, const qk_planes *pl, void *stream);
+
 /* the mixers' q4 projections of many tokens on MFMA (proj_mm.hip): every
  * segment's out[t * ostride + r] = x[t] . W[r] over operand planes hi, lo
- * [n, K] and pg [n, K/64] of qk_launch_pack_rows (f32 rows).  rows and K
+ * [n, K] and pg of qk_launch_proj_pack.  rows and K
  * are multiples of 64.  With hyper set (one segment): also the inject
  * update of its output, [n, hc, ostride]; out may then be NULL. */
 #define QK_PROJ_SEGS 3
@@ -247,12 +259,6 @@ int qk_launch_proj_bf16(const uint16_t *w0, const uint16_t *w1, int rows, const 
  * against 37..97. */
 #define QK_DN_MM_N 6
 #define QK_AT_MM_N 16
-/* operand planes of a mixer call, in its scratch: hi, lo [n, K], pg [n, K/64] */
-typedef struct {
-    uint16_t *hi, *lo;
-    float *pg;
-} qk_planes;
-
 /* the gated DeltaNet mixer (deltanet.hip) */
 typedef struct {
     int d, hk, hv, dk, dv, kc; /* hidden, key/value heads, head dims, conv taps */
