@@ -1081,7 +1081,7 @@ extern "C" int qk_launch_at(const qk_at_shape *s, const qk_at_dev *W, const floa
     int rc;
     const bool mm = n >= QK_AT_MM_N;
     if (mm) {
-        if (!sc->pl.hi || !sc->pl.lo || !sc->pl.pg) return (int)hipErrorInvalidValue;
+        if (!sc->pl.a || !sc->pl.pg) return (int)hipErrorInvalidValue;
         rc = qk_launch_proj_pack(x, n, s->d, &sc->pl, stream);
         if (rc) return rc;
         qk_proj p = {};
@@ -1089,7 +1089,7 @@ extern "C" int qk_launch_at(const qk_at_shape *s, const qk_at_dev *W, const floa
         p.seg[1] = {W->k_q, W->k_s, W->k_b, sc->kraw, kvh * hd, kvh * hd};
         p.seg[2] = {W->v_q, W->v_s, W->v_b, sc->vraw, kvh * hd, kvh * hd};
         p.nseg = 3;
-        p.hi = sc->pl.hi; p.lo = sc->pl.lo; p.pg = sc->pl.pg;
+        p.pl = sc->pl;
         p.K = s->d; p.n = n;
         rc = qk_launch_proj(&p, stream);
         if (rc) return rc;
@@ -1157,7 +1157,7 @@ extern "C" int qk_launch_at(const qk_at_shape *s, const qk_at_dev *W, const floa
         qk_proj p = {};
         p.seg[0] = {W->o_q, W->o_s, W->o_b, out, s->d, s->d};
         p.nseg = 1;
-        p.hi = sc->pl.hi; p.lo = sc->pl.lo; p.pg = sc->pl.pg;
+        p.pl = sc->pl;
         p.K = h * hd; p.n = n;
         if (inj && inj->hyper) { p.hyper = inj->hyper; p.inject = inj->inject; p.hc = inj->hc; }
         return qk_launch_proj(&p, stream);

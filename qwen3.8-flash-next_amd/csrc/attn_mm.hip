@@ -40,8 +40,7 @@ struct AmArgs {
     float *po;             /* [n, h, nch, hd] */
     float2 *pml;           /* [n, h, nch]: maximum (log2 units), sum */
     const float *qg;       /* [n, h, 2, hd] */
-    uint16_t *hi, *lo;     /* [n, h * hd] planes */
-    float *pg;             /* [h * hd / 64, qk_planes_ld(n)] */
+    qk_planes pl;          /* of h * hd columns */
     int n, h, kvh, hd, T, tiles, offset, comp, nb, kw, nch, ctiles, nqb;
 };
 
@@ -213,31 +212,6 @@ __device__ void am_slow(const AmArgs &a, int kh, int row0, int kt0, int kt1, int
     }
 }
 
-/* at most N copies of this wave in flight, its LDS reads done, and every
- * wave of the workgroup here */
-template <int N>
-__device__ __forceinline__ void am_sync() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14)); /* vmcnt(N) lgkmcnt(0) */
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
-typedef __attribute__((address_space(3))) uint32_t *am_lptr;
-
-/* one copy of a wave, 64 x 16 bytes from src + OFF + 16 lane to LDS byte
- * lds + OFF + 16 lane.  As an instruction of its own and not the builtin:
- * the compiler waits for every builtin copy in flight before the next LDS
- * read, whichever buffer it reads; am_sync has the waits these need.  No
- * register is written. */
-template <int OFF>
-__device__ __forceinline__ void am_copy(const uint4 *src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2"
-                 :
-                 : "v"(src), "s"(lds), "n"(OFF)
-                 : "memory", "m0");
-}
-
 /*
  * grid (nqb * kvh * nch).  Wave = 32 rows (columns of the instructions: all
  * scores and outputs of a row sit in lanes l and l + 32), transposed
@@ -292,15 +266,15 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void k_am_attn(AmArgs a) {
     }
 
     const uint4 *src = a.img + ((size_t)kh * a.tiles + kt0) * 2 * IMG + 64 * NL * wave + lane;
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(am_lptr)&ring[0][0] + 1024 * NL * wave);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(qm_lptr)&ring[0][0] + 1024 * NL * wave);
     auto copy = [&](int hs) {
         const uint4 *p = src + (size_t)hs * IMG;
         const uint32_t d = lds0 + (uint32_t)(hs % 3) * (IMG * 16);
 #pragma unroll
         for (int i = 0; i < NL; i += 3) { /* NL = 3, 6, 9 or 12 */
-            am_copy<0>(p + 64 * i, d + 1024 * i);
-            am_copy<1024>(p + 64 * i, d + 1024 * i);
-            am_copy<2048>(p + 64 * i, d + 1024 * i);
+            qm_copy<0>(p + 64 * i, d + 1024 * i);
+            qm_copy<1024>(p + 64 * i, d + 1024 * i);
+            qm_copy<2048>(p + 64 * i, d + 1024 * i);
         }
     };
     const int nhs = 2 * (kt1 - kt0);
@@ -320,7 +294,7 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void k_am_attn(AmArgs a) {
         const uint32_t ml = qk_ld(mp + kt); /* used after the scores, so its wait finds the copies done */
         /* image hs is in LDS once this wave's older copies are done and every
          * wave has said so; the ring slot of hs + 2 was last read in hs - 1 */
-        am_sync<NL>();
+        qm_sync<NL>();
         if (hs + 2 < nhs) copy(hs + 2);
         qm_f32x16 st;
 #pragma unroll
@@ -369,8 +343,8 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void k_am_attn(AmArgs a) {
             l += st[i];
         }
         /* image hs + 1, as above */
-        if (hs + 2 < nhs) am_sync<NL>();
-        else am_sync<0>();
+        if (hs + 2 < nhs) qm_sync<NL>();
+        else qm_sync<0>();
         if (hs + 3 < nhs) copy(hs + 3);
         const uint4 *vb = ring[(hs + 1) % 3] + lane;
 #pragma unroll
@@ -407,15 +381,14 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void k_am_attn(AmArgs a) {
     if (lane < 32) a.pml[u] = make_float2(m, l);
 }
 
-/* one thread per 8 columns of a token's attention output: the key ranges up
- * to the token's own merged, the gate, and the planes (k_proj_pack's
- * arithmetic).  Bound: HBM / L2, the partial outputs read once. */
+/* a wave per 8 tokens x 64 columns of the attention output: the key ranges up
+ * to the token's own merged, the gate, and the planes.  Bound: HBM / L2, the
+ * partial outputs read once. */
 __global__ __launch_bounds__(256) void k_am_comb(AmArgs a) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const int cpt = a.h * a.hd / 8;
-    const int t = (int)(i / cpt);
-    if (t >= a.n) return; /* h * hd is a multiple of 64: whole groups leave together */
-    const int col = (int)(i - (size_t)t * cpt) * 8, hh = col / a.hd, d = col - hh * a.hd;
+    const int G = a.h * a.hd / 64, lane = threadIdx.x & 63;
+    const int w = blockIdx.x * 4 + (threadIdx.x >> 6), rb = w / G, gr = w - rb * G;
+    if (8 * rb >= a.n) return;
+    const int t = min(8 * rb + (lane & 7), a.n - 1), col = 64 * gr + 8 * (lane >> 3), hh = col / a.hd, d = col - hh * a.hd;
     const int live = min((a.offset + t) / (AM_KT * a.ctiles) + 1, a.nch);
     const size_t u = ((size_t)t * a.h + hh) * a.nch;
     float M = -INFINITY, L = 0.0f, x[8];
@@ -438,14 +411,7 @@ __global__ __launch_bounds__(256) void k_am_comb(AmArgs a) {
     const float gv[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
     for (int j = 0; j < 8; j++) x[j] = (x[j] * inv) * qk_sigmoid(gv[j]);
-    uint32_t ph[4], pl[4];
-    float s = qk_f32x8_pairs(x, ph, pl);
-    ((uint4 *)a.hi)[i] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-    ((uint4 *)a.lo)[i] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-    s += qk_dpp<QK_DPP_XOR1>(s);
-    s += qk_dpp<QK_DPP_XOR2>(s);
-    s += __shfl_xor(s, 4, QK_WAVE);
-    if ((i & 7) == 0) a.pg[(size_t)(col >> 6) * qk_planes_ld(a.n) + t] = -128.0f * s;
+    qm_pack_store(a.pl, 8 * rb + (lane & 7), a.n, gr, G, x);
 }
 
 /* ------------------------------------------------------------ host side */
@@ -491,7 +457,7 @@ extern "C" int qk_launch_attn_mm(const qk_at_shape *s, int n, int offset, int T,
     a.po = sc->part;
     a.pml = (float2 *)(sc->part + (size_t)n * s->h * a.nch * s->hd);
     a.qg = qg;
-    a.hi = sc->pl.hi; a.lo = sc->pl.lo; a.pg = sc->pl.pg;
+    a.pl = sc->pl;
     hipLaunchKernelGGL(k_am_prep, dim3(a.tiles, s->kvh), dim3(256), 0, st, a);
     int rc = QK_CHECK_LAUNCH();
     if (rc) return rc;
@@ -510,6 +476,6 @@ extern "C" int qk_launch_attn_mm(const qk_at_shape *s, int n, int offset, int T,
     }
     rc = QK_CHECK_LAUNCH();
     if (rc) return rc;
-    hipLaunchKernelGGL(k_am_comb, dim3((unsigned)(((size_t)n * (s->h * s->hd / 8) + 255) / 256)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_am_comb, dim3(qm_pack_wgs(n, s->h * s->hd / 64)), dim3(256), 0, st, a);
     return QK_CHECK_LAUNCH();
 }

@@ -31,7 +31,7 @@
  * for a | b, and k_dn_pack in place of k_dn_out's scaling and conv state.
  * The GEMVs above walk the tokens one after another and convert x again in
  * every wave: at 2048 tokens (hidden 2048, heads 16/32 of 128) 10050 us for
- * k_dn_in and 5830 for k_dn_out, against 315 + 16 and 141 + 21.
+ * k_dn_in and 5830 for k_dn_out, against 240 + 11 and 100 + 24.
  * From QK_DN_CHUNK_N tokens on k_dn_rec gives way to dn_chunk.hip (3225 us
  * there against 103 + 142).
  *
@@ -41,6 +41,7 @@
 #include "qk_device.h"
 #include "gemv_parts.h"
 #include "dn_rec.h"
+#include "mfma_parts.h"
 
 #define DN_RPW 4   /* rows per wave in the two GEMV kernels */
 
@@ -312,22 +313,20 @@ __global__ __launch_bounds__(256) void k_dn_out(DnOutArgs a) {
 
 /*
  * Many tokens: core scaled by its head's 1/sqrt(sum(o^2)/dv + eps) as
- * operand planes of out_proj (k_proj_pack's arithmetic and order), one
- * thread per 8 columns; the workgroups past the planes move the conv state
+ * operand planes of out_proj; the workgroups past the planes move the conv state
  * on by n tokens.
  */
 struct DnPackArgs {
     const float *core, *ssp, *mixed;
     const float *z, *norm_w; /* z set: core is o itself (the chunked recurrence), gated here */
     float *conv_state;
-    uint16_t *hi, *lo;
-    float *pg;
+    qk_planes pl;
     int n, value_dim, dv, kc, conv_dim;
 };
 
 __global__ __launch_bounds__(256) void k_dn_pack(DnPackArgs a) {
-    const size_t nch = (size_t)a.n * (a.value_dim / 8);
-    const unsigned pack_wgs = (unsigned)(nch / 256 + 1);
+    const int G = a.value_dim / 64;
+    const unsigned pack_wgs = qm_pack_wgs(a.n, G);
     if (blockIdx.x >= pack_wgs) {
         const int cc = (int)(blockIdx.x - pack_wgs) * 256 + threadIdx.x;
         if (cc >= a.conv_dim) return;
@@ -344,13 +343,13 @@ __global__ __launch_bounds__(256) void k_dn_pack(DnPackArgs a) {
             if (j < a.kc - 1) a.conv_state[(size_t)j * a.conv_dim + cc] = cv[j];
         return;
     }
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= nch) return; /* nch is a multiple of 8: whole groups leave together */
-    const int cpr = a.value_dim / 8;
-    const size_t t = i / cpr;
-    const int col = (int)(i - t * cpr) * 8, nb = a.dv / DN_RB;
+    const int u = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int rb = u / G, g = u - rb * G, t = 8 * rb + (lane & 7);
+    if (8 * rb >= a.n) return;
+    const int tc = min(t, a.n - 1), col = 64 * g + 8 * (lane >> 3), nb = a.dv / DN_RB;
+    const size_t i = ((size_t)tc * a.value_dim + col) / 8;
     const float4 a0 = qk_ld((const float4 *)a.core + 2 * i), a1 = qk_ld((const float4 *)a.core + 2 * i + 1);
-    const float *sp = a.ssp + (t * (a.value_dim / a.dv) + col / a.dv) * nb;
+    const float *sp = a.ssp + ((size_t)tc * (a.value_dim / a.dv) + col / a.dv) * nb;
     float ss = 0.0f;
     for (int j0 = 0; j0 < nb; j0 += 8) {
         float pv[8];
@@ -372,14 +371,7 @@ __global__ __launch_bounds__(256) void k_dn_pack(DnPackArgs a) {
     }
 #pragma unroll
     for (int j = 0; j < 8; j++) v[j] *= r;
-    uint32_t ph[4], pl[4];
-    float s = qk_f32x8_pairs(v, ph, pl);
-    ((uint4 *)a.hi)[i] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-    ((uint4 *)a.lo)[i] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-    s += qk_dpp<QK_DPP_XOR1>(s);
-    s += qk_dpp<QK_DPP_XOR2>(s);
-    s += __shfl_xor(s, 4, QK_WAVE);
-    if ((i & 7) == 0) a.pg[(size_t)(col >> 6) * qk_planes_ld(a.n) + t] = -128.0f * s;
+    qm_pack_store(a.pl, t, a.n, g, G, v);
 }
 
 /* ------------------------------------------------------------ host side */
@@ -415,18 +407,19 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     int rc;
     const bool mm = n >= QK_DN_MM_N;
     if (mm) {
-        if (!pl || !pl->hi || !pl->lo || !pl->pg) return (int)hipErrorInvalidValue;
+        if (!pl || !pl->a || !pl->pg) return (int)hipErrorInvalidValue;
         rc = qk_launch_proj_pack(x, n, s->d, pl, stream);
         if (rc) return rc;
         qk_proj p = {};
         p.seg[0] = {W->qkv_q, W->qkv_s, W->qkv_b, mixed, conv_dim, conv_dim};
         p.seg[1] = {W->z_q, W->z_s, W->z_b, z, value_dim, value_dim};
         p.nseg = 2;
-        p.hi = pl->hi; p.lo = pl->lo; p.pg = pl->pg;
+        p.pl = *pl;
         p.K = s->d; p.n = n;
+        p.bw[0] = W->a_w; p.bw[1] = W->b_w;
+        p.bout[0] = av; p.bout[1] = bv;
+        p.brows = s->hv;
         rc = qk_launch_proj(&p, stream);
-        if (rc) return rc;
-        rc = qk_launch_proj_bf16(W->a_w, W->b_w, s->hv, pl->hi, pl->lo, s->d, n, av, bv, stream);
         if (rc) return rc;
     } else {
     DnInArgs ia;
@@ -473,16 +466,15 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     if (rc) return rc;
 
     if (mm) {
-        const DnPackArgs ka = {core, ssp, mixed, chunks ? z : nullptr, W->norm_w, conv_state, pl->hi, pl->lo,
-                               pl->pg, n, value_dim, s->dv, s->kc, conv_dim};
-        hipLaunchKernelGGL(k_dn_pack, dim3((unsigned)((size_t)n * (value_dim / 8) / 256 + 1 + (conv_dim + 255) / 256)),
+        const DnPackArgs ka = {core, ssp, mixed, chunks ? z : nullptr, W->norm_w, conv_state, *pl, n, value_dim, s->dv, s->kc, conv_dim};
+        hipLaunchKernelGGL(k_dn_pack, dim3(qm_pack_wgs(n, value_dim / 64) + (unsigned)(conv_dim + 255) / 256),
                            dim3(256), 0, st, ka);
         rc = QK_CHECK_LAUNCH();
         if (rc) return rc;
         qk_proj p = {};
         p.seg[0] = {W->out_q, W->out_s, W->out_b, out, s->d, s->d};
         p.nseg = 1;
-        p.hi = pl->hi; p.lo = pl->lo; p.pg = pl->pg;
+        p.pl = *pl;
         p.K = value_dim; p.n = n;
         if (inj) { p.hyper = inj_in->hyper; p.inject = inj_in->inject; p.hc = inj_in->hc; }
         return qk_launch_proj(&p, stream);

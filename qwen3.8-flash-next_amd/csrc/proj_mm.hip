@@ -6,16 +6,20 @@
  * (reference c/src/model.c:193-202 -> gemm_q4, kernel.c:230-309).
  *
  * The arithmetic is the expert GEMM's (ffn_mfma.hip): f32 activations as
- * bf16 hi + lo planes in (x_i, x_{i+4}) pair order (k_pack_rows), codes as
+ * bf16 hi + lo planes in (x_i, x_{i+4}) pair order (qk_planes), codes as
  * the exact bf16 numbers 16 + q, every 64-column group's accumulator
  * started at -16 sum(x) so it ends at sum x q, one fp32 fma per output
  * and group for the scale, and the bias term sum_g b_g X_g as a K = G
  * product at the end.  Accumulation is fp32 throughout, as in the GEMV.
  *
  * Bound: matrix cores (n = 2048: 103 GFLOP for qkv | z, twice that issued
- * for hi + lo).  Measured 300 us there, 343 TFLOP/s (687 issued); the matrix
- * cores are busy 31 % of the time, the rest goes to the decode, the scale
- * fmas and the waits between them.
+ * for hi + lo).  Measured 240 us there, 430 TFLOP/s (860 issued); the matrix
+ * cores are busy 40 % of the time, the rest goes to the decode, the scale
+ * fmas and the waits between them.  The address path comes next: a load whose
+ * lanes sit in different rows touches a line per row, so the planes lie in
+ * operand order (qk_planes; as rows, staged through registers, 272 us), the
+ * group sums by group and the scales come eight at a time (one at a time with
+ * a sum per row 315).
  *
  * 32x32x16 lane layout: A lane l holds row l%32, B lane l column l%32, both
  * eight K elements of half h = l/32; D lane l holds column l%32, rows
@@ -94,16 +98,16 @@ __device__ __forceinline__ void pj_store(const qk_proj &a, float *out, int ostri
 
 /*
  * Tiles of BM = 32*RT*WR tokens x BN = 64*(4/WR) columns; wave (wr, wc) owns
- * RT row tiles and two column tiles.  Per group the rows' planes go through
- * LDS (two buffers, one barrier, 16-byte chunks xor-swizzled by row so a
- * wave's reads touch every bank), loaded into registers one group ahead;
- * code words and scales come straight into registers one group ahead.
+ * RT row tiles and two column tiles.  Per group the rows' planes are copied
+ * into LDS as they lie (two buffers, one barrier), the next group's under
+ * this one's products; code words and scales come straight into registers
+ * one group ahead.
  */
 template <int RT, int WR, bool INJ, bool S8>
 __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
     constexpr int BM = 32 * RT * WR, WC = 4 / WR;
-    constexpr int ACH = BM * 8 / PJ_THREADS; /* chunks per thread and plane */
-    __shared__ __attribute__((aligned(16))) uint4 s_a[2][2][BM * 8];
+    constexpr int NRT = RT * WR, NC = NRT * 2; /* row tiles; 1 KB copies per wave and group */
+    __shared__ __attribute__((aligned(16))) uint4 s_a[2][NRT][8][64]; /* [plane, K-step][lane] */
     __shared__ __attribute__((aligned(16))) float s_p[2][BM];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 31, h = lane >> 5;
@@ -134,31 +138,24 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
         sp[ct] = s + (size_t)(r0 + 32 * ct + c) * G;
     }
 
-    const uint16_t *ap[ACH];
-#pragma unroll
-    for (int i = 0; i < ACH; i++) {
-        const int ci = tid + PJ_THREADS * i;
-        ap[i] = a.hi + (size_t)min(m0 + (ci >> 3), a.n - 1) * a.K + (ci & 7) * 8;
-    }
-    const size_t lo_off = a.lo - a.hi, ldp = qk_planes_ld(a.n);
-    uint4 ar[2][ACH];
+    /* wave w copies units NC w .. of the group's 8 NRT (a unit: 1 KB); row
+     * tiles past the last repeat it */
+    const size_t ldp = qk_planes_ld(a.n);
+    const int lastrt = (a.n - 1) >> 5;
+    const uint4 *ap = (const uint4 *)a.pl.a + (size_t)min((m0 >> 5) + NC * wave / 8, lastrt) * G * 512 + NC * wave % 8 * 64 + lane;
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(qm_lptr)&s_a[0][0][0][0] + 1024 * NC * wave);
     float pr = 0.0f;
-    auto load_a = [&](int g) {
+    auto copy_a = [&](int g, int buf) {
 #pragma unroll
-        for (int i = 0; i < ACH; i++) {
-            ar[0][i] = qk_ld((const uint4 *)(ap[i] + 64 * g));
-            ar[1][i] = qk_ld((const uint4 *)(ap[i] + lo_off + 64 * g));
+        for (int i = 0; i < NC; i += 4) {
+            const uint4 *src = ap + (size_t)g * 512 + 64 * i;
+            const uint32_t dst = lds0 + buf * (NRT * 8192) + 1024 * i;
+            qm_copy<0>(src, dst);
+            qm_copy<1024>(src, dst);
+            qm_copy<2048>(src, dst);
+            qm_copy<3072>(src, dst);
         }
-        pr = qk_ld(a.pg + ldp * g + min(m0 + min(tid, BM - 1), a.n - 1));
-    };
-    auto store_a = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < ACH; i++) {
-            const int ci = tid + PJ_THREADS * i, row = ci >> 3, kc = ci & 7;
-            s_a[buf][0][row * 8 + (kc ^ (row & 7))] = ar[0][i];
-            s_a[buf][1][row * 8 + (kc ^ (row & 7))] = ar[1][i];
-        }
-        if (tid < BM) s_p[buf][tid] = pr * QM_P16;
+        pr = qk_ld(a.pl.pg + ldp * g + min(m0 + min(tid, BM - 1), a.n - 1));
     };
     uint4 wv[2];
     /* scales: eight groups of a column per load where its row of scales is
@@ -184,12 +181,12 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[rt][ct][i] = 0.0f;
 
-    load_a(0);
+    copy_a(0, 0);
     load_w(0);
     load_s(s8, 0);
+    if (tid < BM) s_p[0][tid] = pr * QM_P16;
     for (int g = 0; g < G; g++) {
         const int buf = g & 1;
-        store_a(buf);
         qm_bf16x8 bop[2][4];
         float sc[2];
 #pragma unroll
@@ -206,8 +203,11 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
                 s8[ct].w >>= 16;
             }
         }
+        /* group g is in LDS; its buffer's partner was last read in group g-1,
+         * before this barrier */
+        qm_sync<0>();
         const int gn = min(g + 1, G - 1); /* past the end: loaded, not used */
-        load_a(gn);
+        if (g + 1 < G) copy_a(gn, buf ^ 1); /* no copy may outlive the workgroup */
         load_w(gn);
         if (!S8) {
             load_s(s8, gn);
@@ -218,11 +218,8 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
                 s8[1] = s8n[1];
             }
         }
-        /* buffer buf was last read in group g-2, before the barrier of g-1 */
-        qk_lds_barrier();
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
-            const int row = 32 * (RT * wr + rt) + c;
             qm_f32x16 p;
 #pragma unroll
             for (int i4 = 0; i4 < 4; i4++) {
@@ -235,7 +232,7 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
             for (int tm = 0; tm < 2; tm++)
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    const qm_bf16x8 A = __builtin_bit_cast(qm_bf16x8, s_a[buf][tm][row * 8 + ((4 * h + j) ^ (row & 7))]);
+                    const qm_bf16x8 A = __builtin_bit_cast(qm_bf16x8, s_a[buf][RT * wr + rt][4 * tm + j][lane]);
 #pragma unroll
                     for (int ct = 0; ct < 2; ct++) t[ct] = PJ_MFMA(A, bop[ct][j], (tm == 0 && j == 0) ? p : t[ct]);
                 }
@@ -244,6 +241,7 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
 #pragma unroll
                 for (int i = 0; i < 16; i++) acc[rt][ct][i] = fmaf(sc[ct], t[ct][i], acc[rt][ct][i]);
         }
+        if (tid < BM) s_p[buf ^ 1][tid] = pr * QM_P16;
     }
 
     /* bias term: acc += sum_g b[col][g] X[row][g] */
@@ -254,7 +252,7 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             qm_bf16x8 X[3];
-            pj_bias_x(a.pg + min(m0 + 32 * (RT * wr + rt) + c, a.n - 1), ldp, k0 + 8 * h, G, X);
+            pj_bias_x(a.pl.pg + min(m0 + 32 * (RT * wr + rt) + c, a.n - 1), ldp, k0 + 8 * h, G, X);
 #pragma unroll
             for (int ct = 0; ct < 2; ct++)
 #pragma unroll
@@ -274,6 +272,65 @@ __global__ __launch_bounds__(PJ_THREADS, 2) void k_proj_mm(qk_proj a) {
 }
 
 /*
+ * Dense bf16 weight rows (DeltaNet in_proj_a | in_proj_b, the hyper
+ * connection's inject) on the same planes: 32 tokens x 32 of the matrices'
+ * rows, K dealt to WK waves.  In k_proj_few these are its last column blocks;
+ * the large tiles run them as a launch of their own.
+ */
+template <int WK, int LDR>
+__device__ __forceinline__ void pj_bf16_tile(const qk_proj &a, int m0, int tile, float (&s_r)[WK][32][LDR]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = lane & 31, h = lane >> 5;
+    const int rows = a.bw[1] ? 2 * a.brows : a.brows;
+    const int cc = min(tile * 32 + c, rows - 1);
+    const uint16_t *wp = (cc < a.brows ? a.bw[0] + (size_t)cc * a.K : a.bw[1] + (size_t)(cc - a.brows) * a.K) + 32 * h;
+    const int G = a.K >> 6;
+    const uint4 *ap = (const uint4 *)a.pl.a + (size_t)(m0 >> 5) * G * 512 + lane;
+    qm_f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i] = 0.0f;
+    uint4 av[2][4], wv[4];
+    auto load = [&](int g) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            av[0][j] = qk_ld(ap + (size_t)g * 512 + 64 * j);
+            av[1][j] = qk_ld(ap + (size_t)g * 512 + 256 + 64 * j);
+            wv[j] = qk_ld((const uint4 *)(wp + 64 * g) + j);
+        }
+    };
+    if (wave < G) load(wave);
+    for (int g = wave; g < G; g += WK) {
+        qm_bf16x8 A[2][4], B[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            uint32_t p[4];
+            qk_bf16x8_to_pairs(wv[j], p);
+            B[j] = __builtin_bit_cast(qm_bf16x8, make_uint4(p[0], p[1], p[2], p[3]));
+            A[0][j] = __builtin_bit_cast(qm_bf16x8, av[0][j]);
+            A[1][j] = __builtin_bit_cast(qm_bf16x8, av[1][j]);
+        }
+        load(min(g + WK, G - 1));
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            acc = PJ_MFMA(A[0][j], B[j], acc);
+            acc = PJ_MFMA(A[1][j], B[j], acc);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) s_r[wave][8 * (i >> 2) + 4 * h + (i & 3)][c] = acc[i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 32 * 32; i += 64 * WK) {
+        const int row = i >> 5, r = tile * 32 + (i & 31);
+        if (m0 + row >= a.n || r >= rows) continue;
+        float v = s_r[0][row][i & 31];
+#pragma unroll
+        for (int w = 1; w < WK; w++) v += s_r[w][row][i & 31];
+        const int k = r >= a.brows;
+        qk_st(a.bout[k] + (size_t)(m0 + row) * a.brows + (r - k * a.brows), v);
+    }
+}
+
+/*
  * Few tokens: 32 tokens x 32*CT columns per workgroup, the K groups dealt to
  * its WK waves (wave w: groups w, w + WK, ..) and their sums added through
  * LDS in wave order.  A tile of 32 rows leaves too few workgroups of the
@@ -286,7 +343,19 @@ __global__ __launch_bounds__(64 * WK) void k_proj_few(qk_proj a) {
     __shared__ float s_r[WK][32][32 * CT + 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 31, h = lane >> 5;
-    const int nt = blockIdx.x, m0 = blockIdx.y * 32;
+    /* workgroup L runs on XCD L % 8.  While the planes are small next to an
+     * XCD's L2 the row tiles of a column block stay together there (the weights
+     * are read once), else the column blocks of a row tile */
+    const int i8 = blockIdx.x >> 3, x8 = blockIdx.x & 7, ncb = a.ntiles + a.btiles;
+    int nt, mt;
+    if (a.byrow) { mt = i8 / ncb * 8 + x8; nt = i8 % ncb; }
+    else { nt = i8 / a.mtiles * 8 + x8; mt = i8 % a.mtiles; }
+    if (mt >= a.mtiles || nt >= ncb) return;
+    const int m0 = mt * 32;
+    if (nt >= a.ntiles) {
+        pj_bf16_tile<WK>(a, m0, nt - a.ntiles, s_r);
+        return;
+    }
     const int G = a.K >> 6;
     const size_t wrow = (size_t)a.K >> 3;
     const uint32_t *q;
@@ -302,54 +371,59 @@ __global__ __launch_bounds__(64 * WK) void k_proj_few(qk_proj a) {
         wq[ct] = q + (size_t)(r0 + 32 * ct + c) * wrow + 4 * h;
         sp[ct] = s + (size_t)(r0 + 32 * ct + c) * G;
     }
-    const size_t lo_off = a.lo - a.hi, ldp = qk_planes_ld(a.n);
-    const uint16_t *ap = a.hi + (size_t)min(m0 + c, a.n - 1) * a.K + 32 * h;
-    uint4 wv[CT], av[2][4];
-    uint16_t sv[CT];
-    float pv[16];
-    auto load = [&](int g) {
+    const size_t ldp = qk_planes_ld(a.n);
+    const uint4 *ap = (const uint4 *)a.pl.a + (size_t)(m0 >> 5) * G * 512 + lane;
+    struct Op {
+        uint4 w[CT], a[2][4];
+        uint16_t s[CT];
+        float4 p[4];
+    };
+    auto load = [&](Op &o, int g) {
+        g = min(g, G - 1); /* past the end: loaded, not used */
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) {
-            wv[ct] = qk_ld((const uint4 *)(wq[ct] + 8 * g));
-            sv[ct] = qk_ld(sp[ct] + g);
+            o.w[ct] = qk_ld((const uint4 *)(wq[ct] + 8 * g));
+            o.s[ct] = qk_ld(sp[ct] + g);
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            av[0][j] = qk_ld((const uint4 *)(ap + 64 * g) + j);
-            av[1][j] = qk_ld((const uint4 *)(ap + lo_off + 64 * g) + j);
+            o.a[0][j] = qk_ld(ap + (size_t)g * 512 + 64 * j);
+            o.a[1][j] = qk_ld(ap + (size_t)g * 512 + 256 + 64 * j);
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++) { /* rows past n: within the leading dimension, not used */
-            const float4 v = qk_ld((const float4 *)(a.pg + ldp * g + m0 + 8 * i + 4 * h));
-            pv[4 * i] = v.x; pv[4 * i + 1] = v.y; pv[4 * i + 2] = v.z; pv[4 * i + 3] = v.w;
-        }
+        for (int i = 0; i < 4; i++) /* rows past n: within the leading dimension, not used */
+            o.p[i] = qk_ld((const float4 *)(a.pl.pg + ldp * g + m0 + 8 * i + 4 * h));
     };
     qm_f32x16 acc[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ct++)
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[ct][i] = 0.0f;
-    if (wave < G) load(wave);
-    for (int g = wave; g < G; g += WK) {
+    auto step = [&](Op &o, int g) {
         qm_bf16x8 A[2][4], bop[CT][4];
         float sc[CT];
         qm_f32x16 t[CT];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            A[0][j] = __builtin_bit_cast(qm_bf16x8, av[0][j]);
-            A[1][j] = __builtin_bit_cast(qm_bf16x8, av[1][j]);
+            A[0][j] = __builtin_bit_cast(qm_bf16x8, o.a[0][j]);
+            A[1][j] = __builtin_bit_cast(qm_bf16x8, o.a[1][j]);
         }
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) {
-            bop[ct][0] = qm_codes16(wv[ct].x);
-            bop[ct][1] = qm_codes16(wv[ct].y);
-            bop[ct][2] = qm_codes16(wv[ct].z);
-            bop[ct][3] = qm_codes16(wv[ct].w);
-            sc[ct] = qk_bf16(sv[ct]);
+            bop[ct][0] = qm_codes16(o.w[ct].x);
+            bop[ct][1] = qm_codes16(o.w[ct].y);
+            bop[ct][2] = qm_codes16(o.w[ct].z);
+            bop[ct][3] = qm_codes16(o.w[ct].w);
+            sc[ct] = qk_bf16(o.s[ct]);
 #pragma unroll
-            for (int i = 0; i < 16; i++) t[ct][i] = pv[i] * QM_P16;
+            for (int i = 0; i < 4; i++) {
+                t[ct][4 * i] = o.p[i].x * QM_P16;
+                t[ct][4 * i + 1] = o.p[i].y * QM_P16;
+                t[ct][4 * i + 2] = o.p[i].z * QM_P16;
+                t[ct][4 * i + 3] = o.p[i].w * QM_P16;
+            }
         }
-        load(min(g + WK, G - 1));
+        load(o, g + 2 * WK);
 #pragma unroll
         for (int tm = 0; tm < 2; tm++)
 #pragma unroll
@@ -360,11 +434,18 @@ __global__ __launch_bounds__(64 * WK) void k_proj_few(qk_proj a) {
         for (int ct = 0; ct < CT; ct++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[ct][i] = fmaf(sc[ct], t[ct][i], acc[ct][i]);
+    };
+    Op o0, o1; /* two groups in flight */
+    load(o0, wave);
+    load(o1, wave + WK);
+    for (int g = wave; g < G; g += 2 * WK) {
+        step(o0, g);
+        if (g + WK < G) step(o1, g + WK);
     }
     /* bias term, 16 groups per step, the steps dealt to the waves */
     for (int k0 = 16 * wave; k0 < G; k0 += 16 * WK) {
         qm_bf16x8 X[3];
-        pj_bias_x(a.pg + min(m0 + c, a.n - 1), ldp, k0 + 8 * h, G, X);
+        pj_bias_x(a.pl.pg + min(m0 + c, a.n - 1), ldp, k0 + 8 * h, G, X);
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) {
             const qm_bf16x8 bb = pj_bias_w(b + (size_t)(r0 + 32 * ct + c) * G, k0 + 8 * h, G);
@@ -387,88 +468,21 @@ __global__ __launch_bounds__(64 * WK) void k_proj_few(qk_proj a) {
     }
 }
 
-/*
- * bf16 weight rows (DeltaNet in_proj_a | in_proj_b, 2*hv of them) on the
- * same planes: workgroup = 32 tokens x 32 rows, K dealt to four waves.
- */
-struct PjBf16Args {
-    const uint16_t *w[2];  /* [rows, K] each */
-    float *out[2];         /* [n, rows] */
-    const uint16_t *hi, *lo;
-    int rows, K, n;
-};
-
-__global__ __launch_bounds__(256) void k_proj_bf16(PjBf16Args a) {
-    __shared__ float s_r[4][32][33];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c = lane & 31, h = lane >> 5;
-    const int m0 = blockIdx.y * 32, col = blockIdx.x * 32 + c;
-    const int cc = min(col, 2 * a.rows - 1);
-    const uint16_t *wp = (cc < a.rows ? a.w[0] + (size_t)cc * a.K : a.w[1] + (size_t)(cc - a.rows) * a.K) + 32 * h;
-    const size_t lo_off = a.lo - a.hi;
-    const uint16_t *ap = a.hi + (size_t)min(m0 + c, a.n - 1) * a.K + 32 * h;
-    const int G = a.K >> 6;
-    qm_f32x16 acc;
-#pragma unroll
-    for (int i = 0; i < 16; i++) acc[i] = 0.0f;
-    uint4 av[2][4], wv[4];
-    auto load = [&](int g) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            av[0][j] = qk_ld((const uint4 *)(ap + 64 * g) + j);
-            av[1][j] = qk_ld((const uint4 *)(ap + lo_off + 64 * g) + j);
-            wv[j] = qk_ld((const uint4 *)(wp + 64 * g) + j);
-        }
-    };
-    if (wave < G) load(wave);
-    for (int g = wave; g < G; g += 4) {
-        qm_bf16x8 A[2][4], B[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            uint32_t p[4];
-            qk_bf16x8_to_pairs(wv[j], p);
-            B[j] = __builtin_bit_cast(qm_bf16x8, make_uint4(p[0], p[1], p[2], p[3]));
-            A[0][j] = __builtin_bit_cast(qm_bf16x8, av[0][j]);
-            A[1][j] = __builtin_bit_cast(qm_bf16x8, av[1][j]);
-        }
-        load(min(g + 4, G - 1));
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            acc = PJ_MFMA(A[0][j], B[j], acc);
-            acc = PJ_MFMA(A[1][j], B[j], acc);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 16; i++) s_r[wave][8 * (i >> 2) + 4 * h + (i & 3)][c] = acc[i];
-    __syncthreads();
-    for (int i = threadIdx.x; i < 32 * 32; i += 256) {
-        const int row = i >> 5, r = blockIdx.x * 32 + (i & 31);
-        if (m0 + row >= a.n || r >= 2 * a.rows) continue;
-        const float v = ((s_r[0][row][i & 31] + s_r[1][row][i & 31]) + s_r[2][row][i & 31]) + s_r[3][row][i & 31];
-        const int k = r >= a.rows;
-        qk_st(a.out[k] + (size_t)(m0 + row) * a.rows + (r - k * a.rows), v);
-    }
+template <int WK>
+__global__ __launch_bounds__(64 * WK) void k_proj_bf16(qk_proj a) {
+    __shared__ float s_r[WK][32][33];
+    pj_bf16_tile<WK>(a, blockIdx.y * 32, blockIdx.x, s_r);
 }
 
-/* k_pack_rows (ffn_mfma.hip) with the group sums transposed: a tile's rows
- * then read them as runs, where a row-major sum is a line per row */
-__global__ __launch_bounds__(256) void k_proj_pack(const float *x, size_t nchunks, int G, size_t ldp, uint16_t *hi,
-                                                   uint16_t *lo, float *pg) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= nchunks) return; /* nchunks is a multiple of 8: whole groups leave together */
-    const float4 a0 = qk_ld((const float4 *)x + 2 * i), a1 = qk_ld((const float4 *)x + 2 * i + 1);
+/* f32 rows -> planes, a wave per 8 rows x 64 columns.  Bound: HBM / L2. */
+__global__ __launch_bounds__(256) void k_proj_pack(const float *x, int n, int G, qk_planes pl) {
+    const int u = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int rb = u / G, g = u - rb * G, t = 8 * rb + (lane & 7);
+    if (8 * rb >= n) return;
+    const float4 *p = (const float4 *)x + ((size_t)min(t, n - 1) * G + g) * 16 + 2 * (lane >> 3);
+    const float4 a0 = qk_ld(p), a1 = qk_ld(p + 1);
     const float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-    uint32_t ph[4], pl[4];
-    float s = qk_f32x8_pairs(v, ph, pl);
-    ((uint4 *)lo)[i] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-    ((uint4 *)hi)[i] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-    s += qk_dpp<QK_DPP_XOR1>(s);
-    s += qk_dpp<QK_DPP_XOR2>(s);
-    s += __shfl_xor(s, 4, QK_WAVE);
-    if ((i & 7) == 0) {
-        const size_t row = (i >> 3) / G;
-        pg[((i >> 3) - row * G) * ldp + row] = -128.0f * s;
-    }
+    qm_pack_store(pl, t, n, g, G, v);
 }
 
 /* ------------------------------------------------------------ host side */
@@ -476,16 +490,14 @@ __global__ __launch_bounds__(256) void k_proj_pack(const float *x, size_t nchunk
 extern "C" int qk_launch_proj_pack(const float *x, int n, int K, const qk_planes *pl, void *stream) {
     if (n <= 0) return 0;
     if (K <= 0 || K % 64) return (int)hipErrorInvalidValue;
-    const size_t nch = (size_t)n * (K / 8);
-    hipLaunchKernelGGL(k_proj_pack, dim3((unsigned)((nch + 255) / 256)), dim3(256), 0, (hipStream_t)stream, x, nch, K / 64,
-                       qk_planes_ld(n), pl->hi, pl->lo, pl->pg);
+    hipLaunchKernelGGL(k_proj_pack, dim3(qm_pack_wgs(n, K / 64)), dim3(256), 0, (hipStream_t)stream, x, n, K / 64, *pl);
     return QK_CHECK_LAUNCH();
 }
 
 extern "C" int qk_launch_proj(const qk_proj *in, void *stream) {
     qk_proj a = *in;
     if (a.n <= 0) return 0;
-    if (a.K <= 0 || a.K % 64 || a.nseg < 1 || a.nseg > QK_PROJ_SEGS || (a.hyper && (a.nseg != 1 || a.hc < 1)))
+    if (a.K <= 0 || a.K % 64 || (a.bw[0] && a.brows < 1) || a.nseg < 1 || a.nseg > QK_PROJ_SEGS || (a.hyper && (a.nseg != 1 || a.hc < 1)))
         return (int)hipErrorInvalidValue;
     int end = 0;
     for (int i = 0; i < a.nseg; i++) {
@@ -512,30 +524,36 @@ extern "C" int qk_launch_proj(const qk_proj *in, void *stream) {
     } while (0)
 #define PJ_FEW(CT, WK)                                                                                       \
     do {                                                                                                     \
-        const dim3 grid(end * 2 / CT, (a.n + 31) / 32);                                                      \
+        a.ntiles = end * 2 / CT;                                                                             \
+        const int ncb = a.ntiles + bt;                                                                       \
+        const dim3 grid(8u * (a.byrow ? (unsigned)(mt + 7) / 8 * ncb : (unsigned)(ncb + 7) / 8 * mt));       \
         if (inj) hipLaunchKernelGGL((k_proj_few<CT, WK, true>), grid, dim3(64 * WK), 0, st, a);              \
         else hipLaunchKernelGGL((k_proj_few<CT, WK, false>), grid, dim3(64 * WK), 0, st, a);                 \
     } while (0)
+    const int mt = (a.n + 31) / 32, bt = a.bw[0] ? ((a.bw[1] ? 2 : 1) * a.brows + 31) / 32 : 0;
+    a.btiles = bt;
     /* The K-split tiles while the others would leave the chip short of
      * workgroups (DeltaNet mixer of hidden 2048, both products, us without
      * the recurrence: 77 tokens 85 against 120, 256 tokens 133 / 145, 512
-     * tokens 245 / 200; up to 32 tokens the narrower one, 9 tokens 47
-     * against 52); 128-row tiles once they give every CU four workgroups
-     * (2048 tokens: 427 together, 64-row tiles 520). */
-    if (a.n <= 32) PJ_FEW(1, 4);
-    else if (a.n <= QK_PROJ_FEW_N) PJ_FEW(2, 4);
-    else if ((long long)((a.n + 127) / 128) * ((end + 1) / 2) < 1024) PJ_MM(1, 2);
+     * tokens 245 / 200), split the deeper the fewer tiles there are: four
+     * waves from a workgroup per CU on (two fit), eight below, of 64 columns
+     * while those are still 128 workgroups.  128-row tiles once they give every
+     * CU four workgroups (2048 tokens: 427 together, 64-row tiles 520). */
+    const long long wg64 = (long long)((a.n + 63) / 64) * ((end + 1) / 2);
+    if (a.n <= QK_PROJ_FEW_N || wg64 < 256) {
+        a.mtiles = mt;
+        a.byrow = (size_t)a.n * a.K * 4 > ((size_t)4 << 20);
+        if (end * mt >= 256 || a.K < 1024) PJ_FEW(2, 4);
+        else if (8 * end * mt >= 1024) PJ_FEW(2, 8);
+        else PJ_FEW(1, 8);
+        return QK_CHECK_LAUNCH();
+    }
+    if ((long long)((a.n + 127) / 128) * ((end + 1) / 2) < 1024) PJ_MM(1, 2);
     else PJ_MM(2, 2);
 #undef PJ_MM
 #undef PJ_FEW
-    return QK_CHECK_LAUNCH();
-}
-
-extern "C" int qk_launch_proj_bf16(const uint16_t *w0, const uint16_t *w1, int rows, const uint16_t *hi,
-                                   const uint16_t *lo, int K, int n, float *out0, float *out1, void *stream) {
-    if (n <= 0) return 0;
-    if (K <= 0 || K % 64 || rows <= 0) return (int)hipErrorInvalidValue;
-    const PjBf16Args a = {{w0, w1}, {out0, out1}, hi, lo, rows, K, n};
-    hipLaunchKernelGGL(k_proj_bf16, dim3((2 * rows + 31) / 32, (n + 31) / 32), dim3(256), 0, (hipStream_t)stream, a);
+    int rc = QK_CHECK_LAUNCH();
+    if (rc || !bt) return rc;
+    hipLaunchKernelGGL(k_proj_bf16<8>, dim3(bt, mt), dim3(512), 0, st, a);
     return QK_CHECK_LAUNCH();
 }

@@ -157,12 +157,13 @@ int qmoe_attn_create(qmoe_attn_ctx **out, const qmoe_attn_config *cfg, qmoe_err 
     const size_t units = n * ((cap + 255) / 256) > (cap + 63) / 64 ? n * ((cap + 255) / 256) : (cap + 63) / 64;
     const size_t kw = (cap / (size_t)s.comp + 31) / 32 + 1;
     const size_t wide = n >= QK_AT_MM_N ? n * (d > ok ? d : ok) : 0;
-    const size_t ssz[15] = {n * qr * 4, n * kr * 4, n * kr * 4, n * (ih + 1) * ihd * 4, n * h * hd * 4,
+    const size_t ssz[14] = {n * qr * 4, n * kr * 4, n * kr * 4, n * (ih + 1) * ihd * 4, n * h * hd * 4,
                             n * ih * ihd * 4, n * kw * 4, units * h * (hd + 2) * 4, n * h * hd * 4,
-                            n * (cap / (size_t)s.comp) * 4, wide * 2, wide * 2, wide ? qk_planes_ld((int)n) * (wide / n / 64) * 4 : 0,
+                            n * (cap / (size_t)s.comp) * 4, wide ? qk_planes_bytes((int)n, wide / n) : 0,
+                           wide ? qk_planes_ld((int)n) * (wide / n / 64) * 4 : 0,
                             wide ? qk_am_img_bytes(&s) : 0, wide ? qk_am_mask_bytes(&s, cfg->max_tokens) : 0};
-    size_t stot = 0, soff[15];
-    for (int i = 0; i < 15; i++) {
+    size_t stot = 0, soff[14];
+    for (int i = 0; i < 14; i++) {
         soff[i] = stot;
         stot = at_align(stot + ssz[i]);
     }
@@ -185,11 +186,10 @@ int qmoe_attn_create(qmoe_attn_ctx **out, const qmoe_attn_config *cfg, qmoe_err 
     c->sc.ao = (float *)(b + soff[8]);
     c->sc.skey = (uint32_t *)(b + soff[9]);
     if (wide) {
-        c->sc.pl.hi = (uint16_t *)(b + soff[10]);
-        c->sc.pl.lo = (uint16_t *)(b + soff[11]);
-        c->sc.pl.pg = (float *)(b + soff[12]);
-        c->sc.img = b + soff[13];
-        c->sc.kmask = (uint32_t *)(b + soff[14]);
+        c->sc.pl.a = b + soff[10];
+        c->sc.pl.pg = (float *)(b + soff[11]);
+        c->sc.img = b + soff[12];
+        c->sc.kmask = (uint32_t *)(b + soff[13]);
     }
     for (int l = 0; l < cfg->n_layers; l++)
         if (at_hip_fail(err, (int)hipMalloc(&c->layers[l].mem, total), "layer weights")) {

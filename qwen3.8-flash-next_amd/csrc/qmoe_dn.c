@@ -111,11 +111,12 @@ int qmoe_dn_create(qmoe_dn_ctx **out, const qmoe_dn_config *cfg, qmoe_err *err) 
     c->layers = (dn_layer *)calloc((size_t)cfg->n_layers, sizeof(dn_layer));
     const size_t n = (size_t)cfg->max_tokens;
     const size_t wide = n >= QK_DN_MM_N ? n * (d > value_dim ? d : value_dim) : 0;
-    const size_t ssz[10] = {n * conv_dim * 4, n * value_dim * 4, n * hv * 4, n * hv * 4, n * value_dim * 4,
-                           n * (value_dim / 16) * 4, wide * 2, wide * 2, wide ? qk_planes_ld((int)n) * (wide / n / 64) * 4 : 0,
+    const size_t ssz[9] = {n * conv_dim * 4, n * value_dim * 4, n * hv * 4, n * hv * 4, n * value_dim * 4,
+                           n * (value_dim / 16) * 4, wide ? qk_planes_bytes((int)n, wide / n) : 0,
+                           wide ? qk_planes_ld((int)n) * (wide / n / 64) * 4 : 0,
                            n >= QK_DN_CHUNK_N ? qk_dn_chunk_bytes(&s, cfg->max_tokens) : 0};
-    size_t stot = 0, soff[10];
-    for (int i = 0; i < 10; i++) {
+    size_t stot = 0, soff[9];
+    for (int i = 0; i < 9; i++) {
         soff[i] = stot;
         stot = dn_align(stot + ssz[i]);
     }
@@ -132,11 +133,10 @@ int qmoe_dn_create(qmoe_dn_ctx **out, const qmoe_dn_config *cfg, qmoe_err *err) 
     c->core = (float *)(b + soff[4]);
     c->ssp = (float *)(b + soff[5]);
     if (wide) {
-        c->pl.hi = (uint16_t *)(b + soff[6]);
-        c->pl.lo = (uint16_t *)(b + soff[7]);
-        c->pl.pg = (float *)(b + soff[8]);
+        c->pl.a = b + soff[6];
+        c->pl.pg = (float *)(b + soff[7]);
     }
-    if (n >= QK_DN_CHUNK_N) c->chunk = (float *)(b + soff[9]);
+    if (n >= QK_DN_CHUNK_N) c->chunk = (float *)(b + soff[8]);
     for (int l = 0; l < cfg->n_layers; l++) {
         if (dn_hip_fail(err, (int)hipMalloc(&c->layers[l].mem, total), "layer weights")) {
             qmoe_dn_destroy(c);

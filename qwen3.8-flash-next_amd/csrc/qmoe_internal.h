@@ -212,21 +212,32 @@ typedef struct {
     int hc;
 } qk_inject;
 
-/* operand planes of a mixer call, in its scratch: hi, lo [n, K] as
- * qk_launch_pack_rows writes them, pg [K/64, qk_planes_ld(n)] */
+/* f32 rows [n, K] as matrix operands, in a call's scratch (K a multiple of
+ * 64).  a: bf16 hi + lo in (x_i, x_{i+4}) pair order per 8 columns, in the
+ * order in which the lanes of v_mfma_f32_32x32x16 take them: per 32 rows and
+ * 64 columns 8 KB, [hi | lo][K-step j][lane l] of 16 bytes with row l % 32
+ * and the 8 columns 8 (4 (l / 32) + j) on, so every operand load or copy is
+ * one run of 1 KB (as rows, a load touched 32 lines).  pg: -128 * the sums of
+ * 64 columns, [K/64, qk_planes_ld(n)]. */
 typedef struct {
-    uint16_t *hi, *lo;
+    void *a; /* qk_planes_bytes */
     float *pg;
 } qk_planes;
 #ifdef __HIPCC__
-__host__ __device__
+#define QK_HD __host__ __device__
+#else
+#define QK_HD
 #endif
-static inline size_t qk_planes_ld(int n) { return ((size_t)n + 31) / 32 * 32; }
+QK_HD static inline size_t qk_planes_ld(int n) { return ((size_t)n + 31) / 32 * 32; }
+static inline size_t qk_planes_bytes(int n, size_t K) { return qk_planes_ld(n) * K * 4; }
+/* 16-byte unit of row t, 8-column chunk ch of K = 64 G columns: hi (lo: + 256) */
+QK_HD static inline size_t qk_planes_at(int t, int ch, int G) {
+    return (((size_t)(t >> 5) * G + (ch >> 3)) * 8 + (ch & 3)) * 64 + ((ch >> 2) & 1) * 32 + (t & 31);
+}
 int qk_launch_proj_pack(const float *x, int n, int K, const qk_planes *pl, void *stream);
 
 /* the mixers' q4 projections of many tokens on MFMA (proj_mm.hip): every
- * segment's out[t * ostride + r] = x[t] . W[r] over operand planes hi, lo
- * [n, K] and pg of qk_launch_proj_pack.  rows and K
+ * segment's out[t * ostride + r] = x[t] . W[r] over the planes pl.  rows and K
  * are multiples of 64.  With hyper set (one segment): also the inject
  * update of its output, [n, hc, ostride]; out may then be NULL. */
 #define QK_PROJ_SEGS 3
@@ -239,18 +250,19 @@ typedef struct {
 typedef struct {
     qk_proj_seg seg[QK_PROJ_SEGS];
     int nseg;
-    const uint16_t *hi, *lo;
-    const float *pg;
+    qk_planes pl;
     int K, n;
     float *hyper;
     const float *inject;
     int hc;
-    int end64[QK_PROJ_SEGS], mtiles, ntiles; /* filled by the launcher */
+    /* one or two dense bf16 matrices [brows, K] on the same planes (bw[0] NULL:
+     * none; bw[1] may be NULL) -> bout [n, brows] */
+    const uint16_t *bw[2];
+    float *bout[2];
+    int brows;
+    int end64[QK_PROJ_SEGS], mtiles, ntiles, btiles, byrow; /* filled by the launcher */
 } qk_proj;
 int qk_launch_proj(const qk_proj *a, void *stream);
-/* two bf16 matrices of `rows` rows on the same planes -> out0, out1 [n, rows] */
-int qk_launch_proj_bf16(const uint16_t *w0, const uint16_t *w1, int rows, const uint16_t *hi,
-                        const uint16_t *lo, int K, int n, float *out0, float *out1, void *stream);
 /* the mixers take their matrix kernels from this many tokens on.  DeltaNet's
  * per-token GEMVs cost 9 us a token at hidden 2048: 66 us the mixer at 6
  * tokens, 94 at 9, against 57 and 63.  Attention's whole path (projections,
