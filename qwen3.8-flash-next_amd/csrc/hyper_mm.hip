@@ -1,20 +1,20 @@
 /*
  * hyper_mm.hip -- the MLP hyper connection's producer (gated_residual,
  * reference C port model.c:728-796) for many tokens, on bf16 MFMA
- * (v_mfma_f32_16x16x32_bf16), in four launches:
+ * (v_mfma_f32_16x16x32_bf16), in three launches, or four from HM_PLANES_N to
+ * HM_PLANES_MAX tokens:
  *
- *   k_hc_pack    per token: the copies' RMS scales r_h = 1/sqrt(ss/d + eps)
- *                and a = x * hc_norm as MFMA operand planes (bf16 hi + lo,
- *                x = hi + lo to 2^-17, in (x_i, x_{i+4}) pair order per 8
- *                columns) with P_g = -128 * (sum of the group's 64 a);
  *   k_hc_mm_down partial products of the down projection over one K range
- *                of one copy h, sum_k a_k W[r, k], and of the inject
- *                projection (bf16 weights; none for the final mixer) as
+ *                of one copy h, sum_k a_k W[r, k] with a = x * hc_norm formed
+ *                as it is read (bf16 hi + lo, x = hi + lo to 2^-17), and of the
+ *                inject projection (bf16 weights; none for the final mixer) as
  *                one more column block;
- *   k_hc_finish  per token: w = silu(sum_h r_h * partial_h / hc) (the norm
- *                scale is constant over a copy, so it applies after the
- *                product), inject = 2 sigmoid(sum_h r_h * partial_h / hc),
- *                and the planes of w;
+ *   k_hc_finish  per token: w = silu(sum_h r_h * partial_h / hc) with the RMS
+ *                scales r_h = 1/sqrt(ss/d + eps) (constant over a copy, so it
+ *                applies after the product), inject = 2 sigmoid(sum_h r_h *
+ *                partial_h / hc), and the planes of w;
+ *   or k_hc_pack (r_h, and the normed rows as qk_planes), the down and inject
+ *                products of proj_mm.hip, and k_hc_act (w, inject);
  *   k_hc_mm_up   the up projection of w for the columns h*d + i of every
  *                copy h of a block of columns i, so each lane ends with all
  *                copies of its (row, i): mixed = mean_h sigmoid(up) *
@@ -456,6 +456,120 @@ __global__ __launch_bounds__(256) void k_hc_normed(const float *hyper, const flo
         normed[(size_t)t * D + i] = hyper[(size_t)t * D + i] * rs[(size_t)t * hc + i / d] * norm_w[i];
 }
 
+/* ------------------------------------------------ normed rows as planes */
+
+struct HcPackArgs {
+    const float *hyper, *norm_w; /* [n, hc*d], [hc*d] */
+    qk_planes pl;                /* of hc * d columns */
+    float *rs;                   /* [n, hc] */
+    int n, hc, d;
+    float eps;
+};
+
+/* grid (ceil(n / 8), hc), 8 waves: wave w normalises copy h of token 8 b + w
+ * (the row stays in registers between its sum of squares and its planes, d <=
+ * 2048) and the workgroup writes normed = (x r_h) hc_norm as operand planes,
+ * through LDS so that each 128-byte run of 8 rows is stored whole.  Bound:
+ * HBM, 4 bytes in and 4 out per element. */
+__global__ __launch_bounds__(512) void k_hc_pack(HcPackArgs a) {
+    __shared__ __attribute__((aligned(16))) uint4 s_p[2][256 * 8]; /* [chunk][row ^ chunk % 8] */
+    __shared__ float s_g[32][8];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = blockIdx.y;
+    const int t = min((int)blockIdx.x * 8 + w, a.n - 1);
+    const int c8 = a.d >> 3; /* 8-column chunks of a copy, a multiple of 8 */
+    const size_t base = ((size_t)t * a.hc + h) * c8;
+    float x[4][8];
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int c = lane + 64 * i;
+        const float4 *p = (const float4 *)a.hyper + 2 * (base + min(c, c8 - 1));
+        const float4 x0 = qk_ld(p), x1 = qk_ld(p + 1);
+        const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            x[i][j] = v[j];
+            ss = c < c8 ? fmaf(v[j], v[j], ss) : ss;
+        }
+    }
+    ss = qk_group_sum<64>(ss);
+    const float r = 1.0f / sqrtf(ss / (float)a.d + a.eps);
+    if (lane == 0) a.rs[(size_t)t * a.hc + h] = r; /* a repeated last token: the same value */
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int c = lane + 64 * i;
+        if (c < c8) { /* whole groups of 8 lanes together */
+            const float4 *p = (const float4 *)(a.norm_w + (size_t)h * a.d) + 2 * c;
+            const float4 w0 = qk_ld(p), w1 = qk_ld(p + 1);
+            const float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = (x[i][j] * r) * wv[j];
+            uint32_t ph[4], pl[4];
+            float s = qk_f32x8_pairs(v, ph, pl);
+            s_p[0][8 * c + (w ^ (c & 7))] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
+            s_p[1][8 * c + (w ^ (c & 7))] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
+            s += qk_dpp<QK_DPP_XOR1>(s);
+            s += qk_dpp<QK_DPP_XOR2>(s);
+            s += __shfl_xor(s, 4, QK_WAVE);
+            if ((c & 7) == 0) s_g[c >> 3][w] = -128.0f * s;
+        }
+    }
+    __syncthreads();
+    const int G = a.hc * a.d >> 6;
+    for (int i = threadIdx.x; i < 8 * c8; i += 512) {
+        const int c = i >> 3, rw = i & 7, tt = (int)blockIdx.x * 8 + rw;
+        if (tt >= a.n) continue;
+        uint4 *o = (uint4 *)a.pl.a + qk_planes_at(tt, h * c8 + c, G);
+        o[0] = s_p[0][8 * c + (rw ^ (c & 7))];
+        o[256] = s_p[1][8 * c + (rw ^ (c & 7))];
+        if ((c & 7) == 0) a.pl.pg[(size_t)((h * c8 + c) >> 3) * qk_planes_ld(a.n) + tt] = s_g[c >> 3][rw];
+    }
+}
+
+struct HcActArgs {
+    const float *pre, *ipre; /* [n, R], [n, hc] */
+    uint4 *whi, *wlo;
+    float *wp, *inject;
+    int hc, R, n;
+};
+
+/* w = silu(pre / hc) as planes, one thread per 8 columns; the last workgroups
+ * inject = 2 sigmoid(ipre / hc) */
+__global__ __launch_bounds__(256) void k_hc_act(HcActArgs a) {
+    const size_t nch = (size_t)a.n * (a.R >> 3);
+    const unsigned wgs = (unsigned)((nch + 255) / 256);
+    const float inv = 1.0f / (float)a.hc;
+    if (blockIdx.x >= wgs) {
+        const int i = (int)(blockIdx.x - wgs) * 256 + threadIdx.x;
+        if (i < a.n * a.hc) a.inject[i] = 2.0f * qk_sigmoid(qk_ld(a.ipre + i) * inv);
+        return;
+    }
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nch) return; /* nch is a multiple of 8 */
+    const float4 a0 = qk_ld((const float4 *)a.pre + 2 * i), a1 = qk_ld((const float4 *)a.pre + 2 * i + 1);
+    float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = qk_silu(v[j] * inv);
+    uint32_t hi[4], lo[4];
+    float g = qk_f32x8_pairs(v, hi, lo);
+    a.whi[i] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    a.wlo[i] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    g += qk_dpp<QK_DPP_XOR1>(g);
+    g += qk_dpp<QK_DPP_XOR2>(g);
+    g += __shfl_xor(g, 4, QK_WAVE);
+    if ((i & 7) == 0) a.wp[i >> 3] = -128.0f * g;
+}
+
+/* Token counts whose down product runs on packed planes (proj_mm.hip): the
+ * partial products of k_hc_mm_down form the operands again in every column
+ * pass and copy.  hc 4, hidden 2048, rank 320, the whole mix in us, parts
+ * against planes: 200 tokens 40 / 45, 256 tokens 40 / 54, 300 tokens 68 / 54,
+ * 512 tokens 68 / 56, 1024 tokens 107 / 77, 1400 tokens 125 / 123, 2000 tokens
+ * 132 / 138, 4096 tokens 205 / 277. */
+#define HM_PLANES_N 257
+#define HM_PLANES_MAX 1280
+
 /* ---------------------------------------------------------------- launch */
 
 /* column tiles per pass of the down GEMM: few tokens take narrow passes
@@ -493,6 +607,16 @@ static void hc_launch_up(int hc, dim3 grid, hipStream_t st, const HcMmUpArgs &ua
     }
 }
 
+static size_t hm_up256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+/* workspace of a packed pass over n tokens: planes, group sums, the products
+ * before their activation, rs, the planes of w */
+static size_t hm_planes_bytes(int hc, int d, int R, int n) {
+    const size_t D = (size_t)hc * d, N = (size_t)n;
+    return hm_up256(qk_planes_bytes(n, D)) + hm_up256(qk_planes_ld(n) * (D / 64) * 4) + hm_up256(N * R * 4) + hm_up256(N * hc * 4) * 2 +
+           2 * hm_up256(N * R * 2) + hm_up256(N * (R / 64) * 4);
+}
+
 extern "C" int qk_launch_hc_mm(const float *hyper, const float *norm_w, const uint32_t *dq,
                                const uint16_t *ds, const uint16_t *db, const uint32_t *uq,
                                const uint16_t *us, const uint16_t *ub, const uint16_t *inject_w,
@@ -502,6 +626,43 @@ extern "C" int qk_launch_hc_mm(const float *hyper, const float *norm_w, const ui
     if (hc < 1 || hc > HC_MAX || d % 64 || R % 64 || R > 2048) return (int)hipErrorInvalidValue;
     if (inject_w && !inject) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)stream;
+    if (n >= HM_PLANES_N && n <= HM_PLANES_MAX) {
+        const size_t D = (size_t)hc * d;
+        char *p = (char *)ws;
+        auto take = [&](size_t bytes) {
+            char *r = p;
+            p += hm_up256(bytes);
+            return (void *)r;
+        };
+        qk_planes pl;
+        pl.a = take(qk_planes_bytes(n, D));
+        pl.pg = (float *)take(qk_planes_ld(n) * (D / 64) * 4);
+        float *pre = (float *)take((size_t)n * R * 4);
+        float *rs = (float *)take((size_t)n * hc * 4), *ipre = (float *)take((size_t)n * hc * 4);
+        uint4 *whi = (uint4 *)take((size_t)n * R * 2), *wlo = (uint4 *)take((size_t)n * R * 2);
+        float *wp = (float *)take((size_t)n * (R / 64) * 4);
+        const HcPackArgs pa = {hyper, norm_w, pl, rs, n, hc, d, eps};
+        hipLaunchKernelGGL(k_hc_pack, dim3((n + 7) / 8, hc), dim3(512), 0, st, pa);
+        int rc = QK_CHECK_LAUNCH();
+        if (rc) return rc;
+        qk_proj q = {};
+        q.seg[0] = {dq, ds, db, pre, R, R};
+        q.nseg = 1;
+        q.pl = pl;
+        q.K = (int)D; q.n = n;
+        q.bw[0] = inject_w; q.bout[0] = ipre; q.brows = hc;
+        rc = qk_launch_proj(&q, stream);
+        if (rc) return rc;
+        const HcActArgs aa = {pre, ipre, whi, wlo, wp, inject_w ? inject : nullptr, hc, R, n};
+        const unsigned wgs = (unsigned)(((size_t)n * (R >> 3) + 255) / 256);
+        hipLaunchKernelGGL(k_hc_act, dim3(wgs + (inject_w ? (n * hc + 255) / 256 : 0)), dim3(256), 0, st, aa);
+        rc = QK_CHECK_LAUNCH();
+        if (rc) return rc;
+        HcMmUpArgs ua{whi, wlo, wp, uq, us, ub, hyper, norm_w, rs, mixed, d, R, n};
+        hc_launch_up<4>(hc, dim3((n + HM_BM - 1) / HM_BM, d / 64), st, ua);
+        if (normed) hipLaunchKernelGGL(k_hc_normed, dim3(n), dim3(256), 0, st, hyper, norm_w, rs, hc, d, normed);
+        return QK_CHECK_LAUNCH();
+    }
     const int kspl = qk_hc_mm_kspl(hc, d, R, n), parts = hc * kspl;
     /* workspace carve-up (qk_hc_mm_ws_bytes) */
     char *p = (char *)ws;
@@ -538,11 +699,13 @@ extern "C" int qk_launch_hc_mm(const float *hyper, const float *norm_w, const ui
 }
 
 extern "C" size_t qk_hc_mm_ws_bytes(int hc, int d, int R, int max_n) {
-    /* the largest carve-up over n <= max_n: every term grows with n except
-     * the parts, whose count times n is at most hc * max(n, 1024) */
+    /* the largest carve-up over n <= max_n.  On the parts every term grows
+     * with n except theirs, whose count times n is at most hc * max(n, 1024);
+     * on the planes all grow */
     const size_t n = (size_t)max_n;
     const size_t pn = (size_t)hc * (n > 1024 ? n : 1024);
-    auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    return up(pn * R * 4) + up(pn * 16 * 4) + up(pn * 4) + up(n * hc * 4) + 2 * up(n * R * 2) +
-           up(n * (R / 64) * 4) + 256;
+    const size_t parts = hm_up256(pn * R * 4) + hm_up256(pn * 16 * 4) + hm_up256(pn * 4) + hm_up256(n * hc * 4) +
+                         2 * hm_up256(n * R * 2) + hm_up256(n * (R / 64) * 4) + 256;
+    const size_t planes = max_n < HM_PLANES_N ? 0 : hm_planes_bytes(hc, d, R, max_n < HM_PLANES_MAX ? max_n : HM_PLANES_MAX);
+    return parts > planes ? parts : planes;
 }

@@ -6,6 +6,7 @@ import pytest
 
 import test_gpu_attention as ta
 import test_gpu_deltanet as td
+import test_gpu_gated_residual as tg
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +117,24 @@ def test_deltanet_values_past_the_products(torch_dev, bad):
             assert td.rel(got[t], ref[t]) < td.REL_L2, t
     else:
         assert np.isnan(got[j:]).all()
+
+
+# the hyper connection's packed planes: the first and last count on them and
+# their neighbours, a repeated last token, odd copies, small copies
+@pytest.mark.parametrize("hc,d,R", [(4, 256, 128), (3, 192, 64), (8, 64, 64), (1, 2048, 320)])
+@pytest.mark.parametrize("n", [256, 257, 1280, 1281])
+def test_hyper_token_counts(torch_dev, hc, d, R, n):
+    torch, dev = torch_dev
+    orc = tg.orc
+    hp = orc.Hyper(hc, d, R, seed=21, layer=1, norm_std=0.1)
+    hyper = orc.gen_hyper(n, hc, d, seed=n) * 2.0
+    with tg.load_pkg().GatedResidualContext(d, hc, R, n_slots=1, max_tokens=1281) as gr:
+        gr.upload_slot(0, hp.arrays())
+        ht = torch.from_numpy(hyper).to(dev)
+        m, i = gr.mix(0, ht)
+        m2, _ = gr.mix(0, ht, want_inject=False)
+        torch.cuda.synchronize()
+        ref = hp.mix(hyper)
+        tg.assert_close(m.cpu().numpy(), ref["mixed"], "mixed")
+        tg.assert_close(i.cpu().numpy(), ref["inject"], "inject")
+        assert torch.equal(m, m2)
