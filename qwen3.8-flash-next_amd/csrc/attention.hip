@@ -71,7 +71,7 @@ template <int P, bool INJ>
 __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
     const int lane = threadIdx.x & 63;
     const int r0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * AT_RPW;
-    if (r0 >= a.start[a.nseg]) return;
+    const bool on = r0 < a.start[a.nseg];
     /* the wave's segment (a segment's row count is a multiple of AT_RPW) */
     RowSeg S = a.seg[0];
     int rr = r0;
@@ -80,28 +80,39 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
     if (a.nseg > 3 && r0 >= a.start[3]) { S = a.seg[3]; rr = r0 - a.start[3]; }
     const int CH = a.K >> 5, G = a.K >> 6;
     const size_t wrow = (size_t)a.K >> 3;
-    if (S.q) {
+    /* the waves of a workgroup with q4 rows all take part in x's way through
+     * LDS, also one that has bf16 rows or none */
+    const int w0 = blockIdx.x * 4 * AT_RPW;
+    bool q4 = false;
+    for (int i = 0; i < a.nseg; i++)
+        if (a.seg[i].q && a.start[i] < w0 + 4 * AT_RPW && a.start[i + 1] > w0) q4 = true;
+    if (q4) {
+        const bool mine = on && S.q;
+        __shared__ XWg<P> sh;
+        XWgRaw<P> xr;
+        load_xwg<P>(a.x, a.K, xr);
         uint4 wq[AT_RPW][P];
         float ws[AT_RPW][P], wb[AT_RPW][P];
+        if (mine)
 #pragma unroll
-        for (int j = 0; j < AT_RPW; j++) {
-            const int r = rr + j;
+            for (int j = 0; j < AT_RPW; j++) {
+                const int r = rr + j;
 #pragma unroll
-            for (int ps = 0; ps < P; ps++) {
-                const int c0 = ps * 64 + lane;
-                const bool ok = c0 < CH;
-                const int c = ok ? c0 : 0;
-                wq[j][ps] = qk_ld((const uint4 *)(S.q + (size_t)r * wrow + 4 * (size_t)c));
-                ws[j][ps] = ok ? qk_bf16(qk_ld(S.s + (size_t)r * G + (c >> 1))) : 0.0f;
-                wb[j][ps] = ok ? qk_bf16(qk_ld(S.b + (size_t)r * G + (c >> 1))) : 0.0f;
-                if (!ok) wq[j][ps] = make_uint4(0u, 0u, 0u, 0u);
+                for (int ps = 0; ps < P; ps++) {
+                    const int c0 = ps * 64 + lane;
+                    const bool ok = c0 < CH;
+                    const int c = ok ? c0 : 0;
+                    wq[j][ps] = qk_ld((const uint4 *)(S.q + (size_t)r * wrow + 4 * (size_t)c));
+                    ws[j][ps] = ok ? qk_bf16(qk_ld(S.s + (size_t)r * G + (c >> 1))) : 0.0f;
+                    wb[j][ps] = ok ? qk_bf16(qk_ld(S.b + (size_t)r * G + (c >> 1))) : 0.0f;
+                    if (!ok) wq[j][ps] = make_uint4(0u, 0u, 0u, 0u);
+                }
             }
-        }
         for (int t = 0; t < a.n; t++) {
             /* INJ: the token's inject weights and the hyper values of this
              * wave's rows, loaded with x (clamped addresses) */
             float iv[INJ ? QK_INJECT_MAX_HC : 1], hv[INJ ? AT_RPW : 1][INJ ? QK_INJECT_MAX_HC : 1];
-            if (INJ) {
+            if (INJ && mine) {
 #pragma unroll
                 for (int q = 0; q < QK_INJECT_MAX_HC; q++) {
                     const int qc = min(q, a.hc - 1);
@@ -112,26 +123,30 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
                             qk_ld(a.hyper + ((size_t)t * a.hc + qc) * S.ostride + min(rr + j, S.rows - 1));
                 }
             }
-            XRaw<P, false> xr;
-            load_xraw<64, P, false>(a.x, (size_t)t, a.K, lane, xr);
-            XPairs<64, P, false> xp;
-            convert_xraw<64, P, false>(xr, a.K, lane, xp);
+            store_xwg<P>(xr, a.K, sh);
+            qk_lds_barrier();
+            if (t + 1 < a.n) load_xwg<P>(a.x + (size_t)(t + 1) * a.K, a.K, xr);
+            if (mine) {
+                XPairs<64, P, false> xp;
+                read_xwg<P>(sh, lane, xp);
 #pragma unroll
-            for (int j = 0; j < AT_RPW; j++) {
-                const float v = qk_group_sum<64>(row_part<64, P, false>(wq[j], ws[j], wb[j], xp));
-                if (lane == 0) {
-                    if (S.out) qk_st(S.out + (size_t)t * S.ostride + rr + j, v);
-                    if (INJ)
+                for (int j = 0; j < AT_RPW; j++) {
+                    const float v = qk_group_sum<64>(row_part<64, P, false>(wq[j], ws[j], wb[j], xp));
+                    if (lane == 0) {
+                        if (S.out) qk_st(S.out + (size_t)t * S.ostride + rr + j, v);
+                        if (INJ)
 #pragma unroll
-                        for (int q = 0; q < QK_INJECT_MAX_HC; q++)
-                            if (q < a.hc)
-                                qk_st(a.hyper + ((size_t)t * a.hc + q) * S.ostride + rr + j,
-                                      fmaf(iv[INJ ? q : 0], v, hv[INJ ? j : 0][INJ ? q : 0]));
+                            for (int q = 0; q < QK_INJECT_MAX_HC; q++)
+                                if (q < a.hc)
+                                    qk_st(a.hyper + ((size_t)t * a.hc + q) * S.ostride + rr + j,
+                                          fmaf(iv[INJ ? q : 0], v, hv[INJ ? j : 0][INJ ? q : 0]));
+                    }
                 }
             }
+            if (t + 1 < a.n) qk_lds_barrier(); /* sh is rewritten for the next token */
         }
-        return;
     }
+    if (!on || S.q) return;
     /* bf16 rows (index_qk_proj): f32 x times the bf16 weights in the
      * router's R64 order -- 8-element chunk c on lane c % 64, an fma chain
      * per lane over its chunks in ascending order from +0, the lanes added

@@ -56,26 +56,20 @@ struct DnInArgs {
     int d, n, conv_dim, value_dim, hv;
 };
 
-/* x chunks of token t as bf16 pairs: lane owns chunks ps*64 + lane */
-template <int P>
-__device__ __forceinline__ void dn_x_pairs(const float *x, int t, int K, int lane, XPairs<64, P, false> &xp) {
-    XRaw<P, false> xr;
-    load_xraw<64, P, false>(x, (size_t)t, K, lane, xr);
-    convert_xraw<64, P, false>(xr, K, lane, xp);
-}
-
 template <int P>
 __global__ __launch_bounds__(256) void k_dn_in(DnInArgs a) {
     const int lane = threadIdx.x & 63;
     const int r0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * DN_RPW;
     const int R1 = a.conv_dim, R2 = R1 + a.value_dim, R3 = R2 + a.hv, R = R3 + a.hv;
-    if (r0 >= R) return;
     const int CH = a.d >> 5, G = a.d >> 6;
     const size_t wrow = (size_t)a.d >> 3;
+    __shared__ XWg<P> sh;
+    XWgRaw<P> xr;
+    load_xwg<P>(a.x, a.d, xr);
+    /* q4 rows: codes, scales and biases of the wave's rows stay in registers */
+    uint4 wq[DN_RPW][P];
+    float ws[DN_RPW][P], wb[DN_RPW][P];
     if (r0 < R2) {
-        /* q4 rows: codes, scales and biases of the wave's rows stay in registers */
-        uint4 wq[DN_RPW][P];
-        float ws[DN_RPW][P], wb[DN_RPW][P];
 #pragma unroll
         for (int j = 0; j < DN_RPW; j++) {
             const int r = min(r0 + j, R2 - 1);
@@ -95,9 +89,14 @@ __global__ __launch_bounds__(256) void k_dn_in(DnInArgs a) {
                 if (!ok) wq[j][ps] = make_uint4(0u, 0u, 0u, 0u);
             }
         }
-        for (int t = 0; t < a.n; t++) {
-            XPairs<64, P, false> xp;
-            dn_x_pairs<P>(a.x, t, a.d, lane, xp);
+    }
+    for (int t = 0; t < a.n; t++) {
+        store_xwg<P>(xr, a.d, sh);
+        qk_lds_barrier();
+        if (t + 1 < a.n) load_xwg<P>(a.x + (size_t)(t + 1) * a.d, a.d, xr);
+        XPairs<64, P, false> xp;
+        read_xwg<P>(sh, lane, xp);
+        if (r0 < R2) {
 #pragma unroll
             for (int j = 0; j < DN_RPW; j++) {
                 const float v = qk_group_sum<64>(row_part<64, P, false>(wq[j], ws[j], wb[j], xp));
@@ -107,43 +106,40 @@ __global__ __launch_bounds__(256) void k_dn_in(DnInArgs a) {
                     else qk_st(a.z + (size_t)t * a.value_dim + (r - R1), v);
                 }
             }
-        }
-        return;
-    }
-    /* bf16 rows (in_proj_a, in_proj_b): w pairs against the x pairs */
-    for (int t = 0; t < a.n; t++) {
-        XPairs<64, P, false> xp;
-        dn_x_pairs<P>(a.x, t, a.d, lane, xp);
+        } else if (r0 < R) {
+            /* bf16 rows (in_proj_a, in_proj_b): w pairs against the x pairs */
 #pragma unroll
-        for (int j = 0; j < DN_RPW; j++) {
-            const int r = r0 + j;
-            const int rc = min(r, R - 1);
-            const bool isb = rc >= R3;
-            const uint16_t *w = (isb ? a.b_w : a.a_w) + (size_t)(isb ? rc - R3 : rc - R2) * a.d;
-            float part = 0.0f;
+            for (int j = 0; j < DN_RPW; j++) {
+                const int r = r0 + j;
+                const int rc = min(r, R - 1);
+                const bool isb = rc >= R3;
+                const uint16_t *w = (isb ? a.b_w : a.a_w) + (size_t)(isb ? rc - R3 : rc - R2) * a.d;
+                float part = 0.0f;
 #pragma unroll
-            for (int ps = 0; ps < P; ps++) {
-                const int c0 = ps * 64 + lane;
-                const bool ok = c0 < CH;
-                const uint4 *src = (const uint4 *)(w + 32 * (size_t)(ok ? c0 : 0));
+                for (int ps = 0; ps < P; ps++) {
+                    const int c0 = ps * 64 + lane;
+                    const bool ok = c0 < CH;
+                    const uint4 *src = (const uint4 *)(w + 32 * (size_t)(ok ? c0 : 0));
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    uint32_t wp[4];
-                    qk_bf16x8_to_pairs(qk_ld(src + g), wp);
+                    for (int g = 0; g < 4; g++) {
+                        uint32_t wp[4];
+                        qk_bf16x8_to_pairs(qk_ld(src + g), wp);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const uint32_t w2 = ok ? wp[i] : 0u;
-                        part = qk_dot2(xp.hi[ps][4 * g + i], w2, part);
-                        part = qk_dot2(xp.lo[ps][4 * g + i], w2, part);
+                        for (int i = 0; i < 4; i++) {
+                            const uint32_t w2 = ok ? wp[i] : 0u;
+                            part = qk_dot2(xp.hi[ps][4 * g + i], w2, part);
+                            part = qk_dot2(xp.lo[ps][4 * g + i], w2, part);
+                        }
                     }
                 }
-            }
-            const float v = qk_group_sum<64>(part);
-            if (lane == 0 && r < R) {
-                if (r < R3) qk_st(a.a + (size_t)t * a.hv + (r - R2), v);
-                else qk_st(a.b + (size_t)t * a.hv + (r - R3), v);
+                const float v = qk_group_sum<64>(part);
+                if (lane == 0 && r < R) {
+                    if (r < R3) qk_st(a.a + (size_t)t * a.hv + (r - R2), v);
+                    else qk_st(a.b + (size_t)t * a.hv + (r - R3), v);
+                }
             }
         }
+        if (t + 1 < a.n) qk_lds_barrier(); /* sh is rewritten for the next token */
     }
 }
 
@@ -203,10 +199,10 @@ struct DnOutArgs {
  * One wave per DN_ORW rows of out_proj.  The gated norm's head factor
  * r = 1/sqrt(sum(o^2)/dv + eps) comes from the per-block sums of squares
  * of k_dn_rec (dv/16 of them per head, loaded together and added in
- * order); each lane scales its own chunks (32 columns of one head) and
- * splits them into bf16 hi + lo pairs.  The code words are loaded first;
- * the conv state moves on at the end (its stores would otherwise hold the
- * loads back).  No LDS and no barrier.
+ * order); each thread scales its units (8 columns of one head) and
+ * splits them into bf16 hi + lo pairs for the workgroup (XWg).  The code
+ * words are loaded first; the conv state moves on at the end (its stores
+ * would otherwise hold the loads back).
  */
 template <int P, bool INJ>
 __global__ __launch_bounds__(256) void k_dn_out(DnOutArgs a) {
@@ -230,7 +226,8 @@ __global__ __launch_bounds__(256) void k_dn_out(DnOutArgs a) {
     }
 
     const int r0 = (blockIdx.x * 4 + (tid >> 6)) * DN_ORW;
-    if (r0 < a.d) {
+    const int nb = a.dv / DN_RB;
+    __shared__ XWg<P> sh;
     uint4 wq[DN_ORW][P];
     float ws[DN_ORW][P], wb[DN_ORW][P];
 #pragma unroll
@@ -262,15 +259,12 @@ __global__ __launch_bounds__(256) void k_dn_out(DnOutArgs a) {
                         qk_ld(a.hyper + ((size_t)t * a.hc + jc) * a.d + min(r0 + q, a.d - 1));
             }
         }
-        XRaw<P, false> xr;
+        XWgRaw<P> xr;
+        load_xwg<P>(a.core + (size_t)t * K, K, xr);
 #pragma unroll
-        for (int ps = 0; ps < P; ps++) {
-            const int c0 = ps * 64 + lane;
-            const bool ok = c0 < CH;
-            const int c = ok ? c0 : 0;
-            const float4 *o = (const float4 *)(a.core + (size_t)t * K + 32 * c);
-            const int head = (32 * c) / a.dv, nb = a.dv / DN_RB;
-            const float *sp = a.ssp + ((size_t)t * (K / a.dv) + head) * nb;
+        for (int k = 0; k < P; k++) {
+            const int u = tid + 256 * k, c8 = u < (K >> 3) ? 8 * u : 0;
+            const float *sp = a.ssp + ((size_t)t * (K / a.dv) + c8 / a.dv) * nb;
             float ss = 0.0f;
             for (int j0 = 0; j0 < nb; j0 += DN_NBU) {
                 float pv[DN_NBU];
@@ -281,13 +275,15 @@ __global__ __launch_bounds__(256) void k_dn_out(DnOutArgs a) {
             }
             const float r = 1.0f / sqrtf(ss / (float)a.dv + 1e-6f);
 #pragma unroll
-            for (int w = 0; w < 8; w++) {
-                const float4 v = qk_ld(o + w);
-                xr.f[ps][w] = make_float4(v.x * r, v.y * r, v.z * r, v.w * r);
+            for (int w = 0; w < 2; w++) {
+                const float4 v = xr.f[k][w];
+                xr.f[k][w] = make_float4(v.x * r, v.y * r, v.z * r, v.w * r);
             }
         }
+        store_xwg<P>(xr, K, sh);
+        qk_lds_barrier();
         XPairs<64, P, false> xp;
-        convert_xraw<64, P, false>(xr, K, lane, xp);
+        read_xwg<P>(sh, lane, xp);
 #pragma unroll
         for (int j = 0; j < DN_ORW; j++) {
             const float v = qk_group_sum<64>(row_part<64, P, false>(wq[j], ws[j], wb[j], xp));
@@ -302,7 +298,7 @@ __global__ __launch_bounds__(256) void k_dn_out(DnOutArgs a) {
                                   fmaf(iv[INJ ? q : 0], v, hv[INJ ? j : 0][INJ ? q : 0]));
             }
         }
-    }
+        if (t + 1 < a.n) qk_lds_barrier(); /* sh is rewritten for the next token */
     }
     if (cthr) {
 #pragma unroll

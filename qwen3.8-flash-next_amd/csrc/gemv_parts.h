@@ -148,6 +148,77 @@ __device__ __forceinline__ void convert_xshare(const XShare<NG> &xq, int K, int 
     qk_wave_lds_sync();
 }
 
+/*
+ * One f32 row [K], K <= 2048 P, as the pairs of its chunks for the four waves
+ * of a workgroup: thread u loads and converts the 8-column units u + 256 k,
+ * and every lane takes its chunks from LDS, with exactly what convert_xraw
+ * gives.  A lane that loads its own 32 columns touches a line per lane and
+ * load, and each wave converts the row again: the DeltaNet mixer's rows at
+ * hidden 2048 (12352 of them, one token) took 9.0 us that way, DN_IN_US so.  hi, lo [w]: unit w of each
+ * chunk, rows 2 units apart modulo 8 so that the stores of 8 lanes (2 chunks)
+ * fall on distinct banks.
+ */
+template <int P>
+struct XWg {
+    uint4 hi[4][64 * P + 2], lo[4][64 * P + 2];
+    float4 gs[64 * P];
+};
+template <int P>
+struct XWgRaw {
+    float4 f[P][2];
+};
+
+template <int P>
+__device__ __forceinline__ void load_xwg(const float *x, int K, XWgRaw<P> &xr) {
+#pragma unroll
+    for (int k = 0; k < P; k++) {
+        const int u = threadIdx.x + 256 * k;
+        const float4 *src = (const float4 *)x + 2 * (u < (K >> 3) ? u : 0);
+        xr.f[k][0] = qk_ld(src);
+        xr.f[k][1] = qk_ld(src + 1);
+    }
+}
+
+template <int P>
+__device__ __forceinline__ void store_xwg(const XWgRaw<P> &xr, int K, XWg<P> &sh) {
+#pragma unroll
+    for (int k = 0; k < P; k++) {
+        const int u = threadIdx.x + 256 * k;
+        const float4 a0 = xr.f[k][0], a1 = xr.f[k][1];
+        float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        if (u >= (K >> 3))
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = 0.0f;
+        uint32_t hi[4], lo[4];
+        const float gs = qk_f32x8_pairs(v, hi, lo);
+        sh.hi[u & 3][u >> 2] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        sh.lo[u & 3][u >> 2] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        ((float *)sh.gs)[u] = gs;
+    }
+}
+
+template <int P>
+__device__ __forceinline__ void read_xwg(const XWg<P> &sh, int lane, XPairs<64, P, false> &xp) {
+#pragma unroll
+    for (int ps = 0; ps < P; ps++) {
+        const int c = 64 * ps + lane;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const uint4 h = sh.hi[w][c], l = sh.lo[w][c];
+            xp.hi[ps][4 * w] = h.x;
+            xp.hi[ps][4 * w + 1] = h.y;
+            xp.hi[ps][4 * w + 2] = h.z;
+            xp.hi[ps][4 * w + 3] = h.w;
+            xp.lo[ps][4 * w] = l.x;
+            xp.lo[ps][4 * w + 1] = l.y;
+            xp.lo[ps][4 * w + 2] = l.z;
+            xp.lo[ps][4 * w + 3] = l.w;
+        }
+        const float4 g = sh.gs[c];
+        xp.xs[ps] = (((0.0f + g.x) + g.y) + g.z) + g.w;
+    }
+}
+
 /* sum over one 32-code chunk of x * (128 + q) */
 template <int LPR, int P, bool XBF16>
 __device__ __forceinline__ float chunk_dot(uint4 q4, const XPairs<LPR, P, XBF16> &xp, int ps) {

@@ -45,10 +45,46 @@ struct HcDownArgs {
 
 #define HD_RW 2 /* down-matrix rows per workgroup */
 
+/*
+ * A wave's chunks (32 floats per lane, 64 P chunks of base, clamped past CPC)
+ * in two steps: loads of 64-byte runs, four lanes to a chunk half, and the
+ * turn through 4 KB of LDS of the wave's own, swizzled so that the eight lanes
+ * of an LDS pass meet distinct banks both ways.  A lane that loads its own
+ * chunk touches a line per lane and load: 6.3 us a token for the down kernel
+ * (hc 4, hidden 2048, rank 320), 5.7 so.
+ */
+template <int P>
+__device__ __forceinline__ void hc_load_runs(const float *base, int CPC, int lane, float4 (&f)[P][8]) {
+#pragma unroll
+    for (int ps = 0; ps < P; ps++)
+#pragma unroll
+        for (int v = 0; v < 8; v++) {
+            const int c = ps * 64 + 16 * (v & 3) + (lane >> 2);
+            f[ps][v] = qk_ld((const float4 *)base + 8 * (c < CPC ? c : 0) + 4 * (v >> 2) + (lane & 3));
+        }
+}
+template <int P>
+__device__ __forceinline__ void hc_turn(const float4 (&f)[P][8], float4 *buf, int lane, float4 (&o)[P][8]) {
+#pragma unroll
+    for (int ps = 0; ps < P; ps++)
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int c = 16 * v + (lane >> 2);
+                buf[4 * c + ((lane & 3) ^ ((c >> 1) & 3))] = f[ps][4 * hf + v];
+            }
+            qk_wave_lds_sync();
+#pragma unroll
+            for (int u = 0; u < 4; u++) o[ps][4 * hf + u] = buf[4 * lane + (u ^ ((lane >> 1) & 3))];
+            qk_wave_lds_sync();
+        }
+}
+
 /* one task of k_hc_down: INJ = one row of the inject matrix, else HD_RW
  * rows of the down matrix */
 template <int P, bool INJ>
-__device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int rb, int nrb) {
+__device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int rb, int nrb, float4 *turn) {
     constexpr int RW = INJ ? 1 : HD_RW; /* rows of this task */
     __shared__ float s_part[2][HC_MAX][HD_RW];
     const int lane = threadIdx.x & 63, h = threadIdx.x >> 6;
@@ -69,6 +105,12 @@ __device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int 
         cok[ps] = cc < CPC;
         gc[ps] = h * CPC + (cok[ps] ? cc : 0);
     }
+    /* x and hc_norm first: they are turned while the weights arrive */
+    float4 *buf = turn + 256 * h;
+    float4 xr[P][8], wn[P][8];
+    auto load_x = [&](int t) { hc_load_runs<P>(a.hyper + (size_t)t * D + (size_t)h * a.d, CPC, lane, xr); };
+    load_x(t0);
+    hc_load_runs<P>(a.norm_w + (size_t)h * a.d, CPC, lane, wn);
     /* weights: q4 rows (codes, scale, bias) or one bf16 row (32 weights a chunk) */
     uint4 wq[RW][P];
     float ws[RW][P], wb[RW][P];
@@ -94,32 +136,19 @@ __device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int 
             }
         }
     }
-    float4 wn[P][8];
-#pragma unroll
-    for (int ps = 0; ps < P; ps++)
-#pragma unroll
-        for (int v = 0; v < 8; v++)
-            wn[ps][v] = qk_ld((const float4 *)(a.norm_w + (size_t)gc[ps] * 32) + v);
     const bool store_normed = !INJ && rb == 0;
 
-    float4 xr[P][8];
-    auto load_x = [&](int t) {
-#pragma unroll
-        for (int ps = 0; ps < P; ps++)
-#pragma unroll
-            for (int v = 0; v < 8; v++)
-                xr[ps][v] = qk_ld((const float4 *)(a.hyper + (size_t)t * D + (size_t)gc[ps] * 32) + v);
-    };
-    load_x(t0);
     for (int j = 0; j < m; j++) {
         const int t = t0 + j;
         float xv[P][32];
         float ss = 0.0f;
+        float4 xc[P][8];
+        hc_turn<P>(xr, buf, lane, xc);
 #pragma unroll
         for (int ps = 0; ps < P; ps++)
 #pragma unroll
             for (int v = 0; v < 8; v++) {
-                const float4 f = xr[ps][v];
+                const float4 f = xc[ps][v];
                 xv[ps][4 * v] = cok[ps] ? f.x : 0.0f;
                 xv[ps][4 * v + 1] = cok[ps] ? f.y : 0.0f;
                 xv[ps][4 * v + 2] = cok[ps] ? f.z : 0.0f;
@@ -131,6 +160,7 @@ __device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int 
 #pragma unroll
             for (int i = 0; i < 32; i++) ss = fmaf(xv[ps][i], xv[ps][i], ss);
         ss = qk_group_sum<64>(ss);
+        if (j == 0) hc_turn<P>(wn, buf, lane, wn);
         const float r = 1.0f / sqrtf(ss / (float)a.d + a.eps);
         XPairs<64, P, false> xp;
 #pragma unroll
@@ -205,11 +235,12 @@ __device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int 
  */
 template <int P>
 __global__ __launch_bounds__(64 * HC_MAX) void k_hc_down(HcDownArgs a) {
+    extern __shared__ float4 hc_turn_buf[]; /* 4 KB a wave */
     const int nrb = (a.R + HD_RW - 1) / HD_RW;
     const int nblk = nrb + (a.inject_w ? a.hc : 0);
     const int tblk = blockIdx.x / nblk, rb = blockIdx.x - tblk * nblk;
-    if (rb >= nrb) hc_down_body<P, true>(a, tblk, rb, nrb);
-    else hc_down_body<P, false>(a, tblk, rb, nrb);
+    if (rb >= nrb) hc_down_body<P, true>(a, tblk, rb, nrb, hc_turn_buf);
+    else hc_down_body<P, false>(a, tblk, rb, nrb, hc_turn_buf);
 }
 
 /* ------------------------------------------------------- up + mean mix */
@@ -366,7 +397,7 @@ extern "C" int qk_launch_hc_down(const float *hyper, const float *norm_w, const 
     HcDownArgs a{hyper, norm_w, q, s, b, inject_w, normed, w, inject, hc, d, R, n, tb, eps};
     const dim3 grid((unsigned)(((n + tb - 1) / tb) * nblk)), blk(64 * hc);
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_hc_down<1>, grid, blk, 0, st, a);
+    hipLaunchKernelGGL(k_hc_down<1>, grid, blk, 4096 * hc, st, a);
     return QK_CHECK_LAUNCH();
 }
 
