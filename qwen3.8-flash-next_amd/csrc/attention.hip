@@ -109,19 +109,15 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
                 }
             }
         for (int t = 0; t < a.n; t++) {
-            /* INJ: the token's inject weights and the hyper values of this
-             * wave's rows, loaded with x (clamped addresses) */
-            float iv[INJ ? QK_INJECT_MAX_HC : 1], hv[INJ ? AT_RPW : 1][INJ ? QK_INJECT_MAX_HC : 1];
-            if (INJ && mine) {
-#pragma unroll
-                for (int q = 0; q < QK_INJECT_MAX_HC; q++) {
-                    const int qc = min(q, a.hc - 1);
-                    iv[INJ ? q : 0] = qk_ld(a.inject + (size_t)t * a.hc + qc);
-#pragma unroll
-                    for (int j = 0; j < AT_RPW; j++)
-                        hv[INJ ? j : 0][INJ ? q : 0] =
-                            qk_ld(a.hyper + ((size_t)t * a.hc + qc) * S.ostride + min(rr + j, S.rows - 1));
-                }
+            /* INJ: lane (row, copy) has the copy's inject weight and the
+             * hyper value of the row, loaded with x */
+            const int ir = lane / QK_INJECT_MAX_HC, iq = lane % QK_INJECT_MAX_HC;
+            const bool il = INJ && mine && ir < AT_RPW && iq < a.hc;
+            float iv = 0.0f, hv = 0.0f;
+            float *hp = INJ ? a.hyper + ((size_t)t * a.hc + (il ? iq : 0)) * S.ostride + (il ? rr + ir : 0) : nullptr;
+            if (il) {
+                iv = qk_ld(a.inject + (size_t)t * a.hc + iq);
+                hv = qk_ld(hp);
             }
             store_xwg<P>(xr, a.K, sh);
             qk_lds_barrier();
@@ -132,15 +128,8 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
 #pragma unroll
                 for (int j = 0; j < AT_RPW; j++) {
                     const float v = qk_group_sum<64>(row_part<64, P, false>(wq[j], ws[j], wb[j], xp));
-                    if (lane == 0) {
-                        if (S.out) qk_st(S.out + (size_t)t * S.ostride + rr + j, v);
-                        if (INJ)
-#pragma unroll
-                            for (int q = 0; q < QK_INJECT_MAX_HC; q++)
-                                if (q < a.hc)
-                                    qk_st(a.hyper + ((size_t)t * a.hc + q) * S.ostride + rr + j,
-                                          fmaf(iv[INJ ? q : 0], v, hv[INJ ? j : 0][INJ ? q : 0]));
-                    }
+                    if (lane == 0 && S.out) qk_st(S.out + (size_t)t * S.ostride + rr + j, v);
+                    if (il && ir == j) qk_st(hp, fmaf(iv, v, hv));
                 }
             }
             if (t + 1 < a.n) qk_lds_barrier(); /* sh is rewritten for the next token */

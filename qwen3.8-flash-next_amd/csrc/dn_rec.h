@@ -59,7 +59,7 @@ __device__ __forceinline__ void dn_conv_silu(const DnRecArgs &a, int t, const in
 
 template <int DK>
 struct DnRecSmem {
-    alignas(16) float ch[2 * DK + DN_RB]; /* q, k, v of the block's rows */
+    alignas(16) float ch[2 * DK + DN_RB]; /* q, k, v of the block's rows, read 16 bytes at a time */
     float sc[4];              /* q and k norms, decay, beta */
     float o[DN_RB];           /* the block's outputs of this token */
 };

@@ -154,7 +154,8 @@ __device__ __forceinline__ void convert_xshare(const XShare<NG> &xq, int K, int 
  * and every lane takes its chunks from LDS, with exactly what convert_xraw
  * gives.  A lane that loads its own 32 columns touches a line per lane and
  * load, and each wave converts the row again: the DeltaNet mixer's rows at
- * hidden 2048 (12352 of them, one token) took 9.0 us that way, DN_IN_US so.  hi, lo [w]: unit w of each
+ * hidden 2048 (12352 of them, one token) took 9.0 us that way and its
+ * out_proj 7.6, against 8.2 and 5.5 so.  hi, lo [w]: unit w of each
  * chunk, rows 2 units apart modulo 8 so that the stores of 8 lanes (2 chunks)
  * fall on distinct banks.
  */

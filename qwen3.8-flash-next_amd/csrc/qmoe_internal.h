@@ -264,8 +264,8 @@ typedef struct {
 } qk_proj;
 int qk_launch_proj(const qk_proj *a, void *stream);
 /* the mixers take their matrix kernels from this many tokens on.  DeltaNet's
- * per-token GEMVs cost 9 us a token at hidden 2048: 66 us the mixer at 6
- * tokens, 94 at 9, against 57 and 63.  Attention's whole path (projections,
+ * per-token GEMVs cost 7 us a token at hidden 2048: 45 us the mixer at 5
+ * tokens and on that slope 52 at 6 and 65 at 8, against 46 and 50.  Attention's whole path (projections,
  * indexer rows, attn_mm.hip) has more launches: at 9 tokens 50..71 us on the
  * per-token kernels and 46..86 on these over four shapes, at 16 tokens 59..122
  * against 37..97. */

@@ -138,3 +138,33 @@ def test_hyper_token_counts(torch_dev, hc, d, R, n):
         tg.assert_close(m.cpu().numpy(), ref["mixed"], "mixed")
         tg.assert_close(i.cpu().numpy(), ref["inject"], "inject")
         assert torch.equal(m, m2)
+
+
+# the per-token kernels where x's way through LDS has its edges: one chunk
+# pair, a full pass of 2048 columns, one group past one, two and three passes
+@pytest.mark.parametrize("d,hv,dk,dv", [(64, 2, 32, 32), (2048, 2, 32, 64), (2112, 33, 64, 64), (4160, 33, 32, 128), (8192, 49, 32, 128)])
+def test_deltanet_few_tokens(torch_dev, d, hv, dk, dv):
+    torch, dev = torch_dev
+    td.run_steps(torch, dev, (d, 1, hv, dk, dv, 4), [1, 5, 2], seed=14)
+
+
+@pytest.mark.parametrize("d,h,hd", [(64, 1, 64), (2048, 5, 64), (2112, 33, 64), (4160, 12, 64)])
+def test_attention_few_tokens(torch_dev, d, h, hd):
+    torch, dev = torch_dev
+    ta.run_calls(torch, dev, (d, h, 1, hd, 3, 68, 12, 3, 64, 1.0), [1, 15, 2], seed=15)
+
+
+@pytest.mark.parametrize("hc,d,R", [(8, 64, 64), (1, 2048, 320), (3, 1984, 128), (2, 1088, 64)])
+@pytest.mark.parametrize("n", [1, 2, 15])
+def test_hyper_few_tokens(torch_dev, hc, d, R, n):
+    torch, dev = torch_dev
+    orc = tg.orc
+    hp = orc.Hyper(hc, d, R, seed=22, layer=1, norm_std=0.1)
+    hyper = orc.gen_hyper(n, hc, d, seed=n) * 2.0
+    with tg.load_pkg().GatedResidualContext(d, hc, R, n_slots=1, max_tokens=n) as gr:
+        gr.upload_slot(0, hp.arrays())
+        m, i = gr.mix(0, torch.from_numpy(hyper).to(dev))
+        torch.cuda.synchronize()
+        ref = hp.mix(hyper)
+        tg.assert_close(m.cpu().numpy(), ref["mixed"], "mixed")
+        tg.assert_close(i.cpu().numpy(), ref["inject"], "inject")
