@@ -17,12 +17,13 @@
  * is a K = G product done once per tile on MFMA: b is exact in bf16 and
  * X_g = P_g / -128 is split into bf16 hi + lo.  Weights are never rounded.
  *
- * Tiles.  A task is (segment, chunk of up to MM_BM rows); the grid is tasks
+ * Tiles.  A task is (segment, chunk of up to MM_BM or MM_NBM rows); the grid is tasks
  * x column tiles.  The workgroup's 4 waves each own CT = 4 column tiles of
  * 16 (gate/up: 32 columns of Wg and the same 32 of Wu, so h = silu(g)*u is
  * formed in registers; down: 64 columns of Wd) and every 16-row tile of
- * the chunk.  Batches of at most MM_NARROW_N tokens use CT = 2 and 64-row
- * chunks: twice the workgroups, each with less LDS and fewer registers.  Per group the chunk's activation rows are staged in LDS
+ * the chunk.  The narrow kernels (mm_narrow) have CT = 2 and 64-row
+ * chunks: twice the workgroups, each with less LDS and fewer registers.
+ * Per group the chunk's activation rows are staged in LDS
  * (double buffered, XOR-swizzled 16-byte chunks), the code words come from
  * a register ring MM_WD groups ahead, and the scales of the whole tile sit
  * in LDS.  The kernel body is specialised on the number of 16-row tiles.
@@ -379,8 +380,7 @@ __device__ __forceinline__ void mm_body(const MmArgs &a, MmSmem<TERMS, BMT, CT, 
     }
 }
 
-/* BMT * 16 must hold every chunk: BMT = MM_MT, or any BMT when the host
- * knows that no segment has more rows (a segment has at most n rows) */
+/* BMT * 16 is the row count of the task list's chunks */
 /* bf16 gate/up at full tiles stages two groups per barrier (the LDS of two
  * workgroups per CU still fits) */
 template <int TERMS, int BMT>
@@ -459,8 +459,8 @@ __global__ __launch_bounds__(256) void k_pack_rows(const void *x, size_t nchunks
 }
 
 /*
- * Down projection of batches of at most MM_NARROW_N tokens, K = 512, on the
- * dispatch's 16-row task list.  The 64-row kernel waits, every group, on
+ * Down projection of the narrow calls, K = 512, on the dispatch's 16-row
+ * task list.  The 64-row kernel waits, every group, on
  * the chain activation load -> LDS store -> barrier -> LDS read (~1 us per
  * group at 1..16 rows).  Here the code words of the whole K slice of the
  * tile (8 groups, 16 bytes per lane and column tile) are loaded into
@@ -633,8 +633,8 @@ __global__ __launch_bounds__(256, 2) void k_mm_down16(MmArgs a) {
 
 /* the task list as its own launch (mm_tasks.h) */
 __global__ __launch_bounds__(1024) void k_mm_tasks(const int32_t *segtab, int n, int k, int E,
-                                                   int min_m, int32_t *tasks, int32_t *small) {
-    mm_tasks_block(segtab, n, k, E, min_m, tasks, small);
+                                                   int min_m, qk_mm_lists lists) {
+    mm_tasks_block(segtab, n, k, E, min_m, lists);
 }
 
 /* Up to MM_NARROW_N tokens the kernels hold 64-row chunks and give each wave
@@ -646,24 +646,25 @@ __global__ __launch_bounds__(1024) void k_mm_tasks(const int32_t *segtab, int n,
  * f32 333 tokens 437 / 388, 512 tokens 452 / 407, 768 tokens 475 / 453;
  * bf16 96 tokens 292 / 279, 333 tokens 389 / 356, 768 tokens 414 / 410,
  * 1024 tokens 438 / 471; with Zipf-skewed routing 128 tokens 138 / 108, 333
- * tokens 181 / 185, 512 tokens 222 / 223, 768 tokens 254 / 286. */
+ * tokens 181 / 185, 512 tokens 222 / 223, 768 tokens 254 / 286.  The results
+ * are the same bits either way, so a layer call short of memory takes the wide
+ * kernels, whose lists are shorter (lean). */
+#define MM_NARROW_N 512
+static bool mm_narrow(qk_shape s, int n) { return n <= MM_NBM || (!s.lean && n <= MM_NARROW_N); }
 
-static int mm_launch(MmArgs &a, bool down, int terms, int max_tasks, hipStream_t st,
-                     const int32_t *list16 = nullptr, int max16 = 0) {
-    const bool narrow = a.n <= MM_NARROW_N;
-    const int ct = narrow ? 2 : 4;
+static int mm_launch(MmArgs &a, bool down, int terms, const qk_mm_lists &l, hipStream_t st) {
+    const bool narrow = l.bm == MM_NBM, d16 = down && l.list16;
+    const int ct = narrow || d16 ? 2 : 4;
     a.ntile = a.N / (down ? 64 * ct : 32 * ct);
-    if (narrow && down && list16 && a.K == 64 * MMD_G) {
-        a.tasks = list16;
-        const long long wgs16 = (long long)(max16 + 7) / 8 * 8 * a.ntile;
-        if (wgs16 <= 0) return 0;
-        hipLaunchKernelGGL(k_mm_down16, dim3((unsigned)wgs16), dim3(256), 0, st, a);
-        return QK_CHECK_LAUNCH();
-    }
-    /* every (task, column tile) once: 8 * ceil(max_tasks / 8) tasks */
-    const long long wgs = (long long)(max_tasks + 7) / 8 * 8 * a.ntile;
+    /* every (task, column tile) once: 8 * ceil(tasks / 8) tasks */
+    const long long wgs = (long long)((d16 ? l.max16 : l.max) + 7) / 8 * 8 * a.ntile;
     if (wgs <= 0) return 0;
     const dim3 grid((unsigned)wgs), blk(256);
+    a.tasks = d16 ? l.list16 : l.tasks;
+    if (d16) {
+        hipLaunchKernelGGL(k_mm_down16, grid, blk, 0, st, a);
+        return QK_CHECK_LAUNCH();
+    }
 #define MM_L(D, T, B, C) hipLaunchKernelGGL((k_mm<D, T, B, C>), grid, blk, 0, st, a)
     /* down: always the two planes formed from f32 h */
     if (narrow) {
@@ -677,35 +678,46 @@ static int mm_launch(MmArgs &a, bool down, int terms, int max_tasks, hipStream_t
     return QK_CHECK_LAUNCH();
 }
 
-extern "C" int qk_mfma_max_tasks(qk_shape s, int n) {
-    /* routed segments: at most min(E, n*k), plus their extra chunks; shared: ceil(n/BM) */
+/* entries of the list of bm-row chunks: the routed segments (at most min(E,
+ * n*k)) and their further chunks, and the shared expert's.  A caller's own
+ * segment table may hold segments of more than n rows; the layer's dispatch,
+ * which lean is for, does not */
+static int mm_max_chunks(qk_shape s, int n, int bm) {
     const long long nk = (long long)n * s.k;
-    const int bm = mm_chunk_rows(n);
-    const long long t = (nk < s.E ? nk : s.E) + nk / bm + (n + bm - 1) / bm + 1;
-    return (int)t;
+    return (int)((nk < s.E ? nk : s.E) + (s.lean && n <= bm ? 0 : nk / bm) + (n + bm - 1) / bm + 1);
 }
 
-/* entries of the 16-row list (0 above MM_NARROW_N tokens) */
-static int mm_max_tasks16(qk_shape s, int n) {
-    if (n > MM_NARROW_N) return 0;
-    const long long nk = (long long)n * s.k;
-    return (int)((nk < s.E ? nk : s.E) + nk / MM_BM16 + (n + MM_BM16 - 1) / MM_BM16 + 1);
+/* past the small list's 2 + E ints, rounded up to 16 bytes for the int4
+ * entries of the list behind it */
+static size_t mm_small_ints(qk_shape s) { return ((size_t)s.E + 2 + 3) & ~(size_t)3; }
+
+extern "C" qk_mm_lists qk_mfma_lists(qk_shape s, int n, int32_t *tasks) {
+    const bool narrow = mm_narrow(s, n), d16 = narrow && s.I == 64 * MMD_G;
+    qk_mm_lists l = {};
+    l.bm = narrow ? MM_NBM : MM_BM;
+    l.max = mm_max_chunks(s, n, l.bm);
+    l.max16 = d16 ? mm_max_chunks(s, n, MM_BM16) : 0;
+    if (!tasks) return l;
+    l.tasks = tasks;
+    l.small = tasks + MM_TASK_HDR + 4 * (size_t)l.max;
+    if (d16) l.list16 = l.small + mm_small_ints(s);
+    return l;
 }
 
-/* the lists of any call of up to n tokens: a call of at most MM_NARROW_N
- * tokens has a second list, so the largest call is not always the largest */
 extern "C" size_t qk_mfma_task_bytes(qk_shape s, int n) {
-    size_t most = 0;
-    for (int m = n;; m = MM_NARROW_N) {
-        const size_t t16 = m <= MM_NARROW_N ? (size_t)MM_TASK_HDR + 4 * (size_t)mm_max_tasks16(s, m) : 0;
-        const size_t b = ((size_t)MM_TASK_HDR + 4 * (size_t)qk_mfma_max_tasks(s, m) + (size_t)MM_SMALL16(s.E) + t16) * 4;
-        most = b > most ? b : most;
-        if (m <= MM_NARROW_N) return most;
-    }
+    const qk_mm_lists l = qk_mfma_lists(s, n, nullptr);
+    return (MM_TASK_HDR + 4 * (size_t)l.max + mm_small_ints(s) + (l.max16 ? MM_TASK_HDR + 4 * (size_t)l.max16 : 0)) * 4;
 }
 
-extern "C" int32_t *qk_mfma_small_list(qk_shape s, int n, int32_t *tasks) {
-    return tasks + MM_TASK_HDR + 4 * (size_t)qk_mfma_max_tasks(s, n);
+/* the narrow lists are the larger ones, so the largest call is not always the
+ * one with the most entries */
+extern "C" size_t qk_mfma_task_bytes_upto(qk_shape s, int n) {
+    size_t most = qk_mfma_task_bytes(s, n);
+    for (int m = n < MM_NARROW_N ? n : MM_NARROW_N; m > 0; m--) {
+        const size_t b = qk_mfma_task_bytes(s, m);
+        most = b > most ? b : most;
+    }
+    return most;
 }
 
 /* gate/up: K = H, N = I in tiles of 128 columns; down: K = I, N = H in
@@ -724,7 +736,7 @@ extern "C" int qk_mfma_down_ok(qk_shape s) {
 extern "C" int qk_launch_mfma_tasks(qk_shape s, int n, const int32_t *segtab, int min_m,
                                     int32_t *tasks, void *stream) {
     hipLaunchKernelGGL(k_mm_tasks, dim3(1), dim3(1024), 0, (hipStream_t)stream, segtab, n, s.k, s.E,
-                       min_m, tasks, qk_mfma_small_list(s, n, tasks));
+                       min_m, qk_mfma_lists(s, n, tasks));
     return QK_CHECK_LAUNCH();
 }
 
@@ -756,12 +768,11 @@ extern "C" int qk_launch_gateup_mfma(const qmoe_layer_weights *W, qk_shape s, co
     a.af = nullptr;
     a.out = h;
     a.perm = perm;
-    a.tasks = tasks;
     a.K = s.H;
     a.N = s.I;
     a.n = n;
     a.k = s.k;
-    return mm_launch(a, false, xlo ? 2 : 1, qk_mfma_max_tasks(s, n), (hipStream_t)stream);
+    return mm_launch(a, false, xlo ? 2 : 1, qk_mfma_lists(s, n, (int32_t *)tasks), (hipStream_t)stream);
 }
 
 extern "C" int qk_launch_down_mfma(const qmoe_layer_weights *W, qk_shape s, const float *h, int n,
@@ -780,12 +791,9 @@ extern "C" int qk_launch_down_mfma(const qmoe_layer_weights *W, qk_shape s, cons
     a.af = h;
     a.out = y;
     a.perm = nullptr;
-    a.tasks = tasks;
     a.K = s.I;
     a.N = s.H;
     a.n = n;
     a.k = s.k;
-    return mm_launch(a, true, 2, qk_mfma_max_tasks(s, n), (hipStream_t)stream,
-                     n <= MM_NARROW_N ? qk_mfma_small_list(s, n, (int32_t *)tasks) + MM_SMALL16(s.E) : nullptr,
-                     mm_max_tasks16(s, n));
+    return mm_launch(a, true, 2, qk_mfma_lists(s, n, (int32_t *)tasks), (hipStream_t)stream);
 }

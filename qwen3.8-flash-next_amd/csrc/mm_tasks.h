@@ -13,10 +13,8 @@
 #define MM_BM (16 * MM_MT)   /* rows per chunk */
 #define MM_TASK_HDR 4        /* int32 header before the int4 task entries */
 
-#define MM_NARROW_N 512      /* batches up to this many tokens: 64-row chunks, and a 16-row list too */
-#define MM_BM16 16
-#define MM_NBM 64            /* rows per chunk up to MM_NARROW_N tokens */
-static __host__ __device__ inline int mm_chunk_rows(int n) { return n <= MM_NARROW_N ? MM_NBM : MM_BM; }
+#define MM_NBM 64            /* rows per chunk of the narrow kernels */
+#define MM_BM16 16           /* and of the 16-row list */
 
 /* a segment-table word: from LDS (the table this workgroup just built,
  * mirrored there) or from global memory */
@@ -113,17 +111,11 @@ static __device__ void mm_tasks_list(const int32_t *segtab, int n, int k, int E,
     }
 }
 
-/* The task lists of a dispatch: chunks of MM_BM rows at `tasks` with the
- * small-segment list at `small`, and, up to MM_NARROW_N tokens, chunks of
- * MM_BM16 rows at small + MM_SMALL16(E) (the down projection's list there:
- * past the small list's 2 + E ints, rounded up to 16 bytes for its int4
- * entries). */
-#define MM_SMALL16(E) ((2 + (E) + 3) & ~3)
+/* the task lists of a dispatch (qk_mfma_lists) */
 template <bool LDS = false>
-static __device__ void mm_tasks_block(const int32_t *segtab, int n, int k, int E, int min_m, int32_t *tasks,
-                               int32_t *small) {
-    mm_tasks_list<LDS>(segtab, n, k, E, min_m, mm_chunk_rows(n), tasks, small);
-    if (n <= MM_NARROW_N) mm_tasks_list<LDS>(segtab, n, k, E, min_m, MM_BM16, small + MM_SMALL16(E), nullptr);
+static __device__ void mm_tasks_block(const int32_t *segtab, int n, int k, int E, int min_m, const qk_mm_lists &l) {
+    mm_tasks_list<LDS>(segtab, n, k, E, min_m, l.bm, l.tasks, l.small);
+    if (l.list16) mm_tasks_list<LDS>(segtab, n, k, E, min_m, MM_BM16, l.list16, nullptr);
 }
 
 #endif

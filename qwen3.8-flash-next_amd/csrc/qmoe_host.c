@@ -172,13 +172,13 @@ static int check_config(const qmoe_config *c, qmoe_err *err) {
 /* the layer scratch for n tokens, carved out of one block: region offsets
  * (QH_SC_COUNT of them) and the total */
 enum { QH_SC_COUNT = 17 };
-static size_t scratch_plan(qk_shape s, size_t n, size_t offs[QH_SC_COUNT]) {
+static size_t scratch_plan(qk_shape s, size_t n, size_t task_bytes, size_t offs[QH_SC_COUNT]) {
     const size_t E = (size_t)s.E, k = (size_t)s.k, H = (size_t)s.H, I = (size_t)s.I;
     const size_t nw = (n + 31) / 32, rows = n * k + n;
     const size_t plane = n * H > rows * I ? n * H : rows * I;
     const size_t sz[QH_SC_COUNT] = {n * (E + 1) * 4, n * k * 4, n * k * 4, n * 4, (E + 1) * 4, n * k * 4,
                                     n * k * 4, E * nw * 4, E * nw * 4, n * H * 4, rows * I * 4,
-                                    rows * H * 4, (3 * E + 1) * 4, qk_mfma_task_bytes(s, (int)n),
+                                    rows * H * 4, (3 * E + 1) * 4, task_bytes,
                                     plane * 2, plane * 2, plane / 64 * 4};
     size_t total = 0;
     for (int i = 0; i < QH_SC_COUNT; i++) {
@@ -250,7 +250,8 @@ int qmoe_create(qmoe_ctx **out, const qmoe_config *cfg, qmoe_err *err) {
     }
     /* scratch */
     size_t offs[QH_SC_COUNT];
-    const size_t total = scratch_plan(c->shape, (size_t)cfg->max_tokens, offs);
+    const size_t total = scratch_plan(c->shape, (size_t)cfg->max_tokens,
+                                      qk_mfma_task_bytes_upto(c->shape, cfg->max_tokens), offs);
     c->scratch_bytes = total;
     if (hip_fail(err, (int)hipMalloc(&c->scratch_mem, total), "hipMalloc(scratch)")) {
         free(c->layers);
@@ -826,7 +827,7 @@ static int run_gateup(const stage_env *e, const qmoe_layer_weights *W, const voi
     if (mm && gemv && fork(e, stream, err)) return -1;
     if (gemv) {
         rc = qk_launch_gateup(W, s, x, xbf, n, perm, segtab, mm ? min_m : 0,
-                              mm ? qk_mfma_small_list(s, n, sc->tasks) : NULL, h, gs);
+                              mm ? qk_mfma_lists(s, n, sc->tasks).small : NULL, h, gs);
         if (hip_fail(err, rc, "gateup")) return -1;
     }
     if (mm) {
@@ -856,7 +857,7 @@ static int run_down(const stage_env *e, const qmoe_layer_weights *W, const float
     if (mm && gemv && fork(e, stream, err)) return -1;
     if (gemv) {
         rc = qk_launch_down(W, s, h, n, segtab, mm ? min_m : 0,
-                            mm ? qk_mfma_small_list(s, n, sc->tasks) : NULL, y, gs);
+                            mm ? qk_mfma_lists(s, n, sc->tasks).small : NULL, y, gs);
         if (hip_fail(err, rc, "down")) return -1;
     }
     if (mm) {
@@ -1124,10 +1125,14 @@ int qmoe_layer_forward_noalloc(const qmoe_config *cfg, const qmoe_layer_weights 
     if (n == 0) return 0;
     NEED(x, "x");
     NEED(out, "out");
-    const qk_shape s = {cfg->hidden, cfg->n_experts, cfg->top_k, cfg->moe_inter, cfg->rms_eps,
-                        cfg->group_size == 32};
+    qk_shape s = {cfg->hidden, cfg->n_experts, cfg->top_k, cfg->moe_inter, cfg->rms_eps,
+                  cfg->group_size == 32, 0};
     size_t offs[QH_SC_COUNT];
-    const size_t bytes = scratch_plan(s, (size_t)n, offs);
+    size_t bytes = scratch_plan(s, (size_t)n, qk_mfma_task_bytes(s, n), offs);
+    if (bytes > QK_NOALLOC_SCRATCH_BYTES) {
+        s.lean = 1;
+        bytes = scratch_plan(s, (size_t)n, qk_mfma_task_bytes(s, n), offs);
+    }
     if (bytes > QK_NOALLOC_SCRATCH_BYTES) {
         set_err(err, "n = %d needs %zu bytes of scratch at this shape; the static scratch holds %zu "
                      "(call with fewer tokens)", n, bytes, (size_t)QK_NOALLOC_SCRATCH_BYTES);

@@ -28,6 +28,7 @@ typedef struct {
     int H, E, k, I;
     float eps;
     int g32; /* 1: the experts' q4 groups are 32 columns (GEMV kernels only), 0: 64 */
+    int lean; /* 1: the shortest task lists of a layer call, whatever their speed */
 } qk_shape;
 
 /* device scratch carved out of one allocation by the host */
@@ -159,11 +160,18 @@ int qk_launch_gateup(const qmoe_layer_weights *W, qk_shape s, const void *x, int
 int qk_launch_down(const qmoe_layer_weights *W, qk_shape s, const float *h, int n,
                    const int32_t *segtab, int max_m, const int32_t *seglist, float *y,
                    void *stream);
-int qk_mfma_max_tasks(qk_shape s, int n);
-size_t qk_mfma_task_bytes(qk_shape s, int n);
-/* the list of segments below min_m rows that the task kernel writes beside
- * the tasks (for the GEMV kernels): [count, segment...] */
-int32_t *qk_mfma_small_list(qk_shape s, int n, int32_t *tasks);
+/* the task lists of a call of n tokens, in its `tasks` scratch: how its
+ * segments are cut and where each list lies */
+typedef struct {
+    int bm;          /* rows per chunk of the list at `tasks` */
+    int max, max16;  /* the most entries of the lists at `tasks` and list16 */
+    int32_t *tasks;
+    int32_t *small;  /* segments below min_m rows, for the GEMV kernels: [count, segment...] */
+    int32_t *list16; /* chunks of 16 rows for the down projection (NULL: none) */
+} qk_mm_lists;
+qk_mm_lists qk_mfma_lists(qk_shape s, int n, int32_t *tasks);
+size_t qk_mfma_task_bytes(qk_shape s, int n); /* of a call of n tokens */
+size_t qk_mfma_task_bytes_upto(qk_shape s, int n); /* of any call of up to n tokens */
 /* shapes the MFMA kernels take (x_bf16: gate/up activations are bf16) */
 int qk_mfma_gateup_ok(qk_shape s, int x_bf16);
 int qk_mfma_down_ok(qk_shape s);

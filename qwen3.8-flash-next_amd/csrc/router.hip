@@ -592,8 +592,8 @@ __device__ void dispatch_block(const int32_t *s_idx, int n, int k, int E, int32_
 struct SmallDispArgs {
     TopkArgs tk;
     int32_t *offsets, *perm, *pos, *segtab;
-    int min_m;            /* MFMA task list from the table, when tasks is set */
-    int32_t *tasks, *small;
+    int min_m;            /* MFMA task lists from the table, when lists.tasks is set */
+    qk_mm_lists lists;
 };
 
 /*
@@ -645,9 +645,9 @@ __global__ __launch_bounds__(1024) void k_topk_dispatch_small(SmallDispArgs a) {
     for (int t = wave; t < a.tk.n; t += 16) topk_token<PL>(a.tk, t, lane, s_idx);
     __syncthreads();
     dispatch_block<1024>(s_idx, a.tk.n, a.tk.k, a.tk.E, a.offsets, a.perm, a.pos, a.segtab, s_seg);
-    if (a.tasks) {
+    if (a.lists.tasks) {
         __syncthreads(); /* the segment table, written by this workgroup */
-        mm_tasks_block<true>(s_seg, a.tk.n, a.tk.k, a.tk.E, a.min_m, a.tasks, a.small);
+        mm_tasks_block<true>(s_seg, a.tk.n, a.tk.k, a.tk.E, a.min_m, a.lists);
     }
 }
 
@@ -656,15 +656,15 @@ __global__ __launch_bounds__(1024) void k_topk_dispatch_small(SmallDispArgs a) {
 __global__ __launch_bounds__(1024) void k_dispatch_small(const int32_t *idx, int n, int k, int E,
                                                          int32_t *offsets, int32_t *perm,
                                                          int32_t *pos, int32_t *segtab, int min_m,
-                                                         int32_t *tasks, int32_t *small) {
+                                                         qk_mm_lists lists) {
     __shared__ int32_t s_idx[QK_SMALL_NK];
     __shared__ int32_t s_seg[1 + 3 * QK_MAX_EXPERTS]; /* the segment table, mirrored */
     for (int f = threadIdx.x; f < n * k; f += 1024) s_idx[f] = qk_ld(idx + f);
     __syncthreads();
     dispatch_block<1024>(s_idx, n, k, E, offsets, perm, pos, segtab, s_seg);
-    if (tasks) {
+    if (lists.tasks) {
         __syncthreads();
-        mm_tasks_block<true>(s_seg, n, k, E, min_m, tasks, small);
+        mm_tasks_block<true>(s_seg, n, k, E, min_m, lists);
     }
 }
 
@@ -681,7 +681,7 @@ extern "C" int qk_launch_topk_dispatch_small(qk_shape s, int n, const float *log
     if (n > QK_SMALL_N || n * s.k > QK_SMALL_NK) return (int)hipErrorInvalidValue;
     if (n == 1 && tasks) return (int)hipErrorInvalidValue;
     SmallDispArgs a{{logits, logits_out, idx, w, sg, s.E, s.k, n}, offsets, perm, pos, segtab,
-                    min_m, tasks, tasks ? qk_mfma_small_list(s, n, tasks) : nullptr};
+                    min_m, qk_mfma_lists(s, n, tasks)};
     hipStream_t st = (hipStream_t)stream;
     if (n == 1) {
         TK_DISPATCH(k_topk_dispatch_one, topk_pl(s.E), dim3(1), dim3(64), a);
@@ -692,8 +692,7 @@ extern "C" int qk_launch_topk_dispatch_small(qk_shape s, int n, const float *log
         if (!offsets) return (int)hipErrorInvalidValue;
         TK_DISPATCH(k_topk, topk_pl(s.E), dim3((n + 3) / 4), dim3(256), a.tk);
         hipLaunchKernelGGL(k_dispatch_small, dim3(1), dim3(1024), 0, st, (const int32_t *)idx, n, s.k,
-                           s.E, offsets, perm, pos, segtab, min_m, tasks,
-                           tasks ? qk_mfma_small_list(s, n, tasks) : nullptr);
+                           s.E, offsets, perm, pos, segtab, min_m, a.lists);
     }
     return QK_CHECK_LAUNCH();
 }
@@ -742,7 +741,7 @@ __global__ __launch_bounds__(1024) void k_word_prefix(const uint32_t *bits, int3
  * expert ids) are set to -1 */
 __global__ __launch_bounds__(1024) void k_count_offsets(int E, int32_t *offsets, int32_t *segtab,
                                                         int32_t *perm, int nk, int n, int k,
-                                                        int min_m, int32_t *tasks, int32_t *small) {
+                                                        int min_m, qk_mm_lists lists) {
     __shared__ int s_scan[16];
     __shared__ int32_t s_seg[1 + 3 * QK_MAX_EXPERTS]; /* the segment table, mirrored */
     const int tid = threadIdx.x;
@@ -750,9 +749,9 @@ __global__ __launch_bounds__(1024) void k_count_offsets(int E, int32_t *offsets,
     __syncthreads();
     const int total = counts_to_offsets<1024>(cnt, E, s_scan, offsets, segtab, nullptr, s_seg);
     for (int i = total + tid; i < nk; i += 1024) perm[i] = -1;
-    if (tasks) {
+    if (lists.tasks) {
         __syncthreads(); /* the segment table, written by this workgroup */
-        mm_tasks_block<true>(s_seg, n, k, E, min_m, tasks, small);
+        mm_tasks_block<true>(s_seg, n, k, E, min_m, lists);
     }
 }
 
@@ -789,7 +788,7 @@ extern "C" int qk_launch_dispatch(qk_shape s, int n, const int32_t *idx, int32_t
     hipLaunchKernelGGL(k_word_prefix, dim3((s.E + 15) / 16), dim3(1024), 0, st, (const uint32_t *)bits,
                        wprefix, s.E, NW, offsets);
     hipLaunchKernelGGL(k_count_offsets, dim3(1), dim3(1024), 0, st, s.E, offsets, segtab, perm, nk, n,
-                       s.k, min_m, tasks, tasks ? qk_mfma_small_list(s, n, tasks) : nullptr);
+                       s.k, min_m, qk_mfma_lists(s, n, tasks));
     hipLaunchKernelGGL(k_scatter, dim3((nk + 255) / 256), dim3(256), 0, st, idx, n, s.k, s.E, NW,
                        (const uint32_t *)bits, (const int32_t *)wprefix, (const int32_t *)offsets,
                        perm, pos);

@@ -102,6 +102,31 @@ def test_noalloc_matches_layer_forward(torch_dev, shape, with_norm, calls):
             assert torch.equal(again, ref)
 
 
+# the last n that the static block holds: with I 320 the lists of the call
+# alone (1927 would do for the lists of every smaller call), with I 512 lists
+# that only fit as 96-row chunks, and a call below 64 tokens
+@pytest.mark.parametrize("shape,n", [((512, 60, 6, 320), 1928), ((1024, 32, 16, 512), 465),
+                                     ((2048, 64, 15, 512), 326), ((8192, 64, 32, 512), 53)])
+def test_noalloc_last_count(torch_dev, shape, n):
+    torch, dev = torch_dev
+    pkg = load_pkg()
+    H, E, k, I = shape
+    say(f"case: no-alloc layer {shape}, {n} tokens")
+    with pkg.MoeContext(H, E, k, I, n_layers=1, max_tokens=n) as ctx:
+        ctx.synth_layer(0, 7)
+        w = device_weights(pkg, ctx)
+        cfg = pkg.QmoeConfig(H, E, k, I, 64, 1, 2 * n, 1e-6)
+        x = torch.randn((n, H), generator=torch.Generator(device="cpu").manual_seed(5)).to(dev)
+        ref = run_ref(pkg, ctx, x, pkg.F32, 0)
+        got = run_noalloc(pkg, cfg, w, x, pkg.F32, 0)
+        torch.cuda.synchronize()
+        assert torch.isfinite(ref).all() and torch.equal(ref, got)
+        err = pkg.QmoeErr()
+        assert pkg.lib().qmoe_layer_forward_noalloc(ctypes.byref(cfg), ctypes.byref(w), x.data_ptr(), pkg.F32, n + 1,
+                                                    ref.data_ptr(), 0, None, ctypes.byref(err)) == -1
+        assert b"static scratch holds" in err.msg
+
+
 def test_noalloc_errors(torch_dev):
     torch, dev = torch_dev
     pkg = load_pkg()
