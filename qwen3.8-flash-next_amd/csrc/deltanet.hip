@@ -99,6 +99,14 @@ __global__ __launch_bounds__(256) void k_dn_in(DnInArgs a) {
         if (r0 < R2) {
 #pragma unroll
             for (int j = 0; j < DN_RPW; j++) {
+                /* the codes stay codes: widened before the token loop, four rows
+                 * of P = 2 took 288 registers, one wave a SIMD, and at P = 4
+                 * they spilled.  One token of the mixer, us: hidden 4096, heads
+                 * 32/32 40.5 -> 29.2, hidden 8192, heads 8/32 96 -> 89 */
+                if (P >= 2)
+#pragma unroll
+                    for (int ps = 0; ps < P; ps++)
+                        asm volatile("" : "+v"(wq[j][ps].x), "+v"(wq[j][ps].y), "+v"(wq[j][ps].z), "+v"(wq[j][ps].w));
                 const float v = qk_group_sum<64>(row_part<64, P, false>(wq[j], ws[j], wb[j], xp));
                 const int r = r0 + j;
                 if (lane == 0 && r < R2) {
