@@ -51,8 +51,13 @@ struct HcDownArgs {
  * turn through 4 KB of LDS of the wave's own, swizzled so that the eight lanes
  * of an LDS pass meet distinct banks both ways.  A lane that loads its own
  * chunk touches a line per lane and load: 6.3 us a token for the down kernel
- * (hc 4, hidden 2048, rank 320), 5.7 so.
+ * (hc 4, hidden 2048, rank 320), 5.7 so.  Below HD_TURN_D columns a copy has
+ * few lines and the turn costs more than they do.  The mix of 8 tokens in us,
+ * own chunks against turned ones, hc 4: rank 320, hidden 256 13.0 / 15.3, 512
+ * 14.7 / 16.4, 1024 18.1 / 18.3, 1536 21.4 / 20.2, 2048 25.3 / 22.4; rank
+ * 1024, hidden 1024 34.7 / 36.6, 1280 38.4 / 39.1, 1536 43.6 / 42.9.
  */
+#define HD_TURN_D 1536
 template <int P>
 __device__ __forceinline__ void hc_load_runs(const float *base, int CPC, int lane, float4 (&f)[P][8]) {
 #pragma unroll
@@ -61,6 +66,17 @@ __device__ __forceinline__ void hc_load_runs(const float *base, int CPC, int lan
         for (int v = 0; v < 8; v++) {
             const int c = ps * 64 + 16 * (v & 3) + (lane >> 2);
             f[ps][v] = qk_ld((const float4 *)base + 8 * (c < CPC ? c : 0) + 4 * (v >> 2) + (lane & 3));
+        }
+}
+/* the same chunks, each lane its own: what hc_load_runs and hc_turn give */
+template <int P>
+__device__ __forceinline__ void hc_load_own(const float *base, int CPC, int lane, float4 (&f)[P][8]) {
+#pragma unroll
+    for (int ps = 0; ps < P; ps++)
+#pragma unroll
+        for (int v = 0; v < 8; v++) {
+            const int c = ps * 64 + lane;
+            f[ps][v] = qk_ld((const float4 *)base + 8 * (c < CPC ? c : 0) + v);
         }
 }
 template <int P>
@@ -83,7 +99,7 @@ __device__ __forceinline__ void hc_turn(const float4 (&f)[P][8], float4 *buf, in
 
 /* one task of k_hc_down: INJ = one row of the inject matrix, else HD_RW
  * rows of the down matrix */
-template <int P, bool INJ>
+template <int P, bool INJ, bool TURN>
 __device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int rb, int nrb, float4 *turn) {
     constexpr int RW = INJ ? 1 : HD_RW; /* rows of this task */
     __shared__ float s_part[2][HC_MAX][HD_RW];
@@ -105,12 +121,19 @@ __device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int 
         cok[ps] = cc < CPC;
         gc[ps] = h * CPC + (cok[ps] ? cc : 0);
     }
-    /* x and hc_norm first: they are turned while the weights arrive */
+    /* TURN: x and hc_norm first, they are turned while the weights arrive */
     float4 *buf = turn + 256 * h;
     float4 xr[P][8], wn[P][8];
-    auto load_x = [&](int t) { hc_load_runs<P>(a.hyper + (size_t)t * D + (size_t)h * a.d, CPC, lane, xr); };
-    load_x(t0);
-    hc_load_runs<P>(a.norm_w + (size_t)h * a.d, CPC, lane, wn);
+    auto load = [&](const float *base, float4 (&f)[P][8]) {
+        if (TURN) hc_load_runs<P>(base, CPC, lane, f);
+        else hc_load_own<P>(base, CPC, lane, f);
+    };
+    auto load_x = [&](int t) { load(a.hyper + (size_t)t * D + (size_t)h * a.d, xr); };
+    auto load_wn = [&]() { load(a.norm_w + (size_t)h * a.d, wn); };
+    if (TURN) {
+        load_x(t0);
+        load_wn();
+    }
     /* weights: q4 rows (codes, scale, bias) or one bf16 row (32 weights a chunk) */
     uint4 wq[RW][P];
     float ws[RW][P], wb[RW][P];
@@ -136,19 +159,22 @@ __device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int 
             }
         }
     }
+    if (!TURN) {
+        load_wn();
+        load_x(t0);
+    }
     const bool store_normed = !INJ && rb == 0;
 
     for (int j = 0; j < m; j++) {
         const int t = t0 + j;
         float xv[P][32];
         float ss = 0.0f;
-        float4 xc[P][8];
-        hc_turn<P>(xr, buf, lane, xc);
+        if (TURN) hc_turn<P>(xr, buf, lane, xr);
 #pragma unroll
         for (int ps = 0; ps < P; ps++)
 #pragma unroll
             for (int v = 0; v < 8; v++) {
-                const float4 f = xc[ps][v];
+                const float4 f = xr[ps][v];
                 xv[ps][4 * v] = cok[ps] ? f.x : 0.0f;
                 xv[ps][4 * v + 1] = cok[ps] ? f.y : 0.0f;
                 xv[ps][4 * v + 2] = cok[ps] ? f.z : 0.0f;
@@ -160,7 +186,7 @@ __device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int 
 #pragma unroll
             for (int i = 0; i < 32; i++) ss = fmaf(xv[ps][i], xv[ps][i], ss);
         ss = qk_group_sum<64>(ss);
-        if (j == 0) hc_turn<P>(wn, buf, lane, wn);
+        if (TURN && j == 0) hc_turn<P>(wn, buf, lane, wn);
         const float r = 1.0f / sqrtf(ss / (float)a.d + a.eps);
         XPairs<64, P, false> xp;
 #pragma unroll
@@ -233,14 +259,14 @@ __device__ __forceinline__ void hc_down_body(const HcDownArgs &a, int tblk, int 
  * inject rows (model.c:790-792).  The two task kinds are separate bodies,
  * so neither carries the other's weight registers.
  */
-template <int P>
+template <int P, bool TURN>
 __global__ __launch_bounds__(64 * HC_MAX) void k_hc_down(HcDownArgs a) {
-    extern __shared__ float4 hc_turn_buf[]; /* 4 KB a wave */
+    extern __shared__ float4 hc_turn_buf[]; /* TURN: 4 KB a wave */
     const int nrb = (a.R + HD_RW - 1) / HD_RW;
     const int nblk = nrb + (a.inject_w ? a.hc : 0);
     const int tblk = blockIdx.x / nblk, rb = blockIdx.x - tblk * nblk;
-    if (rb >= nrb) hc_down_body<P, true>(a, tblk, rb, nrb, hc_turn_buf);
-    else hc_down_body<P, false>(a, tblk, rb, nrb, hc_turn_buf);
+    if (rb >= nrb) hc_down_body<P, true, TURN>(a, tblk, rb, nrb, hc_turn_buf);
+    else hc_down_body<P, false, TURN>(a, tblk, rb, nrb, hc_turn_buf);
 }
 
 /* ------------------------------------------------------- up + mean mix */
@@ -397,7 +423,8 @@ extern "C" int qk_launch_hc_down(const float *hyper, const float *norm_w, const 
     HcDownArgs a{hyper, norm_w, q, s, b, inject_w, normed, w, inject, hc, d, R, n, tb, eps};
     const dim3 grid((unsigned)(((n + tb - 1) / tb) * nblk)), blk(64 * hc);
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_hc_down<1>, grid, blk, 4096 * hc, st, a);
+    if (d >= HD_TURN_D) hipLaunchKernelGGL((k_hc_down<1, true>), grid, blk, 4096 * hc, st, a);
+    else hipLaunchKernelGGL((k_hc_down<1, false>), grid, blk, 0, st, a);
     return QK_CHECK_LAUNCH();
 }
 

@@ -154,7 +154,8 @@ def test_attention_few_tokens(torch_dev, d, h, hd):
     ta.run_calls(torch, dev, (d, h, 1, hd, 3, 68, 12, 3, 64, 1.0), [1, 15, 2], seed=15)
 
 
-@pytest.mark.parametrize("hc,d,R", [(8, 64, 64), (1, 2048, 320), (3, 1984, 128), (2, 1088, 64)])
+# hidden sizes on both sides of the line from which chunks are turned in LDS
+@pytest.mark.parametrize("hc,d,R", [(8, 64, 64), (1, 2048, 320), (3, 1984, 128), (2, 1088, 64), (4, 1472, 64), (5, 1536, 128)])
 @pytest.mark.parametrize("n", [1, 2, 15])
 def test_hyper_few_tokens(torch_dev, hc, d, R, n):
     torch, dev = torch_dev
