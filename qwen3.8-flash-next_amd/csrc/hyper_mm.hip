@@ -1,8 +1,8 @@
 /*
  * hyper_mm.hip -- the MLP hyper connection's producer (gated_residual,
  * reference C port model.c:728-796) for many tokens, on bf16 MFMA
- * (v_mfma_f32_16x16x32_bf16), in three launches, or four from HM_PLANES_N to
- * HM_PLANES_MAX tokens:
+ * (v_mfma_f32_16x16x32_bf16), in three launches, or four where hm_planes says
+ * so:
  *
  *   k_hc_mm_down partial products of the down projection over one K range
  *                of one copy h, sum_k a_k W[r, k] with a = x * hc_norm formed
@@ -561,14 +561,30 @@ __global__ __launch_bounds__(256) void k_hc_act(HcActArgs a) {
     if ((i & 7) == 0) a.wp[i >> 3] = -128.0f * g;
 }
 
-/* Token counts whose down product runs on packed planes (proj_mm.hip): the
- * partial products of k_hc_mm_down form the operands again in every column
- * pass and copy.  hc 4, hidden 2048, rank 320, the whole mix in us, parts
- * against planes: 200 tokens 40 / 45, 256 tokens 40 / 54, 300 tokens 68 / 54,
- * 512 tokens 68 / 56, 1024 tokens 107 / 77, 1400 tokens 125 / 123, 2000 tokens
- * 132 / 138, 4096 tokens 205 / 277. */
+/* Calls whose down product runs on packed planes (proj_mm.hip): the partial
+ * products of k_hc_mm_down form the operands again in every column pass and
+ * copy.  hc 4, hidden 2048, rank 320, the whole mix in us, parts against
+ * planes: 200 tokens 40 / 45, 256 tokens 40 / 54, 300 tokens 68 / 54, 512
+ * tokens 68 / 56, 1024 tokens 107 / 77, 1400 tokens 125 / 123, 2000 tokens 132
+ * / 138, 4096 tokens 205 / 277.
+ *
+ * Of the shape: the planes are one long K for few column tiles, so they need
+ * wide copies, and with several copies a rank that gives the K-split enough
+ * workgroups but not so many that each reads the planes again.  Over 48 shapes
+ * and this range the rule's shapes took 0.41 to 1.00 of the parts' time (hc 1,
+ * 2048, 320: 51 / 31 at 320 tokens; 2, 2048, 768: 65 / 60; 3, 2048, 512: 64 /
+ * 62; 4, 1024, 256: 43 / 40; 4, 2048, 384: 67 / 56), and past it they lose in
+ * part of the range: 4, 2048, 512 70 / 74 and 105 / 112 at 1024; 4, 2048, 64
+ * 42 / 47; 8, 1024, 64 42 / 55; 8, 2048, 512 114 / 138; 2, 2048, 2048 98 /
+ * 104; 2, 512, 64 19 / 22; 1, 512, 64 17 / 20. */
 #define HM_PLANES_N 257
 #define HM_PLANES_MAX 1280
+static bool hm_planes_shape(int hc, int d, int R) {
+    return d >= 1024 && (hc == 1 || (hc <= 4 && R >= 256 && hc * R <= 1536));
+}
+static bool hm_planes(int hc, int d, int R, int n) {
+    return n >= HM_PLANES_N && n <= HM_PLANES_MAX && hm_planes_shape(hc, d, R);
+}
 
 /* ---------------------------------------------------------------- launch */
 
@@ -626,7 +642,7 @@ extern "C" int qk_launch_hc_mm(const float *hyper, const float *norm_w, const ui
     if (hc < 1 || hc > HC_MAX || d % 64 || R % 64 || R > 2048) return (int)hipErrorInvalidValue;
     if (inject_w && !inject) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)stream;
-    if (n >= HM_PLANES_N && n <= HM_PLANES_MAX) {
+    if (hm_planes(hc, d, R, n)) {
         const size_t D = (size_t)hc * d;
         char *p = (char *)ws;
         auto take = [&](size_t bytes) {
@@ -706,6 +722,7 @@ extern "C" size_t qk_hc_mm_ws_bytes(int hc, int d, int R, int max_n) {
     const size_t pn = (size_t)hc * (n > 1024 ? n : 1024);
     const size_t parts = hm_up256(pn * R * 4) + hm_up256(pn * 16 * 4) + hm_up256(pn * 4) + hm_up256(n * hc * 4) +
                          2 * hm_up256(n * R * 2) + hm_up256(n * (R / 64) * 4) + 256;
-    const size_t planes = max_n < HM_PLANES_N ? 0 : hm_planes_bytes(hc, d, R, max_n < HM_PLANES_MAX ? max_n : HM_PLANES_MAX);
+    const int most = max_n < HM_PLANES_MAX ? max_n : HM_PLANES_MAX;
+    const size_t planes = hm_planes(hc, d, R, most) ? hm_planes_bytes(hc, d, R, most) : 0;
     return parts > planes ? parts : planes;
 }

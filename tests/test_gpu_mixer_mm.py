@@ -120,8 +120,10 @@ def test_deltanet_values_past_the_products(torch_dev, bad):
 
 
 # the hyper connection's packed planes: the first and last count on them and
-# their neighbours, a repeated last token, odd copies, small copies
-@pytest.mark.parametrize("hc,d,R", [(4, 256, 128), (3, 192, 64), (8, 64, 64), (1, 2048, 320)])
+# their neighbours, a repeated last token, an odd number of copies and of
+# groups, the shapes at the edge of the rule and small ones past it
+@pytest.mark.parametrize("hc,d,R", [(4, 256, 128), (3, 192, 64), (8, 64, 64), (1, 2048, 320),
+                                    (4, 1024, 256), (3, 1088, 512), (2, 2048, 768), (1, 1024, 64), (5, 1024, 256)])
 @pytest.mark.parametrize("n", [256, 257, 1280, 1281])
 def test_hyper_token_counts(torch_dev, hc, d, R, n):
     torch, dev = torch_dev
