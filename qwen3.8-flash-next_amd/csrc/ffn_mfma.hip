@@ -459,16 +459,15 @@ __global__ __launch_bounds__(256) void k_pack_rows(const void *x, size_t nchunks
 }
 
 /*
- * Down projection of the narrow calls, K = 512, on the dispatch's 16-row
- * task list.  The 64-row kernel waits, every group, on
- * the chain activation load -> LDS store -> barrier -> LDS read (~1 us per
- * group at 1..16 rows).  Here the code words of the whole K slice of the
- * tile (8 groups, 16 bytes per lane and column tile) are loaded into
- * registers at the start, the chunk's f32 h is staged in LDS at once (hi +
- * lo planes and the group sums P, the arithmetic of k_pack_rows), and the
- * K loop reads LDS and registers only, with no barrier.  The products,
- * their order and the epilogue are those of mm_body: the outputs are
- * bit-identical.
+ * Down projection, K = 512, on the dispatch's 16-row task list (mm_down16).
+ * k_mm waits, every group, on the chain activation load -> LDS store ->
+ * barrier -> LDS read (~1 us per group at 1..16 rows).  Here the code words of
+ * the whole K slice of the tile (8 groups, 16 bytes per lane and column tile)
+ * are loaded into registers at the start, the chunk's f32 h is staged in LDS
+ * at once (hi + lo planes and the group sums P, the arithmetic of
+ * k_pack_rows), and the K loop reads LDS and registers only, with no barrier.
+ * The products, their order and the epilogue are those of mm_body: the outputs
+ * are bit-identical.
  */
 #define MMD_G 8 /* K / 64 of the shapes this kernel takes */
 
@@ -637,20 +636,54 @@ __global__ __launch_bounds__(1024) void k_mm_tasks(const int32_t *segtab, int n,
     mm_tasks_block(segtab, n, k, E, min_m, lists);
 }
 
-/* Up to MM_NARROW_N tokens the kernels hold 64-row chunks and give each wave
- * 2 column tiles instead of 4, so a batch of mostly small segments spreads
- * over twice the workgroups (with few rows per task the per-group latency,
- * not the MFMA rate, bounds a workgroup); the down projection at K = 512 runs
- * on k_mm_down16 over the 16-row list.  The line lies where the two meet
- * (hidden 2048, 512 experts top-10, the layer in us, wide against narrow):
- * f32 333 tokens 437 / 388, 512 tokens 452 / 407, 768 tokens 475 / 453;
- * bf16 96 tokens 292 / 279, 333 tokens 389 / 356, 768 tokens 414 / 410,
- * 1024 tokens 438 / 471; with Zipf-skewed routing 128 tokens 138 / 108, 333
- * tokens 181 / 185, 512 tokens 222 / 223, 768 tokens 254 / 286.  The results
- * are the same bits either way, so a layer call short of memory takes the wide
- * kernels, whose lists are shorter (lean). */
+/*
+ * The narrow kernels hold 64-row chunks and give each wave 2 column tiles
+ * instead of 4: twice the workgroups, so a batch of small or uneven segments
+ * spreads better (with few rows per task the per-group latency, not the MFMA
+ * rate, bounds a workgroup), but each activation row is staged twice as often.
+ * k_mm_down16 on the 16-row list is the down projection at K = 512.  Both give
+ * the same bits as the wide kernels, so a layer call short of memory takes
+ * those, whose lists are shorter (lean).
+ *
+ * Measured over 12 shapes, f32 and bf16, uniform and Zipf 1.1 routing, 65 to
+ * 768 tokens, the layer in us, wide / narrow + down16 (w16: wide gate/up +
+ * down16); r = n k / E is the rows per expert:
+ *  - up to 64 experts the wide launches leave the chip short of workgroups and
+ *    narrow wins at any r: E 64, k 4, hidden 1024, 333 tokens 91 / 71; E 8, k
+ *    2, 65 tokens 75 / 51, 512 tokens 97 / 77;
+ *  - more experts, r past 6 (5 from 512 experts on): E 512, k 10, f32 333
+ *    tokens 430 / 366, 512 tokens 439 / 378, Zipf 201 / 193; E 256, k 8, 256
+ *    tokens 241 / 200;
+ *  - at 4 to 6 rows an expert has one 16-row tile and narrow only adds
+ *    workgroups: E 128, k 8, inter 1024, 65 tokens 170 / 177, Zipf 80 tokens
+ *    105 / 116; E 512, Zipf 256 tokens 147 / 153, w16 146, uniform 350 / 336,
+ *    w16 318;
+ *  - below 4 rows the same (E 256, k 8, f32 80 tokens 160 / 170, w16 150; E
+ *    256, k 4, inter 1024 218 / 246), but the 2048 workgroups of 512 experts
+ *    at K = 512 run in uneven rounds and narrow evens them, the more so under
+ *    skew: f32 128 tokens 307 / 304, Zipf 160 / 107;
+ *  - between, past 2400 (token, expert) pairs at K = 512, skew turns it: E
+ *    128, k 8, Zipf 333 tokens 146 / 153;
+ *  - from 32 rows on a 16-row task reads its codes too often: E 64, k 8, 512
+ *    tokens narrow 135, with down16 147, wide 149; Zipf 158 / 166 / 160.
+ */
 #define MM_NARROW_N 512
-static bool mm_narrow(qk_shape s, int n) { return n <= MM_NBM || (!s.lean && n <= MM_NARROW_N); }
+/* neither form helps: few enough experts for skew to fill single ones */
+static bool mm_skewed(qk_shape s, long long nk) { return s.I == 64 * MMD_G && s.E > 64 && s.E < 512 && nk > 2400; }
+static bool mm_narrow(qk_shape s, int n) {
+    if (n <= MM_NBM) return true;
+    if (s.lean || n > MM_NARROW_N) return false;
+    const long long nk = (long long)n * s.k, E = s.E;
+    if (E <= 64) return true;
+    if (nk > (E >= 512 ? 5 : 6) * E) return !mm_skewed(s, nk);
+    return nk < 4 * E && E >= 512 && s.I == 64 * MMD_G;
+}
+static bool mm_down16(qk_shape s, int n) {
+    if (s.I != 64 * MMD_G) return false;
+    if (n <= MM_NBM) return true;
+    const long long nk = (long long)n * s.k;
+    return !s.lean && n <= MM_NARROW_N && nk <= 32LL * s.E && !mm_skewed(s, nk);
+}
 
 static int mm_launch(MmArgs &a, bool down, int terms, const qk_mm_lists &l, hipStream_t st) {
     const bool narrow = l.bm == MM_NBM, d16 = down && l.list16;
@@ -692,7 +725,7 @@ static int mm_max_chunks(qk_shape s, int n, int bm) {
 static size_t mm_small_ints(qk_shape s) { return ((size_t)s.E + 2 + 3) & ~(size_t)3; }
 
 extern "C" qk_mm_lists qk_mfma_lists(qk_shape s, int n, int32_t *tasks) {
-    const bool narrow = mm_narrow(s, n), d16 = narrow && s.I == 64 * MMD_G;
+    const bool narrow = mm_narrow(s, n), d16 = mm_down16(s, n);
     qk_mm_lists l = {};
     l.bm = narrow ? MM_NBM : MM_BM;
     l.max = mm_max_chunks(s, n, l.bm);

@@ -106,7 +106,8 @@ def test_noalloc_matches_layer_forward(torch_dev, shape, with_norm, calls):
 # alone (1927 would do for the lists of every smaller call), with I 512 lists
 # that only fit as 96-row chunks, and a call below 64 tokens
 @pytest.mark.parametrize("shape,n", [((512, 60, 6, 320), 1928), ((1024, 32, 16, 512), 465),
-                                     ((2048, 64, 15, 512), 326), ((8192, 64, 32, 512), 53)])
+                                     ((2048, 64, 15, 512), 326), ((1536, 640, 16, 512), 365),
+                                     ((8192, 64, 32, 512), 53)])
 def test_noalloc_last_count(torch_dev, shape, n):
     torch, dev = torch_dev
     pkg = load_pkg()
