@@ -65,6 +65,7 @@ struct RowsArgs {
     float *hyper;               /* INJ (one q4 segment): hyper[t, j] += inject[t, j] * out[t], */
     const float *inject;        /* [n, hc, ostride] and [n, hc] */
     int hc;
+    int tper;                   /* bf16 rows: tokens per workgroup, blockIdx.y the slice */
 };
 
 template <int P, bool INJ>
@@ -141,8 +142,8 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
      * per lane over its chunks in ascending order from +0, the lanes added
      * by qk_group_sum<64> -- so the indexer's keys and queries have the
      * oracle's bits (the block selection downstream compares them) */
-    const int C8 = a.K >> 3;
-    for (int t = 0; t < a.n; t++) {
+    const int C8 = a.K >> 3, t1 = min((int)(blockIdx.y + 1) * a.tper, a.n);
+    for (int t = blockIdx.y * a.tper; t < t1; t++) {
         float acc[AT_RPW];
 #pragma unroll
         for (int j = 0; j < AT_RPW; j++) acc[j] = 0.0f;
@@ -1020,8 +1021,21 @@ __global__ __launch_bounds__(256) void k_at_comb(AtCombArgs a) {
 static int at_rows_launch(RowsArgs &r, hipStream_t st) {
     const int rows = r.start[r.nseg];
     const int waves = (rows + AT_RPW - 1) / AT_RPW;
-    const dim3 grid((waves + 3) / 4);
+    dim3 grid((waves + 3) / 4);
     const bool inj = r.hyper != nullptr;
+    /* index_qk_proj by itself (hidden sizes past at_idx_ok, many tokens) is a
+     * few workgroups, which took the tokens one after another while the other
+     * rows no longer ran beside them: hidden 8192, 640 rows, 16 tokens of the
+     * mixer 187 us against 147 with all rows in one launch.  The tokens are
+     * split until there are about two workgroups per CU: 100 us */
+    r.tper = r.n;
+    bool q4 = false;
+    for (int i = 0; i < r.nseg; i++) q4 = q4 || r.seg[i].q;
+    if (!q4) {
+        const int slices = max(1, min(r.n, 512 / (int)grid.x));
+        r.tper = (r.n + slices - 1) / slices;
+        grid.y = (r.n + r.tper - 1) / r.tper;
+    }
 #define AT_ROWS_L(P)                                                                  \
     do {                                                                              \
         if (inj) hipLaunchKernelGGL((k_rows<P, true>), grid, dim3(256), 0, st, r);    \

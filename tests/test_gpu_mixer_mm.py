@@ -33,6 +33,14 @@ def test_attention_token_counts(torch_dev, case, calls):
     ta.run_calls(torch, dev, case, calls, seed=9)
 
 
+# hidden sizes past the tiled indexer rows: 17 workgroups of rows with one to
+# four tokens each, and 505 workgroups, which take every token
+@pytest.mark.parametrize("case", [(2112, 2, 1, 64, 3, 68, 12, 3, 256, 1.0), (2176, 2, 1, 64, 62, 128, 12, 3, 256, 1.0)])
+def test_attention_indexer_rows_split(torch_dev, case):
+    torch, dev = torch_dev
+    ta.run_calls(torch, dev, case, [16, 33, 1, 100], seed=18)
+
+
 @pytest.mark.parametrize("hd,cap", [(64, 80), (128, 1100), (192, 80), (256, 80)])
 def test_attention_head_dims_and_ranges(torch_dev, hd, cap):
     """every head dim of the matrix kernel, 3 query heads per kv head (rows
