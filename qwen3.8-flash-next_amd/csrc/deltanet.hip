@@ -389,6 +389,12 @@ extern "C" int qk_dn_shape_ok(const qk_dn_shape *s) {
     return 1;
 }
 
+/* conv-state channels that each workgroup of k_dn_out moves on */
+static int dn_ch_per_wg(int d, int conv_dim, int &owgs) {
+    owgs = (d + 4 * DN_ORW - 1) / (4 * DN_ORW);
+    return (conv_dim + owgs - 1) / owgs;
+}
+
 extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const float *x, int n, float *out,
                             float *conv_state, float *rec_state, float *mixed, float *z, float *av,
                             float *bv, float *core, float *ssp, const qk_planes *pl, float *chunk,
@@ -400,6 +406,11 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     const int conv_dim = 2 * key_dim + value_dim;
     const bool inj = inj_in && inj_in->hyper;
     if (inj && (inj_in->hc < 1 || inj_in->hc > QK_INJECT_MAX_HC || !inj_in->inject)) return (int)hipErrorInvalidValue;
+    /* more conv channels to a row of out_proj than k_dn_out can move: refused
+     * at every token count, before anything is launched */
+    int owgs;
+    const int ch_per_wg = dn_ch_per_wg(s->d, conv_dim, owgs);
+    if (ch_per_wg > 256) return (int)hipErrorInvalidValue;
     int rc;
     const bool mm = n >= QK_DN_MM_N;
     if (mm) {
@@ -485,9 +496,7 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     oa.hc = inj ? inj_in->hc : 1;
     oa.n = n; oa.d = s->d; oa.value_dim = value_dim; oa.dv = s->dv; oa.kc = s->kc;
     oa.conv_dim = conv_dim;
-    const int owgs = (s->d + 4 * DN_ORW - 1) / (4 * DN_ORW);
-    oa.ch_per_wg = (conv_dim + owgs - 1) / owgs;
-    if (oa.ch_per_wg > 256) return (int)hipErrorInvalidValue;
+    oa.ch_per_wg = ch_per_wg;
     const int p_out = (value_dim / 32 + 63) / 64;
     switch (p_out) {
 #define DN_OUT_L(P)                                                                          \

@@ -192,6 +192,25 @@ def test_graph_replay_and_reset(torch_dev):
                 assert torch.equal(o, r), rep
 
 
+@pytest.mark.parametrize("n", [1, 5, 6, 33])
+def test_too_many_channels_for_hidden(torch_dev, n):
+    """conv channels past 32 times the hidden size are refused by every call,
+    whichever kernels its token count takes, and the states stay as they were"""
+    torch, dev = torch_dev
+    pkg = load_pkg()
+    run_steps(torch, dev, (64, 4, 16, 128, 64, 4), [n], seed=7)  # 2048 channels: the last that fit
+    shape = (64, 1, 29, 128, 64, 4)  # 2112
+    D = orc.DeltaNet(*shape, seed=7)
+    with pkg.DeltaNetContext(*shape, n_layers=1, max_tokens=n) as ctx:
+        ctx.upload_layer(0, D.arrays())
+        before = read_states(ctx, 0)
+        with pytest.raises(pkg.QmoeError, match="DeltaNet launch"):
+            ctx.forward(0, torch.ones((n, 64), device=dev))
+        torch.cuda.synchronize()
+        after = read_states(ctx, 0)
+        assert all(np.array_equal(a, b) for a, b in zip(before, after))
+
+
 def test_errors(torch_dev):
     torch, dev = torch_dev
     pkg = load_pkg()
