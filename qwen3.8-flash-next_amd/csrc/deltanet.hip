@@ -32,7 +32,7 @@
  * The GEMVs above walk the tokens one after another and convert x again in
  * every wave: at 2048 tokens (hidden 2048, heads 16/32 of 128) 10050 us for
  * k_dn_in and 5830 for k_dn_out, against 240 + 11 and 100 + 24.
- * From QK_DN_CHUNK_N tokens on k_dn_rec gives way to dn_chunk.hip (3225 us
+ * From qk_dn_chunk_n tokens on k_dn_rec gives way to dn_chunk.hip (3225 us
  * there against 103 + 142).
  *
  * Sums run in parallel orders (lane trees), so results match the reference
@@ -458,7 +458,7 @@ extern "C" int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const floa
     ra.n = n; ra.hk = s->hk; ra.hv = s->hv; ra.dk = s->dk; ra.dv = s->dv; ra.kc = s->kc;
     ra.conv_dim = conv_dim;
     const dim3 rgrid(s->dv / DN_RB, s->hv);
-    const bool chunks = n >= QK_DN_CHUNK_N;
+    const bool chunks = n >= qk_dn_chunk_n(s);
     if (chunks) {
         if (!chunk) return (int)hipErrorInvalidValue;
         rc = qk_launch_dn_chunks(&ra, chunk, stream);

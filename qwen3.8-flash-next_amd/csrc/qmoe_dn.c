@@ -114,7 +114,7 @@ int qmoe_dn_create(qmoe_dn_ctx **out, const qmoe_dn_config *cfg, qmoe_err *err) 
     const size_t ssz[9] = {n * conv_dim * 4, n * value_dim * 4, n * hv * 4, n * hv * 4, n * value_dim * 4,
                            n * (value_dim / 16) * 4, wide ? qk_planes_bytes((int)n, wide / n) : 0,
                            wide ? qk_planes_ld((int)n) * (wide / n / 64) * 4 : 0,
-                           n >= QK_DN_CHUNK_N ? qk_dn_chunk_bytes(&s, cfg->max_tokens) : 0};
+                           cfg->max_tokens >= qk_dn_chunk_n(&s) ? qk_dn_chunk_bytes(&s, cfg->max_tokens) : 0};
     size_t stot = 0, soff[9];
     for (int i = 0; i < 9; i++) {
         soff[i] = stot;
@@ -136,7 +136,7 @@ int qmoe_dn_create(qmoe_dn_ctx **out, const qmoe_dn_config *cfg, qmoe_err *err) 
         c->pl.a = b + soff[6];
         c->pl.pg = (float *)(b + soff[7]);
     }
-    if (n >= QK_DN_CHUNK_N) c->chunk = (float *)(b + soff[8]);
+    if (cfg->max_tokens >= qk_dn_chunk_n(&s)) c->chunk = (float *)(b + soff[8]);
     for (int l = 0; l < cfg->n_layers; l++) {
         if (dn_hip_fail(err, (int)hipMalloc(&c->layers[l].mem, total), "layer weights")) {
             qmoe_dn_destroy(c);

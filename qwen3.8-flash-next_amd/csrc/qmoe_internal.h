@@ -294,15 +294,25 @@ int qk_dn_shape_ok(const qk_dn_shape *s);
  * mixed [n, conv_dim], z [n, value_dim], a, b [n, hv], core [n, value_dim]
  * and ssp [n, hv, dv/16] are scratch; pl, planes of max(d, value_dim)
  * columns, is used from QK_DN_MM_N tokens on and chunk, of
- * qk_dn_chunk_bytes, from QK_DN_CHUNK_N on (they may be NULL below) */
+ * qk_dn_chunk_bytes, from qk_dn_chunk_n on (they may be NULL below) */
 int qk_launch_dn(const qk_dn_shape *s, const qk_dn_dev *W, const float *x, int n, float *out,
                  float *conv_state, float *rec_state, float *mixed, float *z, float *a, float *b,
                  float *core, float *ssp, const qk_planes *pl, float *chunk, const qk_inject *inj,
                  void *stream);
-/* the recurrence in chunks (dn_chunk.hip) from QK_DN_CHUNK_N tokens on (up to
- * 32 tokens it takes 28 us at 32 heads of 128, token by token 1.6 each);
- * rec_args is deltanet.hip's DnRecArgs, scratch of qk_dn_chunk_bytes */
-#define QK_DN_CHUNK_N 20
+/* the recurrence in chunks (dn_chunk.hip) from this many tokens on.  A chunk's
+ * time hardly depends on its tokens, up to 32 of them 28 us at 32 heads of 128
+ * against 1.6 each token by token, but k_dc_prep takes the value dim in rounds
+ * of 128 columns one after another, and key dim 256 doubles its products.  The
+ * mixer in us, token by token / in chunks, key dim x value dim: 128 x 128, 18
+ * tokens 66 / 62; 128 x 256, 20 tokens 69 / 70; 256 x 256, 20 tokens 79 / 83,
+ * 24 tokens 87 / 84; 128 x 512, 28 tokens 83 / 86, 32 tokens 89 / 88; 128 x
+ * 1024, 56 tokens 138 / 139; 64 x 2048, 96 tokens 218 / 225, 128 tokens 267 /
+ * 234. */
+static inline int qk_dn_chunk_n(const qk_dn_shape *s) {
+    const int least = s->dk > 128 ? 24 : 20;
+    return s->dv / 16 > least ? s->dv / 16 : least;
+}
+/* rec_args is deltanet.hip's DnRecArgs, scratch of qk_dn_chunk_bytes */
 size_t qk_dn_chunk_bytes(const qk_dn_shape *s, int max_n);
 int qk_launch_dn_chunks(const void *rec_args, float *scratch, void *stream);
 int qk_launch_dn_zero(float *p, size_t count, void *stream);

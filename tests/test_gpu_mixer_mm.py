@@ -92,6 +92,13 @@ def test_deltanet_chunks(torch_dev, shape):
     td.run_steps(torch, dev, shape, [19, 20, 33, 1, 64, 95], seed=14, seed_state=True)
 
 
+# the first count in chunks of key dim 256 and of wide value dims
+@pytest.mark.parametrize("shape,n", [((128, 1, 2, 256, 64, 4), 24), ((128, 1, 1, 32, 512, 4), 32), ((256, 1, 1, 64, 2048, 4), 128)])
+def test_deltanet_chunk_lines(torch_dev, shape, n):
+    torch, dev = torch_dev
+    td.run_steps(torch, dev, shape, [n - 1, n, n + 1], seed=19, seed_state=True)
+
+
 def test_deltanet_segments(torch_dev):
     torch, dev = torch_dev
     td.run_steps(torch, dev, (64, 1, 2, 64, 64, 4), [2048, 2049, 2100], seed=15)
