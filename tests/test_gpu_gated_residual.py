@@ -269,7 +269,7 @@ def test_layer_loop(torch_dev, shape, types, calls, seed):
 
 
 @pytest.mark.parametrize("shape", ["tiny", "model"])
-@pytest.mark.parametrize("n", [1, 3])
+@pytest.mark.parametrize("n", [1, 3, 6, 16, 33])
 def test_mixer_forward_inject(torch_dev, shape, n):
     """qmoe_dn_forward_inject / qmoe_attn_forward_inject (the gated
     residual's update fused into the mixer's last launch) against the
@@ -281,7 +281,7 @@ def test_mixer_forward_inject(torch_dev, shape, n):
     shp = TINY if shape == "tiny" else MODEL
     types = ("dn", "attn")
     say(f"case: mixer forward_inject {shape} n={n}")
-    ch = Chain(torch, dev, shp, types, 7, 4)
+    ch = Chain(torch, dev, shp, types, 7, max(n, 4))
     try:
         h0 = torch.from_numpy(orc.gen_hyper(n, shp["hc"], shp["d"], seed=71)).to(dev)
         for l, t in enumerate(types):
@@ -324,19 +324,21 @@ def pkg_error():
     return load_pkg().QmoeError
 
 
-def test_decoder_stack(torch_dev):
+@pytest.mark.parametrize("calls", [(4, 1, 1), (40, 1)])
+def test_decoder_stack(torch_dev, calls):
     """the benchmark's decoder stack (qmoe.DecoderStack: gated DeltaNet and
     full attention at 3 : 1 by the model's layer types, both hyper
     connections of every layer, the final mixer) at 4 of its 48 layers and
     the model's shapes, end to end against the oracle's own chain from the
-    same hyper states: a 4-token prefill call, then one-token calls.  The
+    same hyper states: a prefill call (4 tokens on the per-token kernels, 40
+    on the matrix kernels of every part), then one-token calls.  The
     final mixer output and the hyper state after the last layer within
     2e-2 max-abs and 1e-3 relative L2."""
     torch, dev = torch_dev
     pkg = load_pkg()
     types = tuple(pkg.decoder_layer_types(4))
     assert types == ("dn", "dn", "dn", "attn")
-    seed, calls = 5, (4, 1, 1)
+    seed = 5
     say(f"case: decoder stack {types} calls {calls}")
     ch = Chain(torch, dev, MODEL, types, seed, max(calls))
     try:
