@@ -75,7 +75,7 @@ __device__ __forceinline__ bool am_bad8(const float x[8]) {
  * (part, 32 dims dt, K-step s of 16 keys), lane l = dim 32 dt + l%32, the
  * keys 16 s + 8 a + 4 (l/32) + b at 4 a + b: the order in which the scores'
  * accumulators hold the keys of a row.  Keys past T are zero.  Bound: HBM /
- * L2 writes (12 bytes out per 4 in).
+ * L2 writes (6 bytes out per 4 in).
  */
 __global__ __launch_bounds__(256) void k_am_prep(AmArgs a) {
     const int tile = blockIdx.x, kh = blockIdx.y, tid = threadIdx.x;

@@ -2,7 +2,10 @@
  * dn_chunk.hip -- the DeltaNet recurrence of many tokens (reference
  * c/src/model.c:1177-1248: conv, silu, l2 norms, decay, delta rule) in
  * chunks of 32 tokens, two launches per 2048 tokens instead of a serial step
- * per token.
+ * per token.  The method is the chunked delta rule of Yang, Wang, Zhang, Shen
+ * and Kim, "Parallelizing Linear Transformers with the Delta Rule over
+ * Sequence Length" (2024), with the decay of Yang, Kautz and Hatamizadeh,
+ * "Gated Delta Networks" (2024).
  *
  * With the decay products g_1..g_t = exp(G_t) inside a chunk and S the state
  * before it, the rule S <- g S; S += beta (v - S k) k^T gives

@@ -1,6 +1,8 @@
 /*
- * mfma_parts.h -- operand helpers for v_mfma_f32_16x16x32_bf16 on q4
- * weights: the vector types and the code word -> B operand conversion.
+ * mfma_parts.h -- operand helpers for v_mfma_f32_16x16x32_bf16 and
+ * v_mfma_f32_32x32x16_bf16 on q4 weights: the vector types, the code word ->
+ * B operand conversions, copies straight to LDS with their waits, and the
+ * packing of rows into operand planes.
  */
 #ifndef MFMA_PARTS_H
 #define MFMA_PARTS_H

@@ -271,12 +271,15 @@ typedef struct {
     int end64[QK_PROJ_SEGS], mtiles, ntiles, btiles, byrow; /* filled by the launcher */
 } qk_proj;
 int qk_launch_proj(const qk_proj *a, void *stream);
-/* the mixers take their matrix kernels from this many tokens on.  DeltaNet's
- * per-token GEMVs cost 7 us a token at hidden 2048: 45 us the mixer at 5
- * tokens and on that slope 52 at 6 and 65 at 8, against 46 and 50.  Attention's whole path (projections,
- * indexer rows, attn_mm.hip) has more launches: at 9 tokens 50..71 us on the
- * per-token kernels and 46..86 on these over four shapes, at 16 tokens 59..122
- * against 37..97. */
+/* the mixers take their matrix kernels from this many tokens on.  DeltaNet in
+ * us, per-token GEMVs against planes, hidden 2048, heads 16/32 of 128: 4
+ * tokens 38 / 42, 5 tokens 45 / 44, 6 tokens 52 / 46, 8 tokens 66 / 49; of
+ * eleven other shapes five lose up to a tenth on planes at 4 tokens (hidden
+ * 1024, heads 4/8 26 / 29) and three are level at 5 (30 / 30), where a call
+ * keeps the one-token calls' bits; all win at 6.  Attention's whole path
+ * (projections, indexer rows, attn_mm.hip) has more launches: at 9 tokens
+ * 50..71 us on the per-token kernels and 46..86 on these over four shapes, at
+ * 16 tokens 59..122 against 37..97. */
 #define QK_DN_MM_N 6
 #define QK_AT_MM_N 16
 /* the gated DeltaNet mixer (deltanet.hip) */
